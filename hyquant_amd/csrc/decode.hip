@@ -1661,11 +1661,20 @@ size_t round256(size_t x) { return (x + 255) / 256 * 256; }
 //     per-piece round trips), G <= 4: every segment cut into pieces of
 //     equal bytes, total / (0.8 CUs) (measured best at B=1 from 2K to 32K
 //     prefixes), at most 48 per head.
-//   few KV heads, G > 4 (each partial is G rows, so the merge weighs more):
-//     int4 pieces of the smallest power-of-two token count >= 128 that gives
-//     at most 32 pieces (2048 at most), bf16 pieces of 128 tokens (without
-//     a prefix, like the prefix: a power of two from 128 to 512).
-//   many KV heads: pieces of about total / (1.25 * slots) bytes, `slots`
+//   up to 64 KV heads and a launch of less than 48 MB (G <= 4) or 80 MB (G > 4;
+//     any size with fewer than 20 heads), 7-25 us that mix one piece's latency
+//     and the merge: the piece count with the least modelled time
+//     (cheapest_pieces).  Swept over 200 shapes (32/8, 64/8 and 32/2 heads,
+//     batches 1-32, 1K-32K tokens; graph replay over 400 MB of copies): in this
+//     range it is 1-2% above each shape's best piece count on average, where
+//     power-of-two pieces (fewer than 32 heads) and 1.25 rounds of at least
+//     96 KiB were 19% above.  12 x 2 heads, G = 16, 4096 tokens 20.5 -> 11.7 us;
+//     3 x 8 heads, G = 8, 4000 tokens 17.7 -> 10.9 us; 4 x 8 heads, G = 4,
+//     1024 tokens 9.6 -> 7.2 us.
+//   G > 8, 20 to 64 KV heads and 60 MB or more: 12 pieces, the most that the
+//     merge loads in one batch (48 heads, 16384 tokens 33.7 -> 29.5 us, 13001
+//     tokens with 2-bit V 27.5 -> 23.4 us; 32 heads, 32768 tokens 38.8 -> 36.8).
+//   else: pieces of about total / (1.25 * slots) bytes, `slots`
 //     being the workgroups the device holds at once: the first round fills
 //     every slot and the remaining quarter, with the short segment pieces,
 //     evens out the workgroups that ran slow.  Pieces stay >= 96 KiB: below
@@ -1677,6 +1686,70 @@ size_t round256(size_t x) { return (x + 255) / 256 * 256; }
 //     shorter round gains (GLM-4-9B shape, 248 KiB: 37.4 -> 40.1 us).
 // Each segment gets its bytes / target pieces (rounded, at least one); the
 // target grows until the pieces fit the merge tables.
+
+// A head's segments as pieces: starting from one each, every further piece
+// goes to the segment whose pieces are the largest.
+struct Pieces {
+    const int64_t *su, *sc;             // units, bytes per unit
+    int ks[4] = {0, 0, 0, 0};
+    int64_t size[4] = {0, 0, 0, 0};     // bytes of the segment's largest piece
+    int total = 0;
+    Pieces(const int64_t (&u)[4], const int64_t (&c)[4]) : su(u), sc(c) {
+        for (int s = 0; s < 4; ++s)
+            if (su[s] > 0) {
+                ks[s] = 1;
+                size[s] = su[s] * sc[s];
+                ++total;
+            }
+    }
+    int largest() const {
+        int w = 0;
+        for (int s = 1; s < 4; ++s)
+            if (size[s] > size[w]) w = s;
+        return w;
+    }
+    bool split() {                      // false: the largest piece is one unit
+        const int w = largest();
+        if (ks[w] >= su[w]) return false;
+        ++ks[w];
+        ++total;
+        size[w] = (su[w] + ks[w] - 1) / ks[w] * sc[w];
+        return true;
+    }
+};
+
+// Partials a merging thread loads for k pieces, rounded up to its batch.
+int merge_loads(int G, int k) {
+    const int items = G <= WAVES ? (k + 1) / 2 : merge_items(G, k);
+    const int step = G <= WAVES ? 4 : 8;
+    return items <= 24 ? (items + step - 1) / step * step : (items + 23) / 24 * 24;
+}
+
+// The piece count (at most kmax, and 15/16 of the resident slots: a full
+// device starts its last workgroups late) with the least modelled time, in us:
+// the largest piece at 32 KB/us on a CU of its own or 26 KB/us shared by a
+// CU's two, plus 0.05 (G <= 4, a wavefront's merge) or 0.095 (a workgroup's)
+// per partial loaded.  Fitted to the sweep above.
+Pieces cheapest_pieces(const int64_t (&su)[4], const int64_t (&sc)[4], int bh_kv, int G, int kmax, int64_t slots,
+                       int64_t cus) {
+    Pieces p(su, sc), best = p;
+    const int most = std::min<int64_t>(kmax, std::max<int64_t>(p.total, slots * 15 / 16 / bh_kv));
+    double least = 1e30;
+    for (;;) {
+        const double m = static_cast<double>(p.size[p.largest()]);
+        const double wgs = static_cast<double>(p.total) * bh_kv;
+        const double stream = wgs <= cus ? m / 32e3 : std::max(m / 32e3, 2.0 * m * (wgs / slots) / 26e3);
+        const double cost = stream + (G <= WAVES ? 0.05 : 0.095) * merge_loads(G, p.total);
+        if (cost < least) {
+            least = cost;
+            for (int s = 0; s < 4; ++s) best.ks[s] = p.ks[s];
+            best.total = p.total;
+        }
+        if (p.total >= most || !p.split()) break;
+    }
+    return best;
+}
+
 Plan make_plan(int64_t n_quant, const int64_t seg_n[3], int bh_kv, int G, int requested, int kb, int vb,
                Slots sl_) {
     const int slots = sl_.slots;
@@ -1711,6 +1784,7 @@ Plan make_plan(int64_t n_quant, const int64_t seg_n[3], int bh_kv, int G, int re
     };
     int total;
     int64_t target;
+    const bool twelve = G > 8 && bh_kv >= 20 && bh_kv <= 64 && head_bytes * bh_kv >= 60000000;
     if (requested > 0) {
         target = std::max<int64_t>(1, (requested + GROUP - 1) / GROUP) * cq;
         total = counts_for(target);
@@ -1723,21 +1797,15 @@ Plan make_plan(int64_t n_quant, const int64_t seg_n[3], int bh_kv, int G, int re
         target = std::max<int64_t>(8 << 10, head_bytes * bh_kv * 5 / (4 * cus));
         target = std::max<int64_t>(target, (head_bytes + 47) / 48);
         total = counts_for(target);
-    } else if (bh_kv < 32) {
-        int64_t split = 4 * GROUP, bsplit = 128;
-        while (split < 2048 && split * 32 < n_quant) split *= 2;
-        if (n_quant == 0) {       // bf16 alone (the full-precision comparator): split like a prefix
-            const int64_t nb = seg_n[0] + seg_n[1] + seg_n[2];
-            while (bsplit < 512 && bsplit * 32 < nb) bsplit *= 2;
+    } else if (bh_kv <= 64 && (twelve || bh_kv < 20 || head_bytes * bh_kv < (G <= WAVES ? 48000000 : 80000000))) {
+        Pieces best(su, sc);
+        if (twelve) {
+            while (best.total < std::min(kmax, 12) && best.split()) {}
+        } else {
+            best = cheapest_pieces(su, sc, bh_kv, G, kmax, slots > 0 ? slots : 512, sl_.cus > 0 ? sl_.cus : 256);
         }
-        const int64_t gsplit = split / GROUP;
-        bsplit /= BUNIT;
-        ks[0] = static_cast<int>((su[0] + gsplit - 1) / gsplit);
-        total = ks[0];
-        for (int s = 1; s < 4; ++s) {
-            ks[s] = static_cast<int>((su[s] + bsplit - 1) / bsplit);
-            total += ks[s];
-        }
+        for (int s = 0; s < 4; ++s) ks[s] = best.ks[s];
+        total = best.total;
         target = (head_bytes + total - 1) / total;
     } else {
         const int64_t sl = slots > 0 ? slots : 512;
