@@ -1263,23 +1263,35 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
 // offset-encoded codes (int4: channel 2j in the high nibble of byte j, value
 // u - 8; int2: channel 4j + i in bits 7-2i..6-2i of byte j, value u - 1.5)
 // with one fp16 scale per (group of tokens, channel), then the top-k,
-// staging and window bf16 rows.  The prefix tiles are dequantised in
-// registers to the bf16 values of legacy_dequant_kernel (legacy_twice_to_bf16)
-// scaled by an exact power of two, and computed by the bf16 tile path
-// (bf16_compute): the result of dequantising the prefix and decoding bf16
-// rows, without the bf16 copy in HBM.  One workgroup per piece
-// (LEG_PIECE prefix tokens or BF_PIECE rows of one segment, the same number
-// of bytes; halved together, down to LEG_PIECE_MIN tokens, while the grid
-// would leave a CU without a workgroup; doubled together while the prefix
-// still gives every resident workgroup slot a piece, up to LEG_PIECE_MAX
-// tokens, and for long caches until the pieces fit the merge tables), merged
-// by the head's last arriving workgroup with decode_kernel's protocol and
-// merge.
-constexpr int LEG_PIECE = 512;
-constexpr int LEG_PIECE_MIN = 128;
-constexpr int LEG_PIECE_MAX = 4096;
-constexpr int BF_PIECE = 128;
-
+// staging and window bf16 rows.
+//
+// The scales are folded out of the products, so that the codes go to the
+// matrix cores as they are:
+//   scores  q . (code * s_k) = (q * s_k) . code: once per scale group each
+//     lane multiplies its 32 query channels by the group's scales in fp32 and
+//     rounds them once to fp16, scaled by a power of two that puts the
+//     column's largest product in [2^14, 2^15) (rounding error 2^-12 of a
+//     channel's product, against 2^-9 for K rounded to bf16); the codes are
+//     exact fp16 subnormals, as in k_operand;
+//   P.V     sum_t P_t (code_t * s_v) = s_v * sum_t P_t code_t: the group's
+//     sum is formed on its own accumulators (bf16(128 + u) operands and the
+//     all-ones product that removes the offset, as in qcompute) and joins the
+//     running one with one fp32 multiply-add per channel at the group's end.
+// A tile's conversion then costs what the per-token format's does, where
+// dequantising every element to bf16 cost about 2.9 VALU instructions an
+// element and kept the VALU busy 59-67% of the time.  128 KV heads at 30011
+// tokens (618 MB with the bf16 rows): K4V4 161 -> 101 us (6.1 TB/s, near the
+// 6.8 TB/s of a read-only stream), K4V2 172 -> 91, K2V4 159 -> 94, K2V2 169 ->
+// 90 us; 60 heads at G = 16, 5838 tokens 43 -> 21 us.  Two workgroups per CU
+// (217-233 VGPRs, no spill).  Error against float64, K4V4: 3.2e-3 -> 2.0e-3 of
+// the output's norm.
+//
+// Prefix units are chunks of 32 tokens that never cross a scale group (a
+// group that is not a multiple of 32 ends in a short chunk).  A wavefront
+// walks blocks of BLK chunks of one scale group (legacy_blk): BLK = 4 shares
+// one folding of the scales among a 128-token group's chunks; BLK = 1 folds
+// them for every chunk.  Pieces, partials, arrival and merge are
+// decode_kernel's.
 struct LegArgs {
     const uint16_t* q;
     int64_t q_stride;
@@ -1291,6 +1303,9 @@ struct LegArgs {
     int64_t ks_bh, ks_g, vs_bh, vs_g;
     int64_t ks_rows, vs_rows;      // scale rows per head (the descriptors' ranges)
     int n_leg, group;
+    int cpg;                       // chunks per scale group
+    int nqg;                       // prefix schedule units (blocks) per head
+    int segu[2];                   // bf16 schedule units (BUNIT tokens) of segments 0 and 1
     const uint16_t* sk[3];         // top-k, staging, window rows [bh][n][D]
     const uint16_t* sv[3];
     int64_t sk_bh[3], sv_bh[3];
@@ -1303,179 +1318,223 @@ struct LegArgs {
     uint16_t* out;
     int64_t out_stride;
     int nwg, mj;
-    int pfirst[5];                 // pieces of segment s (0: the prefix): [pfirst[s], pfirst[s + 1])
-    int plen[4];                   // tokens per piece of segment s
+    int bnd[MAX_NWG + 1];          // piece p: schedule units [bnd[p], bnd[p + 1]) of its head
 };
 
-// the raw loads of one 16-token prefix tile, for the layout of Bf16Raw (the
-// group is a multiple of 16 and tiles start at multiples of 16 tokens, so a
-// tile's tokens share one scale row)
+// one 32-token chunk, in QRaw's layout (the scales are per group)
 template <int KB, int VB>
 struct LegRaw {
-    uint32_t kc[KB];               // token c: codes of channels 32kb .. 32kb + 31 (4 KB bytes)
-    u32x4 ksc[4];                  // their fp16 scales, 8 channels per vector
-    uint32_t vc[4];                // slot e (token 4kb + e): codes of channels 8c .. 8c + 7 (VB bytes, zero-extended)
-    u32x4 vsc;                     // their fp16 scales
+    uint32_t k[2][KB];
+    uint32_t v[8];                 // VB bytes, zero-extended
 };
 
-// Loads of the tile at token t of a piece starting at prefix token lo: the
-// lane's offsets (kco: token c, vco: token 4kb) are fixed, the tile's
-// position goes in the scalar offsets.  The code descriptors cover the piece
-// and the scale descriptors the head's scale rows (the range check covers
-// the scalar offset too): tokens past either read zeros.
+// Chunk starting t tokens into its piece; the rows' strides (bytes) are
+// uniform, so every load's position goes in its scalar offset.  Codes are
+// read once: non-temporal.
 template <int KB, int VB>
-__device__ __forceinline__ void legacy_fetch(LegRaw<KB, VB>& r, const LegArgs& a, Rsrc rkc, Rsrc rvc, Rsrc rks,
-                                             Rsrc rvs, uint32_t kco, uint32_t vco, int lo, int t, int lane) {
-    const int c = lane & 15, kb = lane >> 4;
-    // wave-uniform scalar offsets (left to the compiler, some became vector
-    // values and their loads were wrapped in waterfall loops)
-    const int tu = __builtin_amdgcn_readfirstlane(t);
-    const int g = (lo + tu) / a.group;                     // the tile's scale row
-    const uint32_t skc = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(tu * a.kc_n));
-    const uint32_t sks = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(g * a.ks_g * 2));
-    const uint32_t svc = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(tu * a.vc_n));
-    const uint32_t svs = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(g * a.vs_g * 2));
-    // codes are read once: non-temporal, as the fused decode's packed rows
-    // (with inputs rotated over 1 GiB: 128 KV heads at 62000 tokens 300-307
-    // -> 290 us, 32 heads 50.5-51.0 -> 49.0-49.5 us); the scale rows, read by
-    // every tile of their group, keep the default policy
-    if constexpr (KB == 4) {
-        const u32x4 w = bld128<NT>(rkc, kco, skc);
-        r.kc[0] = w[0]; r.kc[1] = w[1]; r.kc[2] = w[2]; r.kc[3] = w[3];
-    } else {
-        const u32x2 w = bld64<NT>(rkc, kco, skc);
-        r.kc[0] = w[0]; r.kc[1] = w[1];
-    }
+__device__ __forceinline__ void legacy_fetch(LegRaw<KB, VB>& r, Rsrc rk, Rsrc rv, uint32_t klane, uint32_t vlane,
+                                             uint32_t t, uint32_t kc_n, uint32_t vc_n) {
+    const uint32_t sk = __builtin_amdgcn_readfirstlane(t * kc_n);
+    const uint32_t sv = __builtin_amdgcn_readfirstlane(t * vc_n);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) r.ksc[i] = bld128(rks, static_cast<uint32_t>(64 * kb + 16 * i), sks);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        r.vc[e] = VB == 4 ? bld32<NT>(rvc, vco + static_cast<uint32_t>(e * a.vc_n), svc)
-                          : bld16<NT>(rvc, vco + static_cast<uint32_t>(e * a.vc_n), svc);
-    r.vsc = bld128(rvs, static_cast<uint32_t>(16 * c), svs);
-}
-
-// Codes -> bf16 operands at a power-of-two fraction of the dequantised
-// values.  v_cvt_off_f32_i4 turns the low 4 bits of its operand (byte B of
-// the word, picked by SDWA) into that signed 4-bit field divided by 16, so
-// one instruction replaces a bit-field extract and a conversion.
-//   int4: the code word w has every nibble XOR 8, so a nibble read as a
-//     signed field is u - 8; channel 2j sits in the high nibble of byte j
-//     (read from w >> 4), 2j + 1 in the low one (read from w): (u - 8) / 16.
-//   int2: crumb m of every byte (bits 7-2m..6-2m, channel 4j + m) goes to
-//     the low bits of its byte, and 2u + 13 makes a nibble whose signed value
-//     is 2u - 3: (u - 1.5) / 8.
-// The value times an fp16 scale is exact in fp32 and is rounded once by the
-// packed bf16 conversion, which gives exactly 1/16 (int4) or 1/8 (int2) of
-// legacy_twice_to_bf16's bits (every such product is a normal float or zero,
-// so the power-of-two factor commutes with the rounding; the zeros keep their
-// signs).  The kernel multiplies the score scale by 16 (8) for the prefix and
-// its P.V accumulators by 16 (8) after it, both exact.
-template <int B>
-__device__ __forceinline__ float off4_byte(uint32_t w) {
-    float r;
-    if constexpr (B == 0)
-        asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(r) : "v"(w));
-    else if constexpr (B == 1)
-        asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(r) : "v"(w));
-    else if constexpr (B == 2)
-        asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(r) : "v"(w));
-    else
-        asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(r) : "v"(w));
-    return r;
-}
-// x times the fp16 in the low (HI = false) or high half of sw, converted
-// inside v_fma_mix_f32; the addend is neg(0) = -0 so that x * s + a is the
-// product itself, zeros with their signs
-template <bool HI>
-__device__ __forceinline__ float mul_f16_half(float x, uint32_t sw) {
-    float r;
-    if constexpr (HI)
-        asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(x), "v"(sw));
-    else
-        asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[0,0,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(x), "v"(sw));
-    return r;
-}
-// K: byte B's two channels, each with its own fp16 scale (the halves of sw)
-template <int B>
-__device__ __forceinline__ uint32_t leg4_pair_k(uint32_t w, uint32_t wsh, uint32_t sw) {
-    return pack_bf16x2(mul_f16_half<false>(off4_byte<B>(wsh), sw), mul_f16_half<true>(off4_byte<B>(w), sw));
-}
-// V: the lane's eight channel scales are shared by its four code words, so
-// they are converted once and multiplied in fp32
-template <int B>
-__device__ __forceinline__ uint32_t leg4_pair_v(uint32_t w, uint32_t wsh, const float (&s)[8]) {
-    return pack_bf16x2(off4_byte<B>(wsh) * s[2 * B], off4_byte<B>(w) * s[2 * B + 1]);
-}
-
-// int2: crumb m of every byte of w as a nibble of value 2u - 3 in its byte
-template <int M>
-__device__ __forceinline__ uint32_t crumb_nibbles(uint32_t w) {
-    return (((w >> (6 - 2 * M)) & 0x03030303u) << 1) + 0x0d0d0d0du;
-}
-// K, int2: the pair (channels 4j + M, 4j + M + 1) of byte J, with the two
-// halves of the scale word sw
-template <int J, int M>
-__device__ __forceinline__ uint32_t leg2_pair_k(const uint32_t (&n)[4], uint32_t sw) {
-    return pack_bf16x2(mul_f16_half<false>(off4_byte<J>(n[M]), sw), mul_f16_half<true>(off4_byte<J>(n[M + 1]), sw));
-}
-template <int J, int M>
-__device__ __forceinline__ uint32_t leg2_pair_v(const uint32_t (&n)[4], const float (&s)[8]) {
-    return pack_bf16x2(off4_byte<J>(n[M]) * s[4 * J + M], off4_byte<J>(n[M + 1]) * s[4 * J + M + 1]);
-}
-
-template <int KB, int VB>
-__device__ __forceinline__ void legacy_dequant(Bf16Raw& b, const LegRaw<KB, VB>& r) {
-    if constexpr (KB == 4) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t w = r.kc[i] ^ 0x88888888u, wsh = w >> 4;
-            b.k[i] = u32x4{leg4_pair_k<0>(w, wsh, r.ksc[i][0]), leg4_pair_k<1>(w, wsh, r.ksc[i][1]),
-                           leg4_pair_k<2>(w, wsh, r.ksc[i][2]), leg4_pair_k<3>(w, wsh, r.ksc[i][3])};
-        }
-    } else {
-        // word h holds channels 32kb + 16h .. + 15: operand 2h + 0 takes its
-        // bytes 0 and 1, operand 2h + 1 its bytes 2 and 3
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t n[4] = {crumb_nibbles<0>(r.kc[h]), crumb_nibbles<1>(r.kc[h]), crumb_nibbles<2>(r.kc[h]),
-                                   crumb_nibbles<3>(r.kc[h])};
-            const u32x4& s0 = r.ksc[2 * h];
-            const u32x4& s1 = r.ksc[2 * h + 1];
-            b.k[2 * h] = u32x4{leg2_pair_k<0, 0>(n, s0[0]), leg2_pair_k<0, 2>(n, s0[1]), leg2_pair_k<1, 0>(n, s0[2]),
-                               leg2_pair_k<1, 2>(n, s0[3])};
-            b.k[2 * h + 1] = u32x4{leg2_pair_k<2, 0>(n, s1[0]), leg2_pair_k<2, 2>(n, s1[1]),
-                                   leg2_pair_k<3, 0>(n, s1[2]), leg2_pair_k<3, 2>(n, s1[3])};
-        }
-    }
-    float vs[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        vs[2 * j] = f16_bits_to_f32(static_cast<uint16_t>(r.vsc[j]));
-        vs[2 * j + 1] = f16_bits_to_f32(static_cast<uint16_t>(r.vsc[j] >> 16));
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        if constexpr (VB == 4) {
-            const uint32_t w = r.vc[e] ^ 0x88888888u, wsh = w >> 4;
-            b.v[e] = u32x4{leg4_pair_v<0>(w, wsh, vs), leg4_pair_v<1>(w, wsh, vs), leg4_pair_v<2>(w, wsh, vs),
-                           leg4_pair_v<3>(w, wsh, vs)};
+    for (int i = 0; i < 2; ++i) {
+        if constexpr (KB == 4) {
+            const u32x4 w = bld128<NT>(rk, klane, sk + 16 * i * kc_n);
+            r.k[i][0] = w[0]; r.k[i][1] = w[1]; r.k[i][2] = w[2]; r.k[i][3] = w[3];
         } else {
-            const uint32_t n[4] = {crumb_nibbles<0>(r.vc[e]), crumb_nibbles<1>(r.vc[e]), crumb_nibbles<2>(r.vc[e]),
-                                   crumb_nibbles<3>(r.vc[e])};
-            b.v[e] = u32x4{leg2_pair_v<0, 0>(n, vs), leg2_pair_v<0, 2>(n, vs), leg2_pair_v<1, 0>(n, vs),
-                           leg2_pair_v<1, 2>(n, vs)};
+            const u32x2 w = bld64<NT>(rk, klane, sk + 16 * i * kc_n);
+            r.k[i][0] = w[0]; r.k[i][1] = w[1];
         }
     }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        r.v[e] = VB == 4 ? bld32<NT>(rv, vlane, sv + 4 * e * vc_n) : bld16<NT>(rv, vlane, sv + 4 * e * vc_n);
 }
 
-// Three workgroups per CU (168 VGPRs): the tile loop keeps its registers and
-// the merge at the end spills 236 bytes per lane.  Against two per CU (213
-// VGPRs, no spill), same box, 128 KV heads: 31000 tokens K4V4 171.5 ->
-// 167-169 us, K2V2 184 -> 167-169 us; 62000 tokens 322 -> 294-297 us (waves
-// that wait on memory leave the VALU to the others: 59-67% VALU-busy at two).
+// A scale group's row, this lane's channels 32kb .. 32kb + 31 (8 fp16 per
+// vector); every block of the group reads it: default policy.
+__device__ __forceinline__ void legacy_scales(u32x4 (&s)[4], Rsrc r, int g, uint32_t row_bytes, int lane) {
+    const uint32_t so = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(g) * row_bytes);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = bld128(r, static_cast<uint32_t>(64 * (lane >> 4) + 16 * i), so);
+}
+
+// The QK A operand of MFMA m (channels 32kb + 8m + [0..7]) as fp16 subnormals
+// of value u * 2^-24 (int4) or 2u * 2^-24 (int2), in the channel order of
+// leg_slot.
+template <int KB>
+__device__ __forceinline__ f16x8 legacy_k_operand(const uint32_t (&k)[KB], int m) {
+    if constexpr (KB == 4) {
+        const uint32_t x = k[m];
+        const u32x4 o = {x & 0x000f000fu, (x >> 4) & 0x000f000fu, (x >> 8) & 0x000f000fu, (x >> 12) & 0x000f000fu};
+        return __builtin_bit_cast(f16x8, o);
+    } else {
+        const uint32_t w = k[m >> 1];
+        const uint32_t y = (m & 1) ? perm(w, w, 0x0c030c02u) : perm(w, w, 0x0c010c00u);
+        const u32x4 o = {(y << 1) & 0x00060006u, (y >> 1) & 0x00060006u, (y >> 3) & 0x00060006u, (y >> 5) & 0x00060006u};
+        return __builtin_bit_cast(f16x8, o);
+    }
+}
+// channel (of 8) in fp16 half h of operand dword d: the pairs of
+// legacy_k_operand's shifts
+template <int KB>
+__device__ __forceinline__ constexpr int leg_slot(int d, int h) {
+    return KB == 4 ? (d ^ 1) + 4 * h : 3 - d + 4 * h;
+}
+// the code value is (u - 8) (int4) or (2u - 3) / 2 (int2); the operand's
+// constant and the power of two that undoes 2^-24 (and the half)
+template <int KB>
+constexpr uint32_t leg_k_offset() { return KB == 4 ? 8u : 3u; }
+template <int KB>
+constexpr int leg_k_exp() { return KB == 4 ? 24 : 23; }
+template <int VB>
+constexpr float leg_v_offset() { return VB == 4 ? 136.0f : 129.5f; }
+
+// x times the fp16 in the low or high half of sw (converted exactly)
+__device__ __forceinline__ float mul_half(float x, uint32_t sw, int hi) {
+    return x * f16_bits_to_f32(static_cast<uint16_t>(hi ? sw >> 16 : sw));
+}
+
+// The query column times a scale group's K scales: fp16 operands qop (scaled
+// by 2^-e), the accumulators' start kbias and the score factor qk.  qn: the
+// query's bf16 channels scaled by 2^-qex (legacy_norm_q).
+template <int KB>
+__device__ __forceinline__ void legacy_q_operand(f16x8 (&qop)[4], f32x4& kbias, float& qk, const u32x4 (&qn)[4],
+                                                 const u32x4 (&ks)[4], float qk_scale, int qex) {
+    float x[32];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x[8 * i + 2 * j] = mul_half(__uint_as_float(qn[i][j] << 16), ks[i][j], 0);
+            x[8 * i + 2 * j + 1] = mul_half(__uint_as_float(qn[i][j] & 0xffff0000u), ks[i][j], 1);
+        }
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(x[i]));
+    amax = col_max(amax);
+    // 2^-e with e = exponent(amax) - 14; |qn| < 2 and |s| < 2^16, and a column
+    // of zeros (or below 2^-113) keeps e = -127
+    const int eb = max(static_cast<int>(__float_as_uint(amax) >> 23), 14);
+    const float f = __uint_as_float(static_cast<uint32_t>(268 - eb) << 23);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const float* y = x + 8 * m;
+        const f16x8 v = {
+            static_cast<_Float16>(y[leg_slot<KB>(0, 0)] * f), static_cast<_Float16>(y[leg_slot<KB>(0, 1)] * f),
+            static_cast<_Float16>(y[leg_slot<KB>(1, 0)] * f), static_cast<_Float16>(y[leg_slot<KB>(1, 1)] * f),
+            static_cast<_Float16>(y[leg_slot<KB>(2, 0)] * f), static_cast<_Float16>(y[leg_slot<KB>(2, 1)] * f),
+            static_cast<_Float16>(y[leg_slot<KB>(3, 0)] * f), static_cast<_Float16>(y[leg_slot<KB>(3, 1)] * f)};
+        qop[m] = v;
+    }
+    qk = ldexpf(qk_scale, qex + leg_k_exp<KB>() + eb - 141);
+    constexpr uint32_t o = leg_k_offset<KB>() * 0x00010001u;
+    const u32x4 w = {o, o, o, o};
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < 4; ++m) acc = mfma_f16(__builtin_bit_cast(f16x8, w), qop[m], acc);
+    kbias = -acc;
+}
+
+// The query column scaled in place by 2^-qex, so that its largest channel
+// lies in [1, 2); returns qex (the same on the column's four lanes).
+__device__ __forceinline__ int legacy_norm_q(u32x4 (&q)[4]) {
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            amax = fmaxf(amax, fmaxf(fabsf(__uint_as_float(q[i][j] << 16)), fabsf(__uint_as_float(q[i][j] & 0xffff0000u))));
+    amax = col_max(amax);
+    const int qex = max(static_cast<int>(__float_as_uint(amax) >> 23), 1) - 127;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            w[j] = pack_bf16x2(ldexpf(__uint_as_float(q[i][j] << 16), -qex),
+                               ldexpf(__uint_as_float(q[i][j] & 0xffff0000u), -qex));
+        q[i] = u32x4{w[0], w[1], w[2], w[3]};
+    }
+    return qex;
+}
+
+// One chunk: scores, online softmax (the running sums tot rescaled with the
+// group's), P.V onto the group's accumulators st.acc / st.ones.
 template <int KB, int VB>
-__global__ __launch_bounds__(THREADS, 3) void legacy_decode_kernel(LegArgs a) {
+__device__ __forceinline__ void legacy_compute(WaveState& st, f32x4 (&tot)[8], const LegRaw<KB, VB>& r,
+                                               const f16x8 (&qop)[4], const f32x4& kbias, float qk, int nv, int lane) {
+    const int kb = lane >> 4;
+    float s[8];
+#pragma unroll
+    for (int tile = 0; tile < 2; ++tile) {
+        f32x4 acc = kbias;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc = mfma_f16(legacy_k_operand<KB>(r.k[tile], m), qop[m], acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[4 * tile + i] = acc[i] * qk;
+    }
+    if (nv < GROUP) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (slot_token(kb, e) >= nv) s[e] = -INFINITY;
+    }
+    const float m0 = st.m;
+    softmax_step<8>(st, s, true);
+    if (__builtin_amdgcn_ballot_w64(st.m != m0)) {
+        const float alpha = fast_exp2(m0 - st.m);
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) tot[nb] *= alpha;
+    }
+    const u32x4 pw = {pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]),
+                      pack_bf16x2(s[6], s[7])};
+    const bf16x8 pop = __builtin_bit_cast(bf16x8, pw);
+    uint32_t lo[4], hi[4];
+#pragma unroll
+    for (int pr = 0; pr < 4; ++pr) {
+        lo[pr] = perm(r.v[2 * pr + 1], r.v[2 * pr], 0x05040100u);
+        hi[pr] = VB == 4 ? perm(r.v[2 * pr + 1], r.v[2 * pr], 0x07060302u) : 0u;
+    }
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) {
+        // field nb of a row's dword is channel nb ^ 1 (nibbles) or nb ^ 3 (crumbs)
+        u32x4 w;
+        if constexpr (VB == 4) {
+            const uint32_t* src = nb < 4 ? lo : hi;
+            const int sh = 4 * (nb & 3);
+            w = u32x4{nib2(src[0], sh, 0x43004300u), nib2(src[1], sh, 0x43004300u), nib2(src[2], sh, 0x43004300u),
+                      nib2(src[3], sh, 0x43004300u)};
+        } else {
+            const int sh = 2 * nb;
+            w = u32x4{((lo[0] >> sh) & 0x00030003u) | 0x43004300u, ((lo[1] >> sh) & 0x00030003u) | 0x43004300u,
+                      ((lo[2] >> sh) & 0x00030003u) | 0x43004300u, ((lo[3] >> sh) & 0x00030003u) | 0x43004300u};
+        }
+        const int ch = VB == 4 ? nb ^ 1 : nb ^ 3;
+        st.acc[ch] = mfma_bf16(__builtin_bit_cast(bf16x8, w), pop, st.acc[ch]);
+    }
+    const u32x4 onesw = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+    st.ones = mfma_bf16(__builtin_bit_cast(bf16x8, onesw), pop, st.ones);
+}
+
+// The scale group's end: tot += s_v * (acc - offset * sum P), accumulators
+// cleared.  acc[nb][i] is channel 32kb + 8i + nb: element nb of vector i.
+template <int VB>
+__device__ __forceinline__ void legacy_flush(WaveState& st, f32x4 (&tot)[8], const u32x4 (&vs)[4]) {
+    const float corr = leg_v_offset<VB>() * st.ones[0];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) {
+            const float sc = f16_bits_to_f32(static_cast<uint16_t>((nb & 1) ? vs[i][nb >> 1] >> 16 : vs[i][nb >> 1]));
+            tot[nb][i] = __builtin_fmaf(st.acc[nb][i] - corr, sc, tot[nb][i]);
+        }
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) st.acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    st.ones = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+template <int KB, int VB, int BLK>
+__global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
 #ifdef HYQ_PHASE_TRACE
     uint64_t ph[TRACE_PH] = {};    // (the merge stamps; not stored by this kernel)
 #endif
@@ -1489,6 +1548,7 @@ __global__ __launch_bounds__(THREADS, 3) void legacy_decode_kernel(LegArgs a) {
     extern __shared__ float s_acc[];               // [WAVES][G][D+1]; later the merge weights
     __shared__ float s_m[WAVES][16];
     __shared__ float s_l[WAVES][16];
+    __shared__ u32x4 s_q[4][64];                   // the query column of each lane, scaled (prefix pieces)
     __shared__ int s_last;
 
     WaveState st;
@@ -1507,50 +1567,124 @@ __global__ __launch_bounds__(THREADS, 3) void legacy_decode_kernel(LegArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) qs[i] = bld128(rq, qo + 16 * i);
     }
-    const bf16x8 qb[4] = {__builtin_bit_cast(bf16x8, qs[0]), __builtin_bit_cast(bf16x8, qs[1]),
-                          __builtin_bit_cast(bf16x8, qs[2]), __builtin_bit_cast(bf16x8, qs[3])};
 
-    // this piece: segment sg (0: the prefix), tokens [lo, lo + n) of it
-    int sg = 0;
-    while (sg < 3 && wg >= a.pfirst[sg + 1]) ++sg;
-    const int lo = (wg - a.pfirst[sg]) * a.plen[sg];
-    const int seg_n = sg == 0 ? a.n_leg : a.sn[sg - 1];
-    const int n = max(0, min(a.plen[sg], seg_n - lo));
-    constexpr int TSTRIDE = WAVES * TILE;
-    const int ntile = (n + TILE - 1) / TILE;
-    const int nmine = ntile > wave ? (ntile - wave + WAVES - 1) / WAVES : 0;
-    const int t0 = wave * TILE;
-    if (sg == 0) {
-        const Rsrc rkc = make_rsrc(a.kc + head * a.kc_bh + lo * a.kc_n, static_cast<uint32_t>(n * a.kc_n));
-        const Rsrc rvc = make_rsrc(a.vc + head * a.vc_bh + lo * a.vc_n, static_cast<uint32_t>(n * a.vc_n));
-        const Rsrc rks = make_rsrc(a.ks + head * a.ks_bh, static_cast<uint32_t>(a.ks_rows * a.ks_g * 2));
-        const Rsrc rvs = make_rsrc(a.vs + head * a.vs_bh, static_cast<uint32_t>(a.vs_rows * a.vs_g * 2));
-        // tiles wave, wave+WAVES, ... through a two-deep register ring
-        const uint32_t kco = static_cast<uint32_t>(c * a.kc_n + 4 * KB * kb);
-        const uint32_t vco = static_cast<uint32_t>(4 * kb * a.vc_n + VB * c);
-        LegRaw<KB, VB> r0, r1;
-        Bf16Raw b;
-        constexpr float KF = KB == 4 ? 16.f : 8.f, VF = VB == 4 ? 16.f : 8.f;   // the operands are 1/KF, 1/VF of the values
-        const float qk16 = KF * a.qk_scale;
-        legacy_fetch(r0, a, rkc, rvc, rks, rvs, kco, vco, lo, t0, lane);
-        legacy_fetch(r1, a, rkc, rvc, rks, rvs, kco, vco, lo, t0 + TSTRIDE, lane);
-        for (int i = 0; i < nmine; i += 2) {
-            const int t = t0 + i * TSTRIDE;
-            legacy_dequant(b, r0);
-            bf16_compute(st, b, qb, n - t, lane, qk16);
-            if (i + 1 >= nmine) break;
-            legacy_fetch(r0, a, rkc, rvc, rks, rvs, kco, vco, lo, t + 2 * TSTRIDE, lane);
-            legacy_dequant(b, r1);
-            bf16_compute(st, b, qb, n - t - TSTRIDE, lane, qk16);
-            if (i + 2 >= nmine) break;
-            legacy_fetch(r1, a, rkc, rvc, rks, rvs, kco, vco, lo, t + 3 * TSTRIDE, lane);
+    const int u0 = a.bnd[wg], u1 = a.bnd[wg + 1];   // this piece's schedule units
+    if (u0 < a.nqg) {
+        // chunk x of the head: group x / cpg, tokens [x / cpg * group + 32 (x % cpg), ...)
+        const int cpg = a.cpg, group = a.group;
+        auto chunk_token = [&](int x) { return x / cpg * group + x % cpg * GROUP; };
+        const int x0 = u0 * BLK, x1 = min(u1, a.nqg) * BLK;
+        const int lo = chunk_token(x0);
+        const int n = min(a.n_leg, chunk_token(x1)) - lo;      // the piece's tokens
+        const uint32_t kc_n = static_cast<uint32_t>(a.kc_n), vc_n = static_cast<uint32_t>(a.vc_n);
+        const uint32_t ks_row = static_cast<uint32_t>(a.ks_g * 2), vs_row = static_cast<uint32_t>(a.vs_g * 2);
+        const Rsrc rk = make_rsrc(a.kc + head * a.kc_bh + lo * a.kc_n, static_cast<uint32_t>(n) * kc_n);
+        const Rsrc rv = make_rsrc(a.vc + head * a.vc_bh + lo * a.vc_n, static_cast<uint32_t>(n) * vc_n);
+        const Rsrc rks = make_rsrc(a.ks + head * a.ks_bh, static_cast<uint32_t>(a.ks_rows) * ks_row);
+        const Rsrc rvs = make_rsrc(a.vs + head * a.vs_bh, static_cast<uint32_t>(a.vs_rows) * vs_row);
+        const uint32_t klane = static_cast<uint32_t>(krow_token(c)) * kc_n + 4 * KB * kb;
+        const uint32_t vlane = static_cast<uint32_t>(kb) * vc_n + VB * c;
+        const int nblk = (x1 - x0) / BLK;
+        // first token (from lo) and scale group of block b of the piece
+        auto block_at = [&](int b, int& g) {
+            const int x = x0 + b * BLK;
+            g = __builtin_amdgcn_readfirstlane(x / cpg);
+            return __builtin_amdgcn_readfirstlane(g * group + (x - g * cpg) * GROUP - lo);
+        };
+        // tokens of the group (and the prefix) from chunk start t on
+        auto valid = [&](int t, int g) { return min((g + 1) * group, a.n_leg) - lo - t; };
+        f32x4 tot[8];
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) tot[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (BLK == 4) {
+            // a block's four chunks in four register slots
+            LegRaw<KB, VB> r[BLK];
+            u32x4 ksc[4], vsc[4];
+            int g = 0, gn = 0;
+            int t = block_at(wave, g), tn = 0;
+            legacy_scales(ksc, rks, g, ks_row, lane);
+#pragma unroll
+            for (int j = 0; j < BLK; ++j) {
+                legacy_fetch(r[j], rk, rv, klane, vlane, static_cast<uint32_t>(t + GROUP * j), kc_n, vc_n);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the query waits in LDS between the groups (its 16 registers do
+            // not fit beside the four slots)
+            const int qex = legacy_norm_q(qs);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (i == wave) s_q[i][lane] = qs[i];
+            __syncthreads();
+            for (int b = wave; b < nblk; b += WAVES) {
+                tn = block_at(b + WAVES, gn);          // past the piece: its loads read zeros
+                f16x8 qop[4];
+                f32x4 kbias;
+                float qk;
+                {
+                    const u32x4 qn[4] = {s_q[0][lane], s_q[1][lane], s_q[2][lane], s_q[3][lane]};
+                    legacy_q_operand<KB>(qop, kbias, qk, qn, ksc, a.qk_scale, qex);
+                }
+                legacy_scales(vsc, rvs, g, vs_row, lane);
+#pragma unroll
+                for (int j = 0; j < BLK; ++j) {
+                    legacy_compute<KB, VB>(st, tot, r[j], qop, kbias, qk, valid(t + GROUP * j, g), lane);
+                    legacy_fetch(r[j], rk, rv, klane, vlane, static_cast<uint32_t>(tn + GROUP * j), kc_n, vc_n);
+                    if (j == BLK / 2) legacy_scales(ksc, rks, gn, ks_row, lane);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                legacy_flush<VB>(st, tot, vsc);
+                t = tn;
+                g = gn;
+            }
+        } else {
+            // single chunks, each with its scale rows, in two slots
+            struct Slot {
+                LegRaw<KB, VB> r;
+                u32x4 ks[4], vs[4];
+                int t, g;
+            } x[2];
+            auto fetch = [&](Slot& y, int b) {
+                y.t = block_at(b, y.g);                // past the piece: its loads read zeros
+                legacy_scales(y.ks, rks, y.g, ks_row, lane);
+                legacy_fetch(y.r, rk, rv, klane, vlane, static_cast<uint32_t>(y.t), kc_n, vc_n);
+                legacy_scales(y.vs, rvs, y.g, vs_row, lane);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            fetch(x[0], wave);
+            fetch(x[1], wave + WAVES);
+            const int qex = legacy_norm_q(qs);
+            auto compute = [&](const Slot& y) {
+                f16x8 qop[4];
+                f32x4 kbias;
+                float qk;
+                legacy_q_operand<KB>(qop, kbias, qk, qs, y.ks, a.qk_scale, qex);
+                legacy_compute<KB, VB>(st, tot, y.r, qop, kbias, qk, valid(y.t, y.g), lane);
+                legacy_flush<VB>(st, tot, y.vs);
+            };
+            for (int b = wave; b < nblk; b += 2 * WAVES) {
+                compute(x[0]);
+                if (b + WAVES >= nblk) break;
+                fetch(x[0], b + 2 * WAVES);
+                compute(x[1]);
+                if (b + 2 * WAVES >= nblk) break;
+                fetch(x[1], b + 3 * WAVES);
+            }
         }
 #pragma unroll
-        for (int nb = 0; nb < 8; ++nb) st.acc[nb] *= VF;
+        for (int nb = 0; nb < 8; ++nb) st.acc[nb] = tot[nb];
     } else {
-        const int s3 = sg - 1;
-        const uint16_t* kbase = a.sk[s3] + head * a.sk_bh[s3] + static_cast<int64_t>(lo) * BROW;
-        const uint16_t* vbase = a.sv[s3] + head * a.sv_bh[s3] + static_cast<int64_t>(lo) * BROW;
+        const bf16x8 qb[4] = {__builtin_bit_cast(bf16x8, qs[0]), __builtin_bit_cast(bf16x8, qs[1]),
+                              __builtin_bit_cast(bf16x8, qs[2]), __builtin_bit_cast(bf16x8, qs[3])};
+        constexpr int TSTRIDE = WAVES * TILE;
+        const int t0 = wave * TILE;
+        const int b1 = a.nqg + a.segu[0], b2 = b1 + a.segu[1];
+        const int sg = u0 < b1 ? 0 : u0 < b2 ? 1 : 2;            // a piece lies inside one segment
+        const int lo = (u0 - (sg == 0 ? a.nqg : sg == 1 ? b1 : b2)) * BUNIT;
+        const int n = min((u1 - u0) * BUNIT, a.sn[sg] - lo);
+        const int ntile = (n + TILE - 1) / TILE;
+        const int nmine = ntile > wave ? (ntile - wave + WAVES - 1) / WAVES : 0;
+        const uint16_t* kbase = a.sk[sg] + head * a.sk_bh[sg] + static_cast<int64_t>(lo) * BROW;
+        const uint16_t* vbase = a.sv[sg] + head * a.sv_bh[sg] + static_cast<int64_t>(lo) * BROW;
         const uint32_t nbytes = static_cast<uint32_t>(n) * (BROW * 2);
         const Rsrc rk = make_rsrc(kbase, nbytes), rv = make_rsrc(vbase, nbytes);
         Bf16Raw r0, r1;
@@ -1646,9 +1780,20 @@ struct Slots {
 
 struct Plan {
     int nwg;               // pieces per head
-    int nqg, segu[3];      // schedule units: int4 groups, bf16 units per segment
+    int nqg, segu[3];      // schedule units: prefix units, bf16 units per segment
     int bnd[MAX_NWG + 1];  // piece p covers units [bnd[p], bnd[p+1])
 };
+
+// The prefix as schedule units: int4 groups of GROUP tokens, or the legacy
+// format's blocks.
+struct PrefixUnits {
+    int64_t units;
+    int tokens;            // per unit (full ones)
+    int64_t bytes;         // per unit
+};
+PrefixUnits group_units(int64_t n_quant, int kb, int vb) {
+    return {(n_quant + GROUP - 1) / GROUP, GROUP, static_cast<int64_t>(GROUP) * (16 * kb + 16 * vb + 4)};
+}
 
 size_t round256(size_t x) { return (x + 255) / 256 * 256; }
 
@@ -1750,13 +1895,12 @@ Pieces cheapest_pieces(const int64_t (&su)[4], const int64_t (&sc)[4], int bh_kv
     return best;
 }
 
-Plan make_plan(int64_t n_quant, const int64_t seg_n[3], int bh_kv, int G, int requested, int kb, int vb,
-               Slots sl_) {
+Plan make_plan(const PrefixUnits& pre, const int64_t seg_n[3], int bh_kv, int G, int requested, Slots sl_) {
     const int slots = sl_.slots;
     Plan p{};
-    p.nqg = static_cast<int>((n_quant + GROUP - 1) / GROUP);
+    p.nqg = static_cast<int>(pre.units);
     for (int s = 0; s < 3; ++s) p.segu[s] = static_cast<int>((seg_n[s] + BUNIT - 1) / BUNIT);
-    const int64_t cq = static_cast<int64_t>(GROUP) * (16 * kb + 16 * vb + 4);   // bytes of an int4 group
+    const int64_t cq = pre.bytes;                                               // bytes of a prefix unit
     const int64_t cb = static_cast<int64_t>(BUNIT) * 4 * D;                     // bytes of a bf16 unit (K and V)
     const int64_t su[4] = {p.nqg, p.segu[0], p.segu[1], p.segu[2]};             // units per segment
     const int64_t sc[4] = {cq, cb, cb, cb};
@@ -1786,7 +1930,7 @@ Plan make_plan(int64_t n_quant, const int64_t seg_n[3], int bh_kv, int G, int re
     int64_t target;
     const bool twelve = G > 8 && bh_kv >= 20 && bh_kv <= 64 && head_bytes * bh_kv >= 60000000;
     if (requested > 0) {
-        target = std::max<int64_t>(1, (requested + GROUP - 1) / GROUP) * cq;
+        target = std::max<int64_t>(1, (requested + pre.tokens - 1) / pre.tokens) * cq;
         total = counts_for(target);
     } else if (bh_kv < 32 && G <= WAVES) {
         // few heads, G <= 4: pieces of equal bytes, about 0.8 per CU (a
@@ -1847,23 +1991,26 @@ int merge_batch(int G, int nwg) {
     return 124;
 }
 
-// Workgroups of one decode_kernel instance the device holds at once (and
-// the device's CU count), cached per device and GQA width (the LDS size).
-template <int KB, int VB>
-Slots resident_slots_of(int G) {
-    static std::atomic<int> cache[64][17][2];
+// Workgroups of a decode kernel the device holds at once (and the device's
+// CU count), cached per device and GQA width (the LDS size).
+Slots slots_of(const void* kernel, std::atomic<int> (&cache)[64][17][2], int G) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 || G < 1 || G > 16) return {0, 0};
     const int known = cache[dev][G][0].load(std::memory_order_relaxed);
     if (known > 0) return {known, cache[dev][G][1].load(std::memory_order_relaxed)};
     int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&decode_kernel<KB, VB>),
-                                                     THREADS, lds_bytes(G)) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, THREADS, lds_bytes(G)) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return {0, 0};
     cache[dev][G][1].store(cus, std::memory_order_relaxed);
     cache[dev][G][0].store(per_cu * cus, std::memory_order_relaxed);
     return {per_cu * cus, cus};
+}
+
+template <int KB, int VB>
+Slots resident_slots_of(int G) {
+    static std::atomic<int> cache[64][17][2];
+    return slots_of(reinterpret_cast<const void*>(&decode_kernel<KB, VB>), cache, G);
 }
 
 Slots resident_slots(int kb, int vb, int G) {
@@ -1882,7 +2029,7 @@ Slots resident_slots(int kb, int vb, int G) {
 
 Plan plan_for(const hyq_decode_params* p) {
     const int kb = p->n_quant > 0 ? p->k_bits : 4, vb = p->n_quant > 0 ? p->v_bits : 4;
-    return make_plan(p->n_quant, p->seg_n, p->bh_kv, p->kv_repeat, p->split_tokens, kb, vb,
+    return make_plan(group_units(p->n_quant, kb, vb), p->seg_n, p->bh_kv, p->kv_repeat, p->split_tokens,
                      resident_slots(kb, vb, p->kv_repeat));
 }
 
@@ -1956,71 +2103,54 @@ int validate(const hyq_decode_params* p) {
 }
 
 // ---- legacy-format decode: plan and checks ----
-struct LegPlan {
-    int nwg = 0;
-    int pfirst[5] = {0, 0, 0, 0, 0};
-    int plen[4] = {LEG_PIECE, BF_PIECE, BF_PIECE, BF_PIECE};
-};
-// Workgroups of legacy_decode_kernel<KB, VB> the device holds at once (0:
-// unknown), cached per device, variant and GQA width (the LDS size).
-template <int KB, int VB>
-int legacy_slots_of(int G) {
-    static std::atomic<int> cache[64][17];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 || G < 1 || G > 16) return 0;
-    const int known = cache[dev][G].load(std::memory_order_relaxed);
-    if (known > 0) return known;
-    int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(&legacy_decode_kernel<KB, VB>), THREADS, lds_bytes(G)) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return 0;
-    cache[dev][G].store(per_cu * cus, std::memory_order_relaxed);
-    return per_cu * cus;
+// Scale-group length as the kernel walks it: a group that covers the whole
+// prefix is cut to the prefix (rounded up to chunks).
+int legacy_group(const hyq_legacy_params* p) {
+    const int64_t whole = (p->n + GROUP - 1) / GROUP * GROUP;
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(p->group, whole)));
 }
-int legacy_slots(int kb, int vb, int G) {
-    switch (10 * kb + vb) {
-        case 44: return legacy_slots_of<4, 4>(G);
-        case 42: return legacy_slots_of<4, 2>(G);
-        case 24: return legacy_slots_of<2, 4>(G);
-        default: return legacy_slots_of<2, 2>(G);
+// Chunks per block: four, which share one folding of the scales, when the
+// group's chunk count is a multiple of four (128-token groups) and one
+// workgroup per CU gets a block for each of its wavefronts; else single
+// chunks, which spread a short cache over more wavefronts (8 KV heads at 1100
+// tokens, kernel time: 7.8 us with single chunks, 9.5 us with blocks of four;
+// at 31000 tokens, where the rule changes over, 16.6 us with blocks against
+// 20.5 us for dequantising every element).
+int legacy_blk(const hyq_legacy_params* p, int cus) {
+    const int64_t cpg = (legacy_group(p) + GROUP - 1) / GROUP;
+    return cpg % 4 == 0 && p->n / (4 * GROUP) * p->bh_kv >= WAVES * (cus > 0 ? cus : 256) ? 4 : 1;
+}
+
+template <int KB, int VB, int BLK>
+Slots legacy_slots_of(int G) {
+    static std::atomic<int> cache[64][17][2];
+    return slots_of(reinterpret_cast<const void*>(&legacy_decode_kernel<KB, VB, BLK>), cache, G);
+}
+Slots legacy_slots(int kb, int vb, int blk, int G) {
+    switch (100 * kb + 10 * vb + blk) {
+        case 444: return legacy_slots_of<4, 4, 4>(G);
+        case 424: return legacy_slots_of<4, 2, 4>(G);
+        case 244: return legacy_slots_of<2, 4, 4>(G);
+        case 224: return legacy_slots_of<2, 2, 4>(G);
+        case 441: return legacy_slots_of<4, 4, 1>(G);
+        case 421: return legacy_slots_of<4, 2, 1>(G);
+        case 241: return legacy_slots_of<2, 4, 1>(G);
+        default: return legacy_slots_of<2, 2, 1>(G);
     }
 }
 
-// Pieces grow while the prefix alone would still hand every resident slot a
-// piece after the doubling: a piece carries a fixed cost (the Q load, the
-// partial store, the arrival and merge), and a 512-token piece is only four
-// two-tile iterations per wave.  Measured on one MI355X (128 key heads,
-// 31000 tokens): 209 us with 512-token pieces, 187 us with 1024, 176 us with
-// 2048; with 8 key heads 2048-token pieces left most CUs idle (33 us against
-// 23 us).
-LegPlan legacy_plan(const hyq_legacy_params* p) {
-    LegPlan pl;
-    const int64_t n[4] = {p->n, p->seg_n[0], p->seg_n[1], p->seg_n[2]};
-    const int sl = legacy_slots(p->k_bits, p->v_bits, p->kv_repeat);
-    const int64_t slots = sl > 0 ? sl : 768;
-    // few heads: halve the pieces (down to 128 prefix tokens) while the grid
-    // would leave CUs without a workgroup (slots / 3: one per CU)
-    auto pieces = [&]() {
-        int64_t t = 0;
-        for (int s = 0; s < 4; ++s) t += (n[s] + pl.plen[s] - 1) / pl.plen[s];
-        return t * p->bh_kv;
-    };
-    while (pl.plen[0] > LEG_PIECE_MIN && pieces() < slots / 3)
-        for (int s = 0; s < 4; ++s) pl.plen[s] /= 2;
-    while (pl.plen[0] < LEG_PIECE_MAX &&
-           static_cast<int64_t>(p->bh_kv) * ((n[0] + 2 * pl.plen[0] - 1) / (2 * pl.plen[0])) >= slots)
-        for (int s = 0; s < 4; ++s) pl.plen[s] *= 2;
-    for (;;) {
-        int64_t total = 0;
-        for (int s = 0; s < 4; ++s) total += (n[s] + pl.plen[s] - 1) / pl.plen[s];
-        if (total <= MAX_NWG && total * p->kv_repeat <= MAX_PARTIALS) break;
-        for (int s = 0; s < 4; ++s) pl.plen[s] *= 2;
+Plan legacy_plan(const hyq_legacy_params* p) {
+    PrefixUnits pre{0, GROUP, 1};
+    int blk = 4;
+    if (p->n > 0) {
+        const int group = legacy_group(p);
+        blk = legacy_blk(p, legacy_slots(p->k_bits, p->v_bits, 4, p->kv_repeat).cus);
+        const int64_t cpg = (group + GROUP - 1) / GROUP, full = p->n / group, rest = p->n - full * group;
+        pre.units = full * (cpg / blk) + ((rest + GROUP - 1) / GROUP + blk - 1) / blk;
+        pre.tokens = blk * GROUP;
+        pre.bytes = static_cast<int64_t>(pre.tokens) * (16 * p->k_bits + 16 * p->v_bits) + 4 * D;
     }
-    for (int s = 0; s < 4; ++s)
-        pl.pfirst[s + 1] = pl.pfirst[s] + static_cast<int>((n[s] + pl.plen[s] - 1) / pl.plen[s]);
-    pl.nwg = pl.pfirst[4];
-    return pl;
+    return make_plan(pre, p->seg_n, p->bh_kv, p->kv_repeat, 0, legacy_slots(p->k_bits, p->v_bits, blk, p->kv_repeat));
 }
 
 int validate_legacy(const hyq_legacy_params* p) {
@@ -2075,16 +2205,19 @@ int validate_legacy(const hyq_legacy_params* p) {
     return HYQ_OK;
 }
 
-int launch_legacy(const hyq_legacy_params* p, const LegPlan& pl, const Layout& L, void* workspace, void* stream) {
+int launch_legacy(const hyq_legacy_params* p, const Plan& pl, const Layout& L, void* workspace, void* stream) {
     LegArgs a{};
     a.q = p->q; a.q_stride = p->q_stride;
     a.kc = p->k_codes; a.vc = p->v_codes;
     a.kc_bh = p->kc_stride_bh; a.kc_n = p->kc_stride_n; a.vc_bh = p->vc_stride_bh; a.vc_n = p->vc_stride_n;
     a.ks = p->k_scale; a.vs = p->v_scale;
     a.ks_bh = p->ks_stride_bh; a.ks_g = p->ks_stride_g; a.vs_bh = p->vs_stride_bh; a.vs_g = p->vs_stride_g;
-    a.group = p->n > 0 ? p->group : 1;
+    a.group = p->n > 0 ? legacy_group(p) : GROUP;
     a.ks_rows = a.vs_rows = (p->n + a.group - 1) / a.group;
     a.n_leg = static_cast<int>(p->n);
+    a.cpg = (a.group + GROUP - 1) / GROUP;
+    a.nqg = pl.nqg;
+    a.segu[0] = pl.segu[0]; a.segu[1] = pl.segu[1];
     for (int s = 0; s < 3; ++s) {
         a.sk[s] = p->seg_k[s]; a.sv[s] = p->seg_v[s];
         a.sk_bh[s] = p->seg_k_stride_bh[s]; a.sv_bh[s] = p->seg_v_stride_bh[s];
@@ -2099,16 +2232,19 @@ int launch_legacy(const hyq_legacy_params* p, const LegPlan& pl, const Layout& L
     a.out = p->out; a.out_stride = p->out_stride;
     a.nwg = pl.nwg;
     a.mj = merge_batch(a.G, pl.nwg);
-    for (int s = 0; s < 5; ++s) a.pfirst[s] = pl.pfirst[s];
-    for (int s = 0; s < 4; ++s) a.plen[s] = pl.plen[s];
+    for (int i = 0; i <= pl.nwg; ++i) a.bnd[i] = pl.bnd[i];
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 grid(static_cast<unsigned>(p->bh_kv), static_cast<unsigned>(pl.nwg));
     const size_t lds = lds_bytes(a.G);
-    switch (10 * p->k_bits + p->v_bits) {
-        case 44: legacy_decode_kernel<4, 4><<<grid, dim3(THREADS), lds, st>>>(a); break;
-        case 42: legacy_decode_kernel<4, 2><<<grid, dim3(THREADS), lds, st>>>(a); break;
-        case 24: legacy_decode_kernel<2, 4><<<grid, dim3(THREADS), lds, st>>>(a); break;
-        default: legacy_decode_kernel<2, 2><<<grid, dim3(THREADS), lds, st>>>(a); break;
+    switch (100 * p->k_bits + 10 * p->v_bits + legacy_blk(p, legacy_slots(p->k_bits, p->v_bits, 4, a.G).cus)) {
+        case 444: legacy_decode_kernel<4, 4, 4><<<grid, dim3(THREADS), lds, st>>>(a); break;
+        case 424: legacy_decode_kernel<4, 2, 4><<<grid, dim3(THREADS), lds, st>>>(a); break;
+        case 244: legacy_decode_kernel<2, 4, 4><<<grid, dim3(THREADS), lds, st>>>(a); break;
+        case 224: legacy_decode_kernel<2, 2, 4><<<grid, dim3(THREADS), lds, st>>>(a); break;
+        case 441: legacy_decode_kernel<4, 4, 1><<<grid, dim3(THREADS), lds, st>>>(a); break;
+        case 421: legacy_decode_kernel<4, 2, 1><<<grid, dim3(THREADS), lds, st>>>(a); break;
+        case 241: legacy_decode_kernel<2, 4, 1><<<grid, dim3(THREADS), lds, st>>>(a); break;
+        default: legacy_decode_kernel<2, 2, 1><<<grid, dim3(THREADS), lds, st>>>(a); break;
     }
     return check_launch("hyq_decode_legacy");
 }
@@ -2279,7 +2415,7 @@ extern "C" int hyq_phase_trace_geometry(int32_t* slots, int32_t* max_wg, int32_t
 extern "C" size_t hyq_decode_bf16_workspace_size(int32_t bh_kv, int32_t kv_repeat, int64_t n, int32_t d) {
     if (bh_kv < 0 || kv_repeat < 1 || kv_repeat > 16 || d != D || n < 0) return 0;
     const int64_t seg_n[3] = {n, 0, 0};
-    const Plan pl = make_plan(0, seg_n, bh_kv, kv_repeat, 0, 4, 4, resident_slots(4, 4, kv_repeat));
+    const Plan pl = make_plan(group_units(0, 4, 4), seg_n, bh_kv, kv_repeat, 0, resident_slots(4, 4, kv_repeat));
     return layout(pl, bh_kv, kv_repeat).total;
 }
 
@@ -2300,18 +2436,14 @@ extern "C" int hyq_decode_bf16(const uint16_t* q, int64_t q_stride, uint16_t* ou
 
 extern "C" size_t hyq_decode_legacy_workspace_size(const hyq_legacy_params* p) {
     if (validate_legacy(p) != HYQ_OK || p->bh_kv == 0) return 0;
-    Plan dp{};
-    dp.nwg = legacy_plan(p).nwg;
-    return layout(dp, p->bh_kv, p->kv_repeat).total;
+    return layout(legacy_plan(p), p->bh_kv, p->kv_repeat).total;
 }
 
 extern "C" int hyq_decode_legacy(const hyq_legacy_params* p, void* workspace, size_t ws_bytes, void* stream) {
     int rc = validate_legacy(p);
     if (rc != HYQ_OK || p->bh_kv == 0) return rc;
-    const LegPlan pl = legacy_plan(p);
-    Plan dp{};
-    dp.nwg = pl.nwg;
-    const Layout L = layout(dp, p->bh_kv, p->kv_repeat);
+    const Plan pl = legacy_plan(p);
+    const Layout L = layout(pl, p->bh_kv, p->kv_repeat);
     if (!workspace || ws_bytes < L.total || !aligned(workspace, 256))
         return fail(HYQ_ENOSPC, "hyq_decode_legacy: workspace too small or misaligned: need " + std::to_string(L.total) + " bytes");
     return launch_legacy(p, pl, L, workspace, stream);

@@ -15,14 +15,15 @@ Drop-in for its entry points:
   per query head and a `[B, H, W, D]` window.
 
 `hyq_decode_legacy` reads the legacy prefix directly (K and V of 4 or 2
-bits, as the reference's MMA variant takes them, :977-1092): each tile's
-codes and group scales are dequantised in registers to the bf16 values of
-`legacy_dequantize`, and the prefix and the three bf16 segments go through
-one softmax.  For the per-token format the prefix is dequantised to the
-model dtype first (`hyq_dequant`), as the reference's legacy path A does
-(:1-8).  The operand roundings are those of the reference's MMA variant: K
-and V of the prefix rounded to bf16, P rounded to bf16 for the P.V product,
-fp32 accumulation.
+bits, as the reference's MMA variant takes them, :977-1092): the codes go to
+the matrix cores exactly, K's group scales folded into the query (fp32
+product, rounded once to fp16) and V's applied to each group's fp32 sum, and
+the prefix and the three bf16 segments go through one softmax.  For the
+per-token format the prefix is dequantised to the model dtype first
+(`hyq_dequant`), as the reference's legacy path A does (:1-8).  The
+reference's MMA variant rounds K and V of the prefix to bf16 (2^-9 each);
+here only the query's product with the scales is rounded (2^-12).  P is
+rounded to bf16 for the P.V product, accumulation is fp32.
 `split_size` / `block_kv` are the reference's tuning knobs and do not change
 the result; they are accepted and ignored.  The model dtype must be bf16.
 """
@@ -35,8 +36,8 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .decode_d_stage import (GROUP_SIZE, _decode, _inner_contig, _packed_dim, _require_gpu, _stream,
-                             _workspace, dequantize_per_token)
+from .decode_d_stage import (GROUP_SIZE, _decode, _inner_contig, _packed_dim, _require_gpu, _stream, _workspace,
+                             _ws_cache, dequantize_per_token)
 
 __all__ = [
     "legacy_dequantize",
@@ -114,8 +115,7 @@ def _legacy_decode(q, k_quant_packed, v_quant_packed, k_scale, v_scale, k_topk, 
 
 def _legacy_direct(q, kp, vp, ks, vs, N_q, BH_KV, segs, kv_repeat, k_bits, v_bits, sm_scale, what):
     """hyq_decode_legacy reads the legacy codes (K and V of 4 or 2 bits) and
-    their group scales directly (dequantised in registers to the bf16 values
-    of legacy_dequantize) together with the three bf16 segments, one
+    their group scales directly, together with the three bf16 segments, one
     softmax."""
     B, H_Q, _, D = q.shape
     L = _lib.lib()
@@ -162,9 +162,13 @@ def _legacy_direct(q, kp, vp, ks, vs, N_q, BH_KV, segs, kv_repeat, k_bits, v_bit
     p.bh_kv, p.kv_repeat, p.head_dim = BH_KV, kv_repeat, D
     p.sm_scale = D ** -0.5 if sm_scale is None else float(sm_scale)
     stream = _stream(q.device)
-    need = L.hyq_decode_legacy_workspace_size(ctypes.byref(p))
-    ws = _workspace(q.device, stream, max(need, 1))
-    st = L.hyq_decode_legacy(ctypes.byref(p), ws.data_ptr(), ws.numel(), stream)
+    # the stream's workspace as it is; one too small is refused before anything is launched
+    ws = _ws_cache.get((q.device.index, stream))
+    st = L.hyq_decode_legacy(ctypes.byref(p), None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+                             stream)
+    if st == _lib.HYQ_ENOSPC:
+        ws = _workspace(q.device, stream, L.hyq_decode_legacy_workspace_size(ctypes.byref(p)))
+        st = L.hyq_decode_legacy(ctypes.byref(p), ws.data_ptr(), ws.numel(), stream)
     _lib.check(st, what)
     return out.view(B, H_Q, 1, D)
 

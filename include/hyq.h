@@ -167,11 +167,10 @@ int hyq_decode_hybrid_noalloc(const hyq_decode_params* p, void* stream);
  * fused_decode_attention_k4v4 (src/ops/d_stage_cache.py:504-591),
  * splitk_decode_attention_k4v4 (:825-951) and
  * splitk_decode_attention_k4v4_mma (:1247-1366, K_BITS / V_BITS of 4 or 2):
- * the prefix codes and their per-(group, channel) fp16 scales are
- * dequantised in registers to the bf16 values of hyq_legacy_dequant (up to
- * an exact power of two that the kernel compensates), and attention runs
- * with bf16 K/V and P operands and fp32 accumulation, over the prefix and
- * three bf16 segments (top-k, staging, window), one softmax.  Codes are
+ * the prefix codes are exact operands, the K scales of their (group, channel)
+ * are folded into the query (fp32 product, rounded once to fp16), the V scales
+ * into each group's fp32 sum; P is rounded to bf16, sums are fp32; one softmax
+ * over the prefix and three bf16 segments (top-k, staging, window).  Codes are
  * offset-encoded: int4 has channel 2j in the HIGH nibble of byte j, value
  * u - 8; int2 has channel 4j + i in bits 7-2i..6-2i of byte j, value u - 1.5.
  *   q, out    bf16 [bh_kv * kv_repeat, 128] (row strides)
