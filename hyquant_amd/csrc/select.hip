@@ -759,6 +759,9 @@ constexpr int TOPK_RANK_MAX = 2048;        // winners the rank path's per-thread
 constexpr int TOPK_RANK_LIMIT = 512;
 // key offsets above the candidate bound that the counting rank covers
 constexpr int TOPK_SPAN = 1024;
+// a bucket of the counting rank with more entries than this is ranked through
+// a bitmap of its positions
+constexpr uint32_t TOPK_BIG = 128;
 constexpr size_t TOPK_LDS_MAX = 64 * 1024; // keys are cached in LDS while the row fits this budget
 
 // Wavefront 0: the bin holding the need-th largest entry of an NBINS-bin
@@ -1098,6 +1101,7 @@ __global__ __launch_bounds__(NT) void topk_kernel(TopkArgs a) {
     __shared__ uint32_t s_bin, s_need, s_count, s_total, s_ovf;
     __shared__ uint32_t s_wtot[(NT / 64)];
     __shared__ uint32_t s_lohist[64];
+    __shared__ uint32_t s_big[64], s_nbig;
     __shared__ double s_q[128];
     const int row = blockIdx.x;
     const int tid = threadIdx.x;
@@ -1251,12 +1255,22 @@ __global__ __launch_bounds__(NT) void topk_kernel(TopkArgs a) {
                 // its key's bucket, a bucket's first rank is the number of
                 // entries with larger keys, and inside a bucket the larger
                 // composite (the lower index) comes first.  The entries ranked
-                // below T are the winners, each written at its rank.
+                // below T are the winners, each written at its rank.  Inside a
+                // bucket of up to TOPK_BIG entries a thread compares its entry
+                // with all of them; a larger one (equal scores: repeated or
+                // near-parallel keys) would cost n^2 / NT steps, so its
+                // positions are set in a bitmap of the row and an entry's rank
+                // is the number of set bits below it (1638 equal keys of 32640
+                // positions, 32 rows: 112 -> 27 us for the kernel;
+                // 806 of 16128, 1024 rows: 97 -> 50 us).
                 {
                     uint32_t* bcnt = brk;                   // bucket counts (then fill counters)
                     uint32_t* bstart = brk + TOPK_SPAN;     // first rank of each bucket
                     for (int i = tid; i < TOPK_SPAN; i += NT) bcnt[i] = 0;
-                    if (tid == 0) s_ovf = 0;
+                    if (tid == 0) {
+                        s_ovf = 0;
+                        s_nbig = 0;
+                    }
                     __syncthreads();
                     for (uint32_t i = tid; i < cnt; i += NT) {
                         const uint32_t key = static_cast<uint32_t>(list[i] >> Comp<C>::IDX_BITS);
@@ -1299,13 +1313,64 @@ __global__ __launch_bounds__(NT) void topk_kernel(TopkArgs a) {
                             if (key >= L) brank_tmp[bstart[key - L] + atomicAdd(&bcnt[key - L], 1u)] = c;
                         }
                         __syncthreads();
+                        // large buckets through bitmaps (in the list's space, which is
+                        // free once the buckets are filled: P / 32 words of bits, then
+                        // the set bits before each word)
+                        const uint32_t words = static_cast<uint32_t>((a.P + 31) / 32);
+                        const bool maps = 2 * static_cast<int64_t>(words) <= static_cast<int64_t>(a.cap) * static_cast<int>(sizeof(C) / 4);
+                        if (maps) {
+                            for (int i = tid; i < TOPK_SPAN; i += NT)
+                                if (bcnt[i] > TOPK_BIG && bstart[i] < static_cast<uint32_t>(a.T)) {
+                                    const uint32_t slot = atomicAdd(&s_nbig, 1u);
+                                    if (slot < 64) s_big[slot] = static_cast<uint32_t>(i);
+                                }
+                        }
+                        __syncthreads();
+                        const uint32_t nbig = min(s_nbig, 64u);
+                        uint32_t* bits = reinterpret_cast<uint32_t*>(list);
+                        uint32_t* before = bits + words;
+                        for (uint32_t u = 0; u < nbig; ++u) {
+                            const uint32_t s0 = bstart[s_big[u]], n = bcnt[s_big[u]];
+                            for (uint32_t i = tid; i < words; i += NT) bits[i] = 0;
+                            __syncthreads();
+                            for (uint32_t j = tid; j < n; j += NT) {
+                                const uint32_t idx = static_cast<uint32_t>(Comp<C>::index(brank_tmp[s0 + j]));
+                                atomicOr(&bits[idx >> 5], 1u << (idx & 31));
+                            }
+                            __syncthreads();
+                            const uint32_t per = (words + NT - 1) / NT, w0 = min(words, tid * per), w1 = min(words, w0 + per);
+                            uint32_t mine = 0;
+                            for (uint32_t i = w0; i < w1; ++i) mine += __popc(bits[i]);
+                            uint32_t run = mine;
+#pragma unroll
+                            for (int off = 1; off < 64; off <<= 1) {
+                                const uint32_t o = __shfl_up(run, off, 64);
+                                if (lane >= off) run += o;
+                            }
+                            if (lane == 63) s_wtot[wave] = run;
+                            __syncthreads();
+                            run -= mine;
+                            for (int w = 0; w < wave; ++w) run += s_wtot[w];
+                            for (uint32_t i = w0; i < w1; ++i) {
+                                before[i] = run;
+                                run += __popc(bits[i]);
+                            }
+                            __syncthreads();
+                            for (uint32_t j = tid; j < n; j += NT) {
+                                const uint32_t idx = static_cast<uint32_t>(Comp<C>::index(brank_tmp[s0 + j]));
+                                const uint32_t r = s0 + before[idx >> 5] + __popc(bits[idx >> 5] & ((1u << (idx & 31)) - 1u));
+                                if (r < static_cast<uint32_t>(a.T)) orow[r] = idx;
+                            }
+                            __syncthreads();
+                        }
                         // the entries at or above L, bucket by bucket (the fill counters are the counts again)
+                        const bool small_only = maps && s_nbig <= 64u;   // every large bucket is placed
                         const uint32_t tot = bstart[0] + bcnt[0];
                         for (uint32_t pos = tid; pos < tot; pos += NT) {
                             const C c = brank_tmp[pos];
                             const uint32_t off = static_cast<uint32_t>(c >> Comp<C>::IDX_BITS) - L;
                             const uint32_t s0 = bstart[off], n = bcnt[off];
-                            if (s0 >= static_cast<uint32_t>(a.T)) continue;
+                            if (s0 >= static_cast<uint32_t>(a.T) || (small_only && n > TOPK_BIG)) continue;
                             uint32_t rin = 0;
                             for (uint32_t j = 0; j < n; ++j) rin += brank_tmp[s0 + j] > c;
                             if (s0 + rin < static_cast<uint32_t>(a.T)) orow[s0 + rin] = Comp<C>::index(c);
