@@ -701,6 +701,7 @@ __device__ __forceinline__ float wave_sum64(float v) {
 // every call gives the same result.
 struct MergeArgs {
     int G, nwg;
+    int64_t first;         // slot of the head's first partial
     const float* part;
     const float* ml;
     uint16_t* out;
@@ -748,8 +749,8 @@ __device__ __forceinline__ void merge_head_waves(const MergeArgs& a, int head, f
     HYQ_STAMP(11);
     const int h = lane >> 5, q = lane & 31;
     const int npair = P * G;
-    const Rsrc rp = make_rsrc(a.part + static_cast<int64_t>(head) * npair * D, static_cast<uint32_t>(npair) * D * 4);
-    const Rsrc rm = make_rsrc(a.ml + static_cast<int64_t>(head) * npair * 2, static_cast<uint32_t>(npair) * 8);
+    const Rsrc rp = make_rsrc(a.part + a.first * G * D, static_cast<uint32_t>(npair) * D * 4);
+    const Rsrc rm = make_rsrc(a.ml + a.first * G * 2, static_cast<uint32_t>(npair) * 8);
     float* wt = lds + g * MAX_NWG;
     // (m, l) of partials lane, lane + 64, ... (past nwg: out of range, zeros);
     // the host's choice of MJ covers every partial in one batch when nwg <=
@@ -820,8 +821,8 @@ __device__ __forceinline__ void merge_head_cols(const MergeArgs& a, int head, fl
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int npair = P * G;
-    const Rsrc rp = make_rsrc(a.part + static_cast<int64_t>(head) * npair * D, static_cast<uint32_t>(npair) * D * 4);
-    const Rsrc rm = make_rsrc(a.ml + static_cast<int64_t>(head) * npair * 2, static_cast<uint32_t>(npair) * 8);
+    const Rsrc rp = make_rsrc(a.part + a.first * G * D, static_cast<uint32_t>(npair) * D * 4);
+    const Rsrc rm = make_rsrc(a.ml + a.first * G * 2, static_cast<uint32_t>(npair) * 8);
     const int NC = G * (D / 4);
     const bool two = NC > THREADS;                       // G > 8
     const int TPC = two ? 1 : THREADS / NC;
@@ -922,20 +923,176 @@ constexpr int merge_items(int G, int nwg) {
     return 32 * G > THREADS ? 2 * nwg : (nwg + THREADS / (32 * G) - 1) / (THREADS / (32 * G));
 }
 
+// The merge instance: for G <= 4 merge_head_waves with the smallest batch
+// covering a lane's partial pairs (else batches of 24); for G > 4
+// merge_head_cols (100 + batch) with the smallest batch covering a thread's
+// items (else batches of 24).
+__host__ __device__ inline int merge_batch(int G, int nwg) {
+    if (G <= WAVES) {
+        const int pairs = (nwg + 1) / 2;
+        return pairs <= 24 ? (pairs + 3) / 4 * 4 : 24;
+    }
+    const int items = merge_items(G, nwg);
+    return items <= 8 ? 108 : items <= 16 ? 116 : 124;
+}
+
+// ---------------------------------------------------------------------------
+// ragged lengths: the pieces planned on the device
+// ---------------------------------------------------------------------------
+// With per-head lengths only the device knows how much there is to read: cut
+// by the longest head, 16 sequences of 700 to 32000 tokens (28% of the padded
+// tokens) left three quarters of the pieces empty and the rest as large as a
+// full batch's.  So every workgroup of a ragged launch reads all lengths (at
+// most RAGGED_HEADS heads, four per thread), forms the same totals and piece
+// sizes, numbers the pieces (int4 pieces of all heads, then bf16 pieces) by a
+// prefix sum and takes the piece of its own number; workgroups past the last
+// piece leave.  Piece size, with `cus` and `slots` as in make_plan: 4/5 of a
+// piece per CU below 48 MB, 5/4 per resident slot above (of at least 96 KiB),
+// at least 16 KiB, and large enough for the merge tables and, with G > 4, for
+// the merge to load a head's partials in one or two batches.  The grid covers
+// any lengths (ragged_grid).  That batch, 32 query heads on 8 key heads, K4V4:
+// 62.8 us by the padded plan, 41.0 us by this one.
+constexpr int RAGGED_HEADS = 4 * THREADS;
+
+// pieces a ragged launch can have: total / target, and one rounded up per
+// head and segment
+__host__ __device__ inline int ragged_grid(int bh, int cus, int slots) {
+    const int a = cus * 4 / 5, b = slots * 5 / 4;
+    return (a > b ? a : b) + 1 + 2 * bh;
+}
+
+struct RaggedPiece {
+    int head, piece, pieces;   // head -1: no piece of this number
+    int first;                 // slot of the head's first partial
+    int u0, u1, nqg, nb;       // schedule units: the piece's, and the head's int4 and bf16 units
+};
+
+template <int KB, int VB>
+__device__ __forceinline__ RaggedPiece ragged_piece(int bh, int G, int nquant, int sn0, const int32_t* len_q,
+                                                    const int32_t* len_s0, int cus, int slots) {
+    constexpr int CQ = GROUP * (16 * KB + 16 * VB + 4), CB = BUNIT * 4 * D;   // bytes per unit
+    __shared__ uint32_t s_sum[WAVES][2];
+    __shared__ float s_max[WAVES];
+    __shared__ uint32_t s_pieces[WAVES];
+    __shared__ int s_out[8];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    uint32_t nq[4], nb[4], sq = 0, sb = 0;
+    float mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int h = 4 * t + i;
+        int lq = 0, lb = 0;
+        if (h < bh) {
+            lq = len_q ? min(nquant, max(0, len_q[h])) : nquant;
+            lb = len_s0 ? min(sn0, max(0, len_s0[h])) : sn0;
+        }
+        nq[i] = static_cast<uint32_t>(lq + GROUP - 1) / GROUP;
+        nb[i] = static_cast<uint32_t>(lb + BUNIT - 1) / BUNIT;
+        sq += nq[i];
+        sb += nb[i];
+        mx = fmaxf(mx, static_cast<float>(nq[i]) * CQ + static_cast<float>(nb[i]) * CB);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        sq += __shfl_xor(sq, off, 64);
+        sb += __shfl_xor(sb, off, 64);
+        mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    }
+    if (lane == 0) {
+        s_sum[wave][0] = sq;
+        s_sum[wave][1] = sb;
+        s_max[wave] = mx;
+    }
+    __syncthreads();
+    sq = sb = 0;
+    mx = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        sq += s_sum[w][0];
+        sb += s_sum[w][1];
+        mx = fmaxf(mx, s_max[w]);
+    }
+    const float total = static_cast<float>(sq) * CQ + static_cast<float>(sb) * CB;
+    float target = total < 48e6f ? total / static_cast<float>(cus * 4 / 5)
+                                 : fmaxf(98304.f, total / static_cast<float>(slots * 5 / 4));
+    const int most = G > 8 ? 24 : G > WAVES ? 24 : MAX_PARTIALS / 16;       // pieces per head (below the tables' limits)
+    target = fmaxf(fmaxf(target, 16384.f), mx / static_cast<float>(most - 3));
+    const uint32_t uq = static_cast<uint32_t>(target / CQ) + 1, ub = static_cast<uint32_t>(target / CB) + 1;
+    uint32_t pc[4], sum = 0;                          // pieces: int4 in the low half, bf16 in the high
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int h = 4 * t + i;
+        const uint32_t pq = (nq[i] + uq - 1) / uq;
+        uint32_t pb = (nb[i] + ub - 1) / ub;
+        if (pq + pb == 0) pb = 1;                     // an empty head still writes its (zero) output
+        pc[i] = h < bh ? pq | pb << 16 : 0u;
+        sum += pc[i];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+    }
+    if (lane == 63) s_pieces[wave] = incl;
+    if (t == 0) s_out[0] = -1;
+    __syncthreads();
+    uint32_t base = incl - sum, all = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        if (w < wave) base += s_pieces[w];
+        all += s_pieces[w];
+    }
+    const int id = blockIdx.x, totq = static_cast<int>(all & 0xffffu);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int bq = static_cast<int>(base & 0xffffu), bb = static_cast<int>(base >> 16);
+        const int pq = static_cast<int>(pc[i] & 0xffffu), pb = static_cast<int>(pc[i] >> 16);
+        const int iq = id - bq, ib = id - totq - bb;
+        const bool q = iq >= 0 && iq < pq, b = ib >= 0 && ib < pb;
+        if (q || b) {                                 // one thread of the workgroup at most
+            const int n0 = static_cast<int>(nq[i]), n1 = static_cast<int>(nb[i]);
+            s_out[0] = 4 * t + i;
+            s_out[1] = q ? iq : pq + ib;
+            s_out[2] = pq + pb;
+            s_out[3] = bq + bb;
+            // units: n0 * (iq + 1) stays below 2^31 (2^19 units, 64 pieces)
+            s_out[4] = q ? n0 * iq / pq : n0 + static_cast<int>(static_cast<int64_t>(n1) * ib / pb);
+            s_out[5] = q ? n0 * (iq + 1) / pq : n0 + static_cast<int>(static_cast<int64_t>(n1) * (ib + 1) / pb);
+            s_out[6] = n0;
+            s_out[7] = n1;
+        }
+        base += pc[i];
+    }
+    __syncthreads();
+    RaggedPiece r;
+    r.head = __builtin_amdgcn_readfirstlane(s_out[0]);
+    r.piece = __builtin_amdgcn_readfirstlane(s_out[1]);
+    r.pieces = __builtin_amdgcn_readfirstlane(s_out[2]);
+    r.first = __builtin_amdgcn_readfirstlane(s_out[3]);
+    r.u0 = __builtin_amdgcn_readfirstlane(s_out[4]);
+    r.u1 = __builtin_amdgcn_readfirstlane(s_out[5]);
+    r.nqg = __builtin_amdgcn_readfirstlane(s_out[6]);
+    r.nb = __builtin_amdgcn_readfirstlane(s_out[7]);
+    return r;
+}
+
 // ---------------------------------------------------------------------------
 // the kernel
 // ---------------------------------------------------------------------------
-template <int KB, int VB>
+// RAGGED: the pieces of ragged_piece (grid: ragged_grid workgroups; bnd[0] and
+// bnd[1] hold the CU and slot counts, segments 1 and 2 are empty).
+template <int KB, int VB, bool RAGGED>
 __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
 #ifdef HYQ_PHASE_TRACE
     uint64_t ph[TRACE_PH] = {};
     HYQ_STAMP(0);
     const uint32_t launch = __hip_atomic_load(&g_trace_launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #endif
-    const int head = blockIdx.x;
-    const int wg = blockIdx.y;                       // piece of the head
+    int head = blockIdx.x;
+    int wg = blockIdx.y;                             // piece of the head
     KArgs K = kernel_args(wg);
-    const int u0 = static_cast<int>(K.bnd[0]), u1 = static_cast<int>(K.bnd[1]);   // its schedule units
+    int u0 = static_cast<int>(K.bnd[0]), u1 = static_cast<int>(K.bnd[1]);         // its schedule units
     const uint16_t* const qp = kptr<const uint16_t>(K, 0);
     const uint8_t* const kp = kptr<const uint8_t>(K, 2);
     const uint8_t* const vp = kptr<const uint8_t>(K, 4);
@@ -959,11 +1116,26 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
     const int nquant = static_cast<int>(kdw(K, 37));
     const int sn0 = static_cast<int>(kdw(K, 38)), sn1 = static_cast<int>(kdw(K, 39)), sn2 = static_cast<int>(kdw(K, 40));
     const int G = static_cast<int>(kdw(K, 41));
-    const int nqg = static_cast<int>(kdw(K, 42));
-    const int su0 = static_cast<int>(kdw(K, 43)), su1 = static_cast<int>(kdw(K, 44));
+    int nqg = static_cast<int>(kdw(K, 42));
+    int su0 = static_cast<int>(kdw(K, 43));
+    const int su1 = static_cast<int>(kdw(K, 44));
     const float qk_scale = __uint_as_float(kdw(K, 45));
     const int io = static_cast<int>(kdw(K, 46));
     HYQ_STAMP(1);
+    int pieces = 0, first = 0;                     // RAGGED: the head's pieces and first slot
+    if constexpr (RAGGED) {
+        epilogue_args(K);                          // (before anything can move the registers of those loads)
+        const RaggedPiece r = ragged_piece<KB, VB>(static_cast<int>(K.e1[3]), G, nquant, sn0, len_q, len_s0, u0, u1);
+        if (r.head < 0) return;
+        head = r.head;
+        wg = r.piece;
+        pieces = r.pieces;
+        first = r.first;
+        u0 = r.u0;
+        u1 = r.u1;
+        nqg = r.nqg;
+        su0 = r.nb;
+    }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int c = lane & 15, kb = lane >> 4;
@@ -1157,10 +1329,11 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
     // ---- wave -> LDS ----------------------------------------------------------
     HYQ_STAMP(4);
     epilogue_args(K);
-    const int mj = static_cast<int>(K.e1[2]);
-    const MergeArgs ma{G, static_cast<int>(K.e1[1]), eptr<const float>(K, 2), eptr<const float>(K, 4),
-                       eptr<uint16_t>(K, 0), static_cast<int64_t>(static_cast<int32_t>(K.e1[0])),
-                       io & HYQ_DT_OUT_FP16};
+    const int nwg = RAGGED ? pieces : static_cast<int>(K.e1[1]);
+    const int mj = RAGGED ? merge_batch(G, nwg) : static_cast<int>(K.e1[2]);
+    const MergeArgs ma{G, nwg, RAGGED ? static_cast<int64_t>(first) : static_cast<int64_t>(head) * nwg,
+                       eptr<const float>(K, 2), eptr<const float>(K, 4), eptr<uint16_t>(K, 0),
+                       static_cast<int64_t>(static_cast<int32_t>(K.e1[0])), io & HYQ_DT_OUT_FP16};
     uint32_t* const cnt = eptr<uint32_t>(K, 6);
     // The rings' last loads (past the piece's end: zeros, no memory access)
     // are drained here, with a wait the compiler sees, so that it has no
@@ -1182,7 +1355,7 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
     HYQ_STAMP(5);
 
     // ---- workgroup merge -> partial acc[G][D] and (m, l)[G] ----------------------
-    const int64_t slot = static_cast<int64_t>(head) * ma.nwg + wg;
+    const int64_t slot = ma.first + wg;
     {
         const Rsrc rpart = make_rsrc(ma.part + slot * G * D, static_cast<uint32_t>(G * D * 4));
         for (int o = threadIdx.x; o < G * (D / 4); o += THREADS) {
@@ -1702,7 +1875,7 @@ __global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
     }
 
     // ---- wave -> LDS -> this piece's partial, then decode_kernel's arrival protocol ----
-    const MergeArgs ma{G, a.nwg, a.part, a.ml, a.out, a.out_stride, 0};
+    const MergeArgs ma{G, a.nwg, static_cast<int64_t>(head) * a.nwg, a.part, a.ml, a.out, a.out_stride, 0};
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the rings' last (empty) loads
     st.l = col_sum(st.l);
     if (kb == 0) {
@@ -1780,6 +1953,7 @@ struct Slots {
 
 struct Plan {
     int nwg;               // pieces per head
+    int grid;              // workgroups of a ragged launch (0: nwg for each head)
     int nqg, segu[3];      // schedule units: prefix units, bf16 units per segment
     int bnd[MAX_NWG + 1];  // piece p covers units [bnd[p], bnd[p+1])
 };
@@ -1974,23 +2148,6 @@ size_t lds_bytes(int G) {
     return std::max(static_cast<size_t>(WAVES) * G * (D + 1), static_cast<size_t>(MERGE_LDS)) * sizeof(float);
 }
 
-// The merge instance: for G <= 4 merge_head_waves with the smallest batch
-// covering a lane's partial pairs (else batches of 24); for G > 4
-// merge_head_cols (100 + batch) with the smallest batch covering a thread's
-// items (else batches of 24).
-int merge_batch(int G, int nwg) {
-    if (G <= WAVES) {
-        const int pairs = (nwg + 1) / 2;
-        for (int mj : {4, 8, 12, 16, 20})
-            if (pairs <= mj) return mj;
-        return 24;
-    }
-    const int items = merge_items(G, nwg);
-    for (int mj : {8, 16})
-        if (items <= mj) return 100 + mj;
-    return 124;
-}
-
 // Workgroups of a decode kernel the device holds at once (and the device's
 // CU count), cached per device and GQA width (the LDS size).
 Slots slots_of(const void* kernel, std::atomic<int> (&cache)[64][17][2], int G) {
@@ -2010,7 +2167,7 @@ Slots slots_of(const void* kernel, std::atomic<int> (&cache)[64][17][2], int G) 
 template <int KB, int VB>
 Slots resident_slots_of(int G) {
     static std::atomic<int> cache[64][17][2];
-    return slots_of(reinterpret_cast<const void*>(&decode_kernel<KB, VB>), cache, G);
+    return slots_of(reinterpret_cast<const void*>(&decode_kernel<KB, VB, false>), cache, G);
 }
 
 Slots resident_slots(int kb, int vb, int G) {
@@ -2027,10 +2184,20 @@ Slots resident_slots(int kb, int vb, int G) {
     }
 }
 
-Plan plan_for(const hyq_decode_params* p) {
+// Ragged lengths are planned on the device (ragged_piece) where its limits
+// allow; else by the padded lengths, like a full batch.
+Plan plan_for(const hyq_decode_params* p, bool ragged = true) {
     const int kb = p->n_quant > 0 ? p->k_bits : 4, vb = p->n_quant > 0 ? p->v_bits : 4;
-    return make_plan(group_units(p->n_quant, kb, vb), p->seg_n, p->bh_kv, p->kv_repeat, p->split_tokens,
-                     resident_slots(kb, vb, p->kv_repeat));
+    const Slots sl = resident_slots(kb, vb, p->kv_repeat);
+    Plan pl = make_plan(group_units(p->n_quant, kb, vb), p->seg_n, p->bh_kv, p->kv_repeat, p->split_tokens, sl);
+    const bool lens = (p->n_quant > 0 && p->seq_lens_quant) || (p->seg_n[0] > 0 && p->seq_lens_seg0);
+    if (ragged && lens && p->bh_kv <= RAGGED_HEADS && p->seg_n[1] == 0 && p->seg_n[2] == 0 && p->split_tokens <= 0 &&
+        sl.slots > 0) {
+        pl.grid = ragged_grid(p->bh_kv, sl.cus, sl.slots);
+        pl.bnd[0] = sl.cus;
+        pl.bnd[1] = sl.slots;
+    }
+    return pl;
 }
 
 // workspace: [arrival counters: CNT_CAP slots, 128 B apart][(m, l) table][partials].
@@ -2040,7 +2207,7 @@ struct Layout {
     size_t cnt, ml, part, total;
 };
 Layout layout(const Plan& pl, int bh_kv, int G) {
-    const size_t slots = static_cast<size_t>(bh_kv) * std::max(pl.nwg, 1) * G;
+    const size_t slots = (pl.grid > 0 ? static_cast<size_t>(pl.grid) : static_cast<size_t>(bh_kv) * std::max(pl.nwg, 1)) * G;
     Layout L;
     L.cnt = 0;
     L.ml = static_cast<size_t>(CNT_CAP) * CNT_PAD * sizeof(uint32_t);
@@ -2288,7 +2455,7 @@ int launch_decode(const hyq_decode_params* p, const Plan& pl, const Layout& L, v
     a.qk_scale = p->sm_scale * LOG2E;
     a.nqg = pl.nqg; a.nwg = pl.nwg;
     a.mj = merge_batch(p->kv_repeat, pl.nwg);
-    for (int i = 0; i <= pl.nwg; ++i) a.bnd[i] = pl.bnd[i];
+    for (int i = 0; i <= (pl.grid > 0 ? 1 : pl.nwg); ++i) a.bnd[i] = pl.bnd[i];
     char* ws = static_cast<char*>(workspace);
     a.cnt = reinterpret_cast<uint32_t*>(ws + L.cnt);
     a.ml = reinterpret_cast<float*>(ws + L.ml);
@@ -2301,16 +2468,24 @@ int launch_decode(const hyq_decode_params* p, const Plan& pl, const Layout& L, v
     const dim3 grid(static_cast<unsigned>(p->bh_kv), static_cast<unsigned>(pl.nwg)), block(THREADS);
     const size_t lds = lds_bytes(p->kv_repeat);
     const int bits = p->n_quant > 0 ? 10 * p->k_bits + p->v_bits : 44;   // no prefix: any instance
+    auto launch = [&](auto k, auto v) {
+        constexpr int KB = decltype(k)::value, VB = decltype(v)::value;
+        if (pl.grid > 0) decode_kernel<KB, VB, true><<<dim3(static_cast<unsigned>(pl.grid)), block, lds, s>>>(a);
+        else decode_kernel<KB, VB, false><<<grid, block, lds, s>>>(a);
+    };
+    constexpr std::integral_constant<int, 2> b2;
+    constexpr std::integral_constant<int, 4> b4;
+    constexpr std::integral_constant<int, 8> b8;
     switch (bits) {
-        case 44: decode_kernel<4, 4><<<grid, block, lds, s>>>(a); break;
-        case 42: decode_kernel<4, 2><<<grid, block, lds, s>>>(a); break;
-        case 48: decode_kernel<4, 8><<<grid, block, lds, s>>>(a); break;
-        case 24: decode_kernel<2, 4><<<grid, block, lds, s>>>(a); break;
-        case 22: decode_kernel<2, 2><<<grid, block, lds, s>>>(a); break;
-        case 28: decode_kernel<2, 8><<<grid, block, lds, s>>>(a); break;
-        case 84: decode_kernel<8, 4><<<grid, block, lds, s>>>(a); break;
-        case 82: decode_kernel<8, 2><<<grid, block, lds, s>>>(a); break;
-        default: decode_kernel<8, 8><<<grid, block, lds, s>>>(a); break;
+        case 44: launch(b4, b4); break;
+        case 42: launch(b4, b2); break;
+        case 48: launch(b4, b8); break;
+        case 24: launch(b2, b4); break;
+        case 22: launch(b2, b2); break;
+        case 28: launch(b2, b8); break;
+        case 84: launch(b8, b4); break;
+        case 82: launch(b8, b2); break;
+        default: launch(b8, b8); break;
     }
     return check_launch("hyq_decode_hybrid");
 }
@@ -2326,6 +2501,17 @@ int prepare(const hyq_decode_params* p, Plan& pl, Layout& L) {
         return fail(HYQ_ENOTSUP, "too many pieces per head for the merge tables");
     L = layout(pl, p->bh_kv, p->kv_repeat);
     return HYQ_OK;
+}
+
+// A ragged call whose workspace is too small for the device's plan, but sized
+// for the padded lengths, runs by those.
+void fit_plan(const hyq_decode_params* p, size_t bytes, Plan& pl, Layout& L) {
+    if (bytes >= L.total || pl.grid == 0) return;
+    const Plan padded = plan_for(p, false);
+    const Layout PL = layout(padded, p->bh_kv, p->kv_repeat);
+    if (PL.total > bytes) return;
+    pl = padded;
+    L = PL;
 }
 
 // ---------------------------------------------------------------------------
@@ -2374,6 +2560,7 @@ extern "C" int hyq_decode_hybrid(const hyq_decode_params* p, void* workspace, si
     Layout L{};
     int rc = prepare(p, pl, L);
     if (rc != HYQ_OK || p->bh_kv == 0) return rc;
+    fit_plan(p, ws_bytes, pl, L);
     if (!workspace || ws_bytes < L.total || !aligned(workspace, 256))
         return fail(HYQ_ENOSPC, "decode workspace too small or misaligned: need " + std::to_string(L.total) + " bytes");
     return launch_decode(p, pl, L, workspace, stream);
@@ -2384,6 +2571,7 @@ extern "C" int hyq_decode_hybrid_noalloc(const hyq_decode_params* p, void* strea
     Layout L{};
     int rc = prepare(p, pl, L);
     if (rc != HYQ_OK || p->bh_kv == 0) return rc;
+    fit_plan(p, SCRATCH_BYTES, pl, L);
     if (L.total > SCRATCH_BYTES)
         return fail(HYQ_ENOSPC, "hyq_decode_hybrid_noalloc: the call needs " + std::to_string(L.total) +
                                     " bytes of workspace, above the " + std::to_string(SCRATCH_BYTES) +
