@@ -34,6 +34,7 @@ EXPORTS = (
     "hyq_last_error",
     "hyq_abi_version",
     "hyq_quant_pack",
+    "hyq_append_rows",
     "hyq_dequant",
     "hyq_legacy_dequant",
     "hyq_decode_workspace_size",
@@ -127,6 +128,9 @@ def _declare(lib):
     lib.hyq_quant_pack.restype = c_int
     lib.hyq_quant_pack.argtypes = [c_void_p, c_int32, c_int64, c_int64, c_int32, c_int64, c_int64, c_int32,
                                    c_void_p, c_int64, c_int64, c_void_p, c_int64, c_void_p]
+    lib.hyq_append_rows.restype = c_int
+    lib.hyq_append_rows.argtypes = ([c_void_p, c_int64, c_int64, c_int64] * 2 + [c_int32, c_int32, c_int64, c_int32]
+                                    + [c_void_p, c_void_p, c_int64, c_int64, c_void_p])
     lib.hyq_dequant.restype = c_int
     lib.hyq_dequant.argtypes = [c_void_p, c_int64, c_int64, c_int32, c_int64, c_int64, c_int32,
                                 c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p]

@@ -181,6 +181,26 @@ __global__ __launch_bounds__(256) void legacy_dequant_kernel(
     reinterpret_cast<uint4*>(out + ib * os_bh + in * os_n)[sub] = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
+// New K and V rows [b][h][n][8 per] into the staging buffers [b * h][cap][8
+// per] at row dst_row: one thread per 16 bytes, K rows first.  A decode step
+// appends one row per head (4 KB at batch 1), so the kernel is its launch:
+// one of 1.7 us in place of two tensor copies of 2.4 us each.
+__global__ __launch_bounds__(256) void append_rows_kernel(
+    const uint16_t* __restrict__ k, int64_t ks_b, int64_t ks_h, int64_t ks_n, const uint16_t* __restrict__ v,
+    int64_t vs_b, int64_t vs_h, int64_t vs_n, uint32_t h, uint32_t n, uint32_t per, uint32_t rows,
+    uint16_t* __restrict__ dst_k, uint16_t* __restrict__ dst_v, int64_t ds_bh, int64_t dst_row) {
+    const uint32_t e = blockIdx.x * 256u + threadIdx.x;
+    uint32_t row = e / per;
+    const uint32_t ch = 8 * (e - row * per);
+    if (row >= 2 * rows) return;
+    const bool is_v = row >= rows;
+    if (is_v) row -= rows;
+    const uint32_t bh = row / n, t = row - bh * n, bb = bh / h, hh = bh - bb * h;
+    const uint16_t* src = is_v ? v + bb * vs_b + hh * vs_h + t * vs_n : k + bb * ks_b + hh * ks_h + t * ks_n;
+    uint16_t* dst = (is_v ? dst_v : dst_k) + bh * ds_bh + (dst_row + t) * static_cast<int64_t>(8 * per);
+    *reinterpret_cast<uint4*>(dst + ch) = *reinterpret_cast<const uint4*>(src + ch);
+}
+
 int lanes_log2(int d) {
     int l = 0;
     while ((1 << l) < d / 8) ++l;
@@ -231,6 +251,26 @@ extern "C" int hyq_quant_pack(const uint16_t* x, int32_t x_is_fp16, int64_t bh, 
     }
 #undef HYQ_QUANT
     return check_launch("hyq_quant_pack");
+}
+
+extern "C" int hyq_append_rows(const uint16_t* k, int64_t ks_b, int64_t ks_h, int64_t ks_n, const uint16_t* v,
+                               int64_t vs_b, int64_t vs_h, int64_t vs_n, int32_t b, int32_t h, int64_t n, int32_t d,
+                               uint16_t* dst_k, uint16_t* dst_v, int64_t dst_stride_bh, int64_t dst_row, void* stream) {
+    if (b < 0 || h < 0 || n < 0 || dst_row < 0) return fail(HYQ_EINVAL, "hyq_append_rows: negative shape");
+    if (d <= 0 || d > 512 || d % 8) return fail(HYQ_ENOTSUP, "hyq_append_rows: head dim must be a multiple of 8 up to 512");
+    const int64_t rows = static_cast<int64_t>(b) * h * n;
+    if (rows == 0) return HYQ_OK;
+    if (!k || !v || !dst_k || !dst_v) return fail(HYQ_EINVAL, "hyq_append_rows: null pointer");
+    if (!aligned(k, 16) || !aligned(v, 16) || !aligned(dst_k, 16) || !aligned(dst_v, 16) ||
+        (ks_b | ks_h | ks_n | vs_b | vs_h | vs_n | dst_stride_bh) % 8)
+        return fail(HYQ_EINVAL, "hyq_append_rows: rows must be 16-byte aligned");
+    if ((dst_row + n) * d > dst_stride_bh) return fail(HYQ_EINVAL, "hyq_append_rows: rows past the end of the buffer");
+    const int64_t pieces = 2 * rows * (d / 8);
+    if (pieces > (int64_t{1} << 31)) return fail(HYQ_ENOTSUP, "hyq_append_rows: too many rows");
+    append_rows_kernel<<<dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
+        k, ks_b, ks_h, ks_n, v, vs_b, vs_h, vs_n, static_cast<uint32_t>(h), static_cast<uint32_t>(n),
+        static_cast<uint32_t>(d / 8), static_cast<uint32_t>(rows), dst_k, dst_v, dst_stride_bh, dst_row);
+    return check_launch("hyq_append_rows");
 }
 
 extern "C" int hyq_dequant(const int8_t* packed, int64_t bh, int64_t n, int32_t d, int64_t p_stride_bh,

@@ -22,6 +22,7 @@ from typing import Any, Callable, Optional, Tuple
 import torch
 
 from . import _lib
+from . import decode_d_stage as dd
 from .decode_d_stage import (
     GROUP_SIZE,
     _packed_dim,
@@ -186,8 +187,7 @@ class DStageLayerCache:
             self.v_window.data_ptr(), self.v_window.stride(0), self.v_window.stride(1),
             ws.data_ptr(), ws.numel(), stream)
         _lib.check(st, "freeze")
-        self._staging_buf_k = torch.zeros(BH, GROUP_SIZE, D, device=dev, dtype=dtype)
-        self._staging_buf_v = torch.zeros(BH, GROUP_SIZE, D, device=dev, dtype=dtype)
+        self._staging_buf_k, self._staging_buf_v = torch.zeros(2, BH, GROUP_SIZE, D, device=dev, dtype=dtype)
         self._staging_ptr = 0
         self._keys = None
         self._values = None
@@ -200,6 +200,16 @@ class DStageLayerCache:
         """Append decode token(s) to the staging ring, flushing every 128
         tokens (src/ops/d_stage_kv_cache.py:195-207)."""
         B, H_KV, S, D = key_states.shape
+        fx = dd._FX if dd._FX is not None else dd._load_fast_ext()
+        if fx and self._staging_ptr + S <= GROUP_SIZE and key_states.is_cuda:
+            # K and V in one launch; whatever it does not take is copied below
+            if fx.append(key_states, value_states, self._staging_buf_k, self._staging_buf_v, self._staging_ptr,
+                         _stream(key_states.device)) == 0:
+                self._staging_ptr += S
+                if self._staging_ptr >= GROUP_SIZE:
+                    self._flush_staging_buffer()
+                self._seq_len += S
+                return
         BH = B * H_KV
         k = key_states.reshape(BH, S, D)
         v = value_states.reshape(BH, S, D)
@@ -223,6 +233,19 @@ class DStageLayerCache:
     def decode_attention(self, query_states: torch.Tensor, kv_repeat: int) -> torch.Tensor:
         """q_len = 1 attention over the four segments (src/ops/d_stage_kv_cache.py:219-354).
         query_states [B, H_Q, 1, D] -> [B, H_Q, 1, D]."""
+        fx = dd._FX if dd._FX is not None else dd._load_fast_ext()
+        if fx:
+            dev = query_states.get_device()
+            if dev >= 0:
+                stream = _stream(query_states.device)
+                w = dd._ws_raw.get((dev, stream), dd._NO_WS)
+                ks, vs = self._kstore, self._vstore
+                st, out = fx.decode_cache(query_states, ks.packed, vs.packed, ks.scale, vs.scale, ks.n, self.k_topk,
+                                          self.v_topk, self._staging_buf_k, self._staging_buf_v, self._staging_ptr,
+                                          self.k_window, self.v_window, self.k_bits, self.v_bits, kv_repeat, stream,
+                                          w[0], w[1])
+                if st == 0:
+                    return out
         B, H_KV, D = self._B, self._H_KV, self._D
         H_Q = H_KV * kv_repeat
         k_staging = self._staging_buf_k[:, :self._staging_ptr]

@@ -311,7 +311,8 @@ def _load_fast_ext():
             return False
         P = _lib.DecodeParams
         if m.layout() == (ctypes.sizeof(P), P.seg_n.offset, P.dtype_flags.offset):
-            m.set_entry(ctypes.cast(_lib.lib().hyq_decode_hybrid, ctypes.c_void_p).value)
+            m.set_entry(*(ctypes.cast(f, ctypes.c_void_p).value
+                          for f in (_lib.lib().hyq_decode_hybrid, _lib.lib().hyq_append_rows)))
             mod = m
     _FX = mod
     return mod

@@ -54,6 +54,21 @@ int hyq_quant_pack(const uint16_t* x, int32_t x_is_fp16, int64_t bh, int64_t n, 
                    uint16_t* scale, int64_t s_stride_bh, void* stream);
 
 /*
+ * The staging append: new K and V rows into the decode cache's bf16 / fp16
+ * staging buffers.  Replaces the two slice copies of append_staging
+ * (src/ops/d_stage_kv_cache.py:195-207) with one launch.
+ *   k, v         16-bit [b, h, n, d] strides (*s_b, *s_h, *s_n), rows 16-byte aligned
+ *   dst_k, dst_v 16-bit [b * h, cap, d] with contiguous rows, head stride
+ *                dst_stride_bh >= cap * d for both; rows [dst_row, dst_row + n)
+ *                of every head are written (they must lie below the head stride)
+ * d a multiple of 8, at most 512; 2 * b * h * n * d / 8 <= 2^31.
+ */
+int hyq_append_rows(const uint16_t* k, int64_t ks_b, int64_t ks_h, int64_t ks_n,
+                    const uint16_t* v, int64_t vs_b, int64_t vs_h, int64_t vs_n,
+                    int32_t b, int32_t h, int64_t n, int32_t d,
+                    uint16_t* dst_k, uint16_t* dst_v, int64_t dst_stride_bh, int64_t dst_row, void* stream);
+
+/*
  * Per-token dequantisation.  Replaces dequantize_per_token
  * (src/ops/decode_d_stage.py:80-101) with _unpack_int4 (:114-123) /
  * _unpack_int2 (:136-149):
