@@ -19,11 +19,12 @@
 //   and O = sum p v16 / sum p, written as bf16.
 //
 // Launch sequence of hyq_prefill_hybrid (all on the caller's stream):
-//   kv_stats_kernel / kv_final_kernel   per-channel K sum (fp64, fixed order)
-//                                        -> km; per-channel |V| max (fp8 V scale)
-//   kv_convert_kernel                   k16, v16 (and fp8 V) per KV head
-//   lists_kernel                         per query head: sorted vertical list,
-//                                        rest list, per-block counts (nr, nv)
+//   prep_kernel                          per query head: sorted vertical list,
+//                                        rest list, per-block counts (nr, nv);
+//                                        per KV head: partial per-channel K sums
+//                                        (fp64, fixed order) and |V| maxima
+//   kv_convert_kernel                   km and the fp8 V scale from the partials;
+//                                        k16, v16 (and fp8 V) per KV head
 //   gather_kernel                        rest K -> int8 per 64-block (+ scale),
 //                                        rest V and vertical K/V rows per head
 //   prefill_main_kernel                  one workgroup per (query block, head)
@@ -52,6 +53,7 @@
 #include "hyq_common.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <string>
 #include <utility>
@@ -71,13 +73,15 @@ constexpr float PF_M_INIT = -1.0e30f;
 constexpr float FP8_MAX = 448.0f;        // src/ops/sage_unified_fp8.py:44
 constexpr float S_FP8_OFFSET = 8.807f;   // vendor/sageattention/csrc/qattn/attn_utils.cuh:30 (log2 448)
 constexpr int LIST_THREADS = 1024;
+constexpr int PREP_THREADS = 512;
 // The main kernel's buffer descriptors take 32-bit byte sizes and offsets:
 // fp16 rows of 256 bytes (rest V, vertical rows, the window) stay below 2^32
 // bytes per head up to 2^24 rows, so a head has at most 2^24 positions.
 constexpr int64_t MAX_N = 1 << 24;        // sequence length per head
 constexpr int64_t MAX_T = 1 << 24;        // vertical indices per head
 constexpr int64_t MAX_P = 1 << 24;        // prefix positions N - W per head
-constexpr int STAT_ROWS = 128;           // rows per kv_stats chunk
+constexpr int STAT_ROWS = 128;           // rows per statistics chunk (a multiple of it, see stat_rows)
+constexpr int STAT_CHUNKS = 32;          // chunks per head at most: every kv_convert workgroup sums them
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -264,150 +268,207 @@ __device__ __forceinline__ uint32_t pack_e4m3x4_raw(float a, float b, float c, f
 // K mean / V max statistics
 // ---------------------------------------------------------------------------
 
-// grid (ceil(N / 128), B*HKV); thread t: channels 2(t%64), 2(t%64)+1, rows
-// chunk*128 + t/64 + 4i.  Partial sums are float64 and reduced in a fixed
-// order, so km does not depend on scheduling.
-__global__ __launch_bounds__(256) void kv_stats_kernel(const uint16_t* __restrict__ k, int64_t k_b, int64_t k_h,
-                                                       int64_t k_n, const uint16_t* __restrict__ v, int64_t v_b,
-                                                       int64_t v_h, int64_t v_n, int HKV, int N, int nch, int f16,
-                                                       double* __restrict__ kpart, float* __restrict__ vpart) {
-    __shared__ double s_sum[4][PD];
-    __shared__ float s_max[4][PD];
-    const int bhk = blockIdx.y, b = bhk / HKV, hk = bhk % HKV;
-    const int chunk = blockIdx.x;
-    const int cp = threadIdx.x & 63, ph = threadIdx.x >> 6;
-    const uint16_t* kb = k + b * k_b + hk * k_h + 2 * cp;
-    const uint16_t* vb = v + b * v_b + hk * v_h + 2 * cp;
-    double s0 = 0.0, s1 = 0.0;
-    float m0 = 0.0f, m1 = 0.0f;
-    const int r_end = min(N, (chunk + 1) * STAT_ROWS);
-    const int r0 = chunk * STAT_ROWS + ph;
-    const int nr = r_end > r0 ? (r_end - r0 + 3) / 4 : 0;     // rows r0, r0 + 4, ...
-    auto add = [&](uint32_t kk, uint32_t vv) {
-        s0 += static_cast<double>(half_to_f32(static_cast<uint16_t>(kk), f16));
-        s1 += static_cast<double>(half_to_f32(static_cast<uint16_t>(kk >> 16), f16));
-        m0 = fmaxf(m0, fabsf(half_to_f32(static_cast<uint16_t>(vv), f16)));
-        m1 = fmaxf(m1, fabsf(half_to_f32(static_cast<uint16_t>(vv >> 16), f16)));
-    };
-    // sixteen rows' loads in flight before their adds, which stay in row order
-    int i = 0;
-    for (; i + 16 <= nr; i += 16) {
-        uint32_t kk[16], vv[16];
+// One chunk of rows of a KV head, THREADS threads: 16 lanes hold a row's
+// channels (8 each), so a load instruction of a wavefront reads four whole
+// rows.  Partial sums are float64 and added in a fixed order, so km does not
+// depend on scheduling.
+struct StatArgs {
+    const uint16_t *k, *v;
+    int64_t k_b, k_h, k_n, v_b, v_h, v_n;
+    int HKV, N, nch, rows, f16;      // rows per chunk
+    double* kpart;                   // [B * HKV][nch][128]
+    float* vpart;
+};
+template <int THREADS>
+__device__ void stats_chunk(const StatArgs& a, int bhk, int chunk) {
+    constexpr int SLOTS = THREADS / 16, WV = THREADS / 64;
+    __shared__ double s_sum[WV][PD];
+    __shared__ float s_max[WV][PD];
+    const int b = bhk / a.HKV, hk = bhk % a.HKV;
+    const int sub = threadIdx.x & 15, slot = threadIdx.x >> 4;
+    const uint16_t* kb = a.k + b * a.k_b + hk * a.k_h + 8 * sub;
+    const uint16_t* vb = a.v + b * a.v_b + hk * a.v_h + 8 * sub;
+    double sum[8];
+    float mx[8];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int64_t r = r0 + 4 * (i + j);
-            kk[j] = *reinterpret_cast<const uint32_t*>(kb + r * k_n);
-            vv[j] = *reinterpret_cast<const uint32_t*>(vb + r * v_n);
+    for (int e = 0; e < 8; ++e) {
+        sum[e] = 0.0;
+        mx[e] = 0.0f;
+    }
+    const int r_end = min(a.N, (chunk + 1) * a.rows);
+    auto add = [&](u32x4 kk, u32x4 vv) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int sh = 16 * (e & 1);
+            sum[e] += static_cast<double>(half_to_f32(static_cast<uint16_t>(kk[e >> 1] >> sh), a.f16));
+            mx[e] = fmaxf(mx[e], fabsf(half_to_f32(static_cast<uint16_t>(vv[e >> 1] >> sh), a.f16)));
+        }
+    };
+    // four rows' loads in flight per thread before their adds, in row order
+    int r = chunk * a.rows + slot;
+    for (; r + 3 * SLOTS < r_end; r += 4 * SLOTS) {
+        u32x4 kk[4], vv[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t x = r + j * SLOTS;
+            kk[j] = *reinterpret_cast<const u32x4*>(kb + x * a.k_n);
+            vv[j] = *reinterpret_cast<const u32x4*>(vb + x * a.v_n);
         }
 #pragma unroll
-        for (int j = 0; j < 16; ++j) add(kk[j], vv[j]);
+        for (int j = 0; j < 4; ++j) add(kk[j], vv[j]);
     }
-    for (; i < nr; ++i) {
-        const int64_t r = r0 + 4 * i;
-        add(*reinterpret_cast<const uint32_t*>(kb + r * k_n), *reinterpret_cast<const uint32_t*>(vb + r * v_n));
+    for (; r < r_end; r += SLOTS)
+        add(*reinterpret_cast<const u32x4*>(kb + static_cast<int64_t>(r) * a.k_n),
+            *reinterpret_cast<const u32x4*>(vb + static_cast<int64_t>(r) * a.v_n));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            sum[e] += __shfl_xor(sum[e], off, 64);
+            mx[e] = fmaxf(mx[e], __shfl_xor(mx[e], off, 64));
+        }
     }
-    s_sum[ph][2 * cp] = s0;
-    s_sum[ph][2 * cp + 1] = s1;
-    s_max[ph][2 * cp] = m0;
-    s_max[ph][2 * cp + 1] = m1;
+    if ((threadIdx.x & 63) < 16) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            s_sum[threadIdx.x >> 6][8 * sub + e] = sum[e];
+            s_max[threadIdx.x >> 6][8 * sub + e] = mx[e];
+        }
+    }
     __syncthreads();
     if (threadIdx.x < PD) {
         const int ch = threadIdx.x;
-        const double s = ((s_sum[0][ch] + s_sum[1][ch]) + s_sum[2][ch]) + s_sum[3][ch];
-        const float m = fmaxf(fmaxf(s_max[0][ch], s_max[1][ch]), fmaxf(s_max[2][ch], s_max[3][ch]));
-        kpart[(static_cast<int64_t>(bhk) * nch + chunk) * PD + ch] = s;
-        vpart[(static_cast<int64_t>(bhk) * nch + chunk) * PD + ch] = m;
+        double t = 0.0;
+        float m = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WV; ++w) {
+            t += s_sum[w][ch];
+            m = fmaxf(m, s_max[w][ch]);
+        }
+        a.kpart[(static_cast<int64_t>(bhk) * a.nch + chunk) * PD + ch] = t;
+        a.vpart[(static_cast<int64_t>(bhk) * a.nch + chunk) * PD + ch] = m;
     }
 }
 
-// grid (B*HKV), 128 threads: km = the model dtype's rounding of sum / N (one
-// rounding of the float64 quotient), fp8 V scale = max|v| / 448.
-__global__ __launch_bounds__(128) void kv_final_kernel(const double* __restrict__ kpart,
-                                                       const float* __restrict__ vpart, int nch, int N, int smooth,
-                                                       int f16, uint16_t* __restrict__ km, float* __restrict__ vscale) {
-    const int bhk = blockIdx.x, ch = threadIdx.x;
-    const double* kp = kpart + static_cast<int64_t>(bhk) * nch * PD + ch;
-    const float* vp = vpart + static_cast<int64_t>(bhk) * nch * PD + ch;
-    double s = 0.0;
-    float m = 0.0f;
-    // eight chunks' loads in flight, added in chunk order (the sum is the
-    // same sequential float64 sum)
-    int i = 0;
-    for (; i + 8 <= nch; i += 8) {
-        double a[8];
-        float x[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            a[j] = kp[(i + j) * PD];
-            x[j] = vp[(i + j) * PD];
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            s += a[j];
-            m = fmaxf(m, x[j]);
-        }
-    }
-    for (; i < nch; ++i) {
-        s += kp[i * PD];
-        m = fmaxf(m, vp[i * PD]);
-    }
-    const double mean = s / static_cast<double>(N);
-    km[bhk * PD + ch] = !smooth ? static_cast<uint16_t>(0) : f16 ? f64_to_f16_rne(mean) : f64_to_bf16_rne(mean);
-    vscale[bhk * PD + ch] = m / FP8_MAX;
-}
-
-// grid (ceil(N*16 / 256), B*HKV): thread = 8 channels of one row.
+// grid (ceil(N / rows), B*HKV), 256 threads: first every workgroup sums its
+// head's nch partials in chunk order (km = the model dtype's rounding of
+// sum / N, one rounding of the float64 quotient, 0 without smoothing; fp8 V
+// scale = max|v| / 448), which saves a launch between the statistics and the
+// conversion; then a thread converts 8 channels of four rows at a time, with
+// the next four rows' loads in flight (one row at a time left the loads' latency
+// bare: 21.4 us at 8K, 8 KV heads; N = 1531: 7.9 us).
 //   bf16 model: k16 = fp16(bf16(k - km)); fp16 model: k16 = fp16(k - km)
 //   (the difference in float32, rounded to the model dtype, then
 //   .to(float16)); v16 = fp16(v); fp8 PV: v8 = e4m3(v / vscale) and
 //   v16 = fp16(v / vscale)
 __global__ __launch_bounds__(256) void kv_convert_kernel(const uint16_t* __restrict__ k, int64_t k_b, int64_t k_h,
                                                          int64_t k_n, const uint16_t* __restrict__ v, int64_t v_b,
-                                                         int64_t v_h, int64_t v_n, int HKV, int N, int f16,
-                                                         const uint16_t* __restrict__ km,
-                                                         const float* __restrict__ vscale, uint16_t* __restrict__ k16,
+                                                         int64_t v_h, int64_t v_n, int HKV, int N, int f16, int rows,
+                                                         const double* __restrict__ kpart,
+                                                         const float* __restrict__ vpart, int nch, int smooth,
+                                                         float* __restrict__ vscale, uint16_t* __restrict__ k16,
                                                          uint16_t* __restrict__ v16, uint8_t* __restrict__ v8) {
+    __shared__ __align__(16) float s_km[PD], s_vs[PD];
     const int bhk = blockIdx.y, b = bhk / HKV, hk = bhk % HKV;
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    const int64_t row = idx >> 4;
-    const int co = static_cast<int>(idx & 15);
-    if (row >= N) return;
-    const u32x4 kk = *reinterpret_cast<const u32x4*>(k + b * k_b + hk * k_h + row * k_n + 8 * co);
-    const u32x4 vv = *reinterpret_cast<const u32x4*>(v + b * v_b + hk * v_h + row * v_n + 8 * co);
-    // the 8 channel means in one 16-byte load (km rows are 256-byte aligned)
-    const u32x4 mm = *reinterpret_cast<const u32x4*>(km + bhk * PD + 8 * co);
-    float kf[8], vf[8];
+    // this thread's next four rows, 16 apart; the first four are loaded before
+    // the partials are summed, the others while the rows before are converted
+    const int co = threadIdx.x & 15;
+    const int row_end = min(N, (static_cast<int>(blockIdx.x) + 1) * rows);
+    const uint16_t* const kr = k + b * k_b + hk * k_h + 8 * co;
+    const uint16_t* const vr = v + b * v_b + hk * v_h + 8 * co;
+    u32x4 kn[4] = {}, vn[4] = {};
+    auto load = [&](int row0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const uint32_t kw = kk[e >> 1], vw = vv[e >> 1], mw = mm[e >> 1];
-        kf[e] = half_to_f32(static_cast<uint16_t>((e & 1) ? (kw >> 16) : kw), f16);
-        vf[e] = half_to_f32(static_cast<uint16_t>((e & 1) ? (vw >> 16) : vw), f16);
-        const float d = kf[e] - half_to_f32(static_cast<uint16_t>((e & 1) ? (mw >> 16) : mw), f16);
-        kf[e] = f16 ? d : bf16_round_f32(d);     // pack_f16x2 below rounds to fp16
+        for (int j = 0; j < 4; ++j) {
+            const int64_t row = row0 + 16 * j;
+            if (row < row_end) {
+                kn[j] = *reinterpret_cast<const u32x4*>(kr + row * k_n);
+                vn[j] = *reinterpret_cast<const u32x4*>(vr + row * v_n);
+            }
+        }
+    };
+    const int first = static_cast<int>(blockIdx.x) * rows + (threadIdx.x >> 4);
+    load(first);
+    {
+        const int ch = threadIdx.x & (PD - 1);
+        if (threadIdx.x < PD) {
+            double t = 0.0;
+            if (smooth) {
+                const double* kp = kpart + static_cast<int64_t>(bhk) * nch * PD + ch;
+                for (int i0 = 0; i0 < nch; i0 += 8) {
+                    double x[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] = i0 + j < nch ? kp[(i0 + j) * PD] : 0.0;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) t += x[j];
+                }
+            }
+            const double mean = t / static_cast<double>(N);
+            s_km[ch] = !smooth ? 0.0f : half_to_f32(f16 ? f64_to_f16_rne(mean) : f64_to_bf16_rne(mean), f16);
+        } else if (v8 != nullptr) {
+            const float* vp = vpart + static_cast<int64_t>(bhk) * nch * PD + ch;
+            float m = 0.0f;
+            for (int i0 = 0; i0 < nch; i0 += 8) {
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = i0 + j < nch ? vp[(i0 + j) * PD] : 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) m = fmaxf(m, x[j]);
+            }
+            s_vs[ch] = m / FP8_MAX;
+            if (blockIdx.x == 0) vscale[bhk * PD + ch] = m / FP8_MAX;
+        }
     }
-    const int64_t o = (static_cast<int64_t>(bhk) * N + row) * PD + 8 * co;
-    const u32x4 ko = {pack_f16x2(kf[0], kf[1]), pack_f16x2(kf[2], kf[3]), pack_f16x2(kf[4], kf[5]),
-                      pack_f16x2(kf[6], kf[7])};
-    const u32x4 vo = {pack_f16x2(vf[0], vf[1]), pack_f16x2(vf[2], vf[3]), pack_f16x2(vf[4], vf[5]),
-                      pack_f16x2(vf[6], vf[7])};
-    *reinterpret_cast<u32x4*>(k16 + o) = ko;
-    if (v8 != nullptr) {
-        // fp8 PV: e4m3(v / vscale) for the rest keys and fp16(v / vscale) for
-        // the vertical and window keys, so that all tiles accumulate in one unit
-        float q[8];
-        const f32x4 vs0 = *reinterpret_cast<const f32x4*>(vscale + bhk * PD + 8 * co);
-        const f32x4 vs1 = *reinterpret_cast<const f32x4*>(vscale + bhk * PD + 8 * co + 4);
+    __syncthreads();
+    float km[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) km[e] = s_km[8 * co + e];
+    auto convert = [&](int64_t row, u32x4 kk, u32x4 vv) __attribute__((always_inline)) {
+        float kf[8], vf[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float s = e < 4 ? vs0[e] : vs1[e - 4];
-            q[e] = s > 0.0f ? vf[e] / s : 0.0f;
+            const uint32_t kw = kk[e >> 1], vw = vv[e >> 1];
+            kf[e] = half_to_f32(static_cast<uint16_t>((e & 1) ? (kw >> 16) : kw), f16);
+            vf[e] = half_to_f32(static_cast<uint16_t>((e & 1) ? (vw >> 16) : vw), f16);
+            const float d = kf[e] - km[e];
+            kf[e] = f16 ? d : bf16_round_f32(d);     // pack_f16x2 below rounds to fp16
         }
-        const u32x2 p = {pack_e4m3x4(q[0], q[1], q[2], q[3]), pack_e4m3x4(q[4], q[5], q[6], q[7])};
-        *reinterpret_cast<u32x2*>(v8 + o) = p;
-        const u32x4 qo = {pack_f16x2(q[0], q[1]), pack_f16x2(q[2], q[3]), pack_f16x2(q[4], q[5]), pack_f16x2(q[6], q[7])};
-        *reinterpret_cast<u32x4*>(v16 + o) = qo;
-    } else {
-        *reinterpret_cast<u32x4*>(v16 + o) = vo;
+        const int64_t o = (static_cast<int64_t>(bhk) * N + row) * PD + 8 * co;
+        const u32x4 ko = {pack_f16x2(kf[0], kf[1]), pack_f16x2(kf[2], kf[3]), pack_f16x2(kf[4], kf[5]),
+                          pack_f16x2(kf[6], kf[7])};
+        const u32x4 vo = {pack_f16x2(vf[0], vf[1]), pack_f16x2(vf[2], vf[3]), pack_f16x2(vf[4], vf[5]),
+                          pack_f16x2(vf[6], vf[7])};
+        *reinterpret_cast<u32x4*>(k16 + o) = ko;
+        if (v8 != nullptr) {
+            // fp8 PV: e4m3(v / vscale) for the rest keys and fp16(v / vscale) for
+            // the vertical and window keys, so that all tiles accumulate in one unit
+            float q[8];
+            const f32x4 vs0 = *reinterpret_cast<const f32x4*>(s_vs + 8 * co);
+            const f32x4 vs1 = *reinterpret_cast<const f32x4*>(s_vs + 8 * co + 4);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float s = e < 4 ? vs0[e] : vs1[e - 4];
+                q[e] = s > 0.0f ? vf[e] / s : 0.0f;
+            }
+            const u32x2 p = {pack_e4m3x4(q[0], q[1], q[2], q[3]), pack_e4m3x4(q[4], q[5], q[6], q[7])};
+            *reinterpret_cast<u32x2*>(v8 + o) = p;
+            const u32x4 qo = {pack_f16x2(q[0], q[1]), pack_f16x2(q[2], q[3]), pack_f16x2(q[4], q[5]), pack_f16x2(q[6], q[7])};
+            *reinterpret_cast<u32x4*>(v16 + o) = qo;
+        } else {
+            *reinterpret_cast<u32x4*>(v16 + o) = vo;
+        }
+    };
+    for (int row0 = first; row0 < row_end; row0 += 64) {
+        u32x4 kk[4], vv[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            kk[j] = kn[j];
+            vv[j] = vn[j];
+        }
+        load(row0 + 64);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (row0 + 16 * j < row_end) convert(row0 + 16 * j, kk[j], vv[j]);
     }
 }
 
@@ -438,21 +499,140 @@ __device__ int block_exclusive_scan(int v, int* s_w) {
     return s_w[w] + x - v;
 }
 
-// grid (B*HQ), 1024 threads.  Per row: sorted list [n2], bitmap [nw], rest
-// count before each word [nw], in dynamic LDS, or (GL) in this row's slice
-// of a global scratch when they do not fit the LDS budget.
-template <bool GL>
+// One row's lists by THREADS threads, from a bitmap of the clamped indices in
+// LDS: without duplicates (the selector's output) a position's place in its
+// list is the number of set (or clear) bits before it, so both lists are
+// written in position order, whole lines at a time, and the counts of a query
+// block are two prefix counts.  A row with duplicates keeps them in `vert`:
+// it sorts its indices (s: n2 ints) and searches the sorted list for the
+// counts.  LDS: [n2][words][words] ints (lists_row_ints).  Sorting
+// every row took 44 us for 32 rows of 1632 indices of 32640 positions (16 us
+// for 403 of 8064); these hide beside the statistics (prep_kernel).
+struct ListArgs {
+    const int64_t* vidx;
+    int64_t vi_b, vi_h, vi_t;
+    int HQ, T, n2, P, nblk, W;
+    int32_t *vert, *rest, *rcount, *nr, *nv;
+};
+template <int THREADS>
+__device__ void lists_row(const ListArgs& a, int bh, int* lds) {
+    __shared__ int s_scan[THREADS / 64 + 1];
+    __shared__ int s_dup;
+    const int P = a.P, T = a.T, n2 = a.n2, nw = (P + 31) >> 5;
+    const int b = bh / a.HQ, h = bh % a.HQ;
+    int* s_sort = lds;
+    uint32_t* s_bm = reinterpret_cast<uint32_t*>(lds + n2);
+    int* s_pre = lds + n2 + nw;
+    const int tid = threadIdx.x;
+    const int64_t* vrow = a.vidx + b * a.vi_b + h * a.vi_h;
+    for (int i = tid; i < nw; i += THREADS) s_bm[i] = 0u;
+    if (tid == 0) s_dup = 0;
+    __syncthreads();
+    for (int i = tid; i < n2; i += THREADS) {
+        int x = 0x7fffffff;
+        if (i < T) {
+            const int64_t y = vrow[i * a.vi_t];
+            x = static_cast<int>(y < 0 ? 0 : (y > P - 1 ? P - 1 : y));
+            const uint32_t bit = 1u << (x & 31);
+            if (atomicOr(&s_bm[x >> 5], bit) & bit) s_dup = 1;
+        }
+        s_sort[i] = x;
+    }
+    __syncthreads();
+    // set bits before each word
+    const int per = (nw + THREADS - 1) / THREADS;
+    const int w0 = min(nw, tid * per), w1 = min(nw, w0 + per);
+    int cnt = 0;
+    for (int wi = w0; wi < w1; ++wi) cnt += __popc(s_bm[wi]);
+    int off = block_exclusive_scan(cnt, s_scan);
+    const int total = s_scan[THREADS >> 6];
+    for (int wi = w0; wi < w1; ++wi) {
+        s_pre[wi] = off;
+        off += __popc(s_bm[wi]);
+    }
+    const bool dup = s_dup != 0;
+    if (dup) {
+        for (int kk = 2; kk <= n2; kk <<= 1) {
+            for (int j = kk >> 1; j > 0; j >>= 1) {
+                __syncthreads();
+                for (int i = tid; i < n2; i += THREADS) {
+                    const int ixj = i ^ j;
+                    if (ixj > i) {
+                        const int x = s_sort[i], c = s_sort[ixj];
+                        if ((x > c) == ((i & kk) == 0)) {
+                            s_sort[i] = c;
+                            s_sort[ixj] = x;
+                        }
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    auto set_before = [&](int p) -> int {      // set bits of [0, p), p <= P
+        if (p >= P) return total;
+        return s_pre[p >> 5] + __popc(s_bm[p >> 5] & ((1u << (p & 31)) - 1u));
+    };
+    int32_t* vout = a.vert + static_cast<int64_t>(bh) * T;
+    int32_t* rout = a.rest + static_cast<int64_t>(bh) * P;
+    for (int p = tid; p < P; p += THREADS) {
+        const int n = set_before(p);
+        if (!((s_bm[p >> 5] >> (p & 31)) & 1u)) rout[p - n] = p;
+        else if (!dup) vout[n] = p;
+    }
+    if (dup)
+        for (int i = tid; i < T; i += THREADS) vout[i] = s_sort[i];
+    if (tid == 0) a.rcount[bh] = P - total;
+    for (int blk = tid; blk < a.nblk; blk += THREADS) {
+        const int wla = window_start(blk, a.W), wl = min(wla, P), n = set_before(wl);
+        int lo = n;                             // entries below wla
+        if (dup) {
+            int hi = T;
+            lo = 0;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (s_sort[mid] < wla) lo = mid + 1; else hi = mid;
+            }
+        }
+        a.nv[static_cast<int64_t>(bh) * a.nblk + blk] = lo;
+        a.nr[static_cast<int64_t>(bh) * a.nblk + blk] = wl - n;
+    }
+}
+
+__global__ __launch_bounds__(LIST_THREADS) void lists_lds_kernel(ListArgs a) {
+    extern __shared__ int s_lists[];
+    lists_row<LIST_THREADS>(a, blockIdx.x, s_lists);
+}
+
+// Blocks [0, nlists): one query head's lists; then one statistics chunk each
+// (chunk fastest).  Neither reads what the other writes.
+// Statistics, their final sum and the lists were three launches: 9.0 + 4.9 +
+// 16.4 us at 8K (8 KV heads, 32 query heads), 10.6 us here; 25.8 + 14.3 + 43.9
+// at 32K with fp8 P.V, 31.5 us here.
+__global__ __launch_bounds__(PREP_THREADS) void prep_kernel(ListArgs l, int nlists, StatArgs st) {
+    extern __shared__ int s_lists[];
+    const int i = blockIdx.x;
+    if (i < nlists) {
+        lists_row<PREP_THREADS>(l, i, s_lists);
+    } else {
+        const int j = i - nlists;
+        stats_chunk<PREP_THREADS>(st, j / st.nch, j % st.nch);
+    }
+}
+
+// Rows whose arrays do not fit the LDS: grid (B*HQ), 1024 threads; sorted list
+// [n2], bitmap [nw], rest count before each word [nw] in this row's slice of
+// a global scratch.
 __global__ __launch_bounds__(LIST_THREADS) void lists_kernel(const int64_t* __restrict__ vidx, int64_t vi_b,
                                                              int64_t vi_h, int64_t vi_t, int HQ, int T, int n2,
                                                              int P, int nblk, int W, int32_t* __restrict__ vert,
                                                              int32_t* __restrict__ rest, int32_t* __restrict__ rcount,
                                                              int32_t* __restrict__ nr, int32_t* __restrict__ nv,
                                                              int* __restrict__ gscratch) {
-    extern __shared__ int s_lists[];
     __shared__ int s_scan[LIST_THREADS / 64 + 1];
     const int nw = (P + 31) >> 5;
     const int bh = blockIdx.x, b = bh / HQ, h = bh % HQ;
-    int* const lbase = GL ? gscratch + static_cast<int64_t>(bh) * (n2 + 2 * static_cast<int64_t>(nw)) : s_lists;
+    int* const lbase = gscratch + static_cast<int64_t>(bh) * (n2 + 2 * static_cast<int64_t>(nw));
     int* s_sort = lbase;
     uint32_t* s_bm = reinterpret_cast<uint32_t*>(lbase + n2);
     int* s_pre = lbase + n2 + nw;
@@ -1767,14 +1947,19 @@ int64_t lists_row_ints(int64_t T, int64_t P) {
 bool lists_in_lds(int64_t T, int64_t P) { return static_cast<size_t>(lists_row_ints(T, P)) * 4 <= lds_budget(); }
 
 struct PrefillLayout {
-    size_t kpart, vpart, km, vscale, k16, v16, v8, vert, rest, rcount, nr, nv, k8r, k8r_scale, vr, kv16, vv16,
+    size_t kpart, vpart, vscale, k16, v16, v8, vert, rest, rcount, nr, nv, k8r, k8r_scale, vr, kv16, vv16,
         lscratch, total;
 };
+
+// rows per statistics chunk: at most STAT_CHUNKS chunks
+int64_t stat_rows(int64_t N) {
+    return STAT_ROWS * std::max<int64_t>(1, (N + STAT_ROWS * STAT_CHUNKS - 1) / (STAT_ROWS * STAT_CHUNKS));
+}
 
 PrefillLayout prefill_layout(int B, int HQ, int HKV, int64_t N, int64_t T, int W, int pv_mode) {
     const int64_t P = std::max<int64_t>(0, N - W);
     const int64_t nblk = (N + BM - 1) / BM;
-    const int64_t nch = (N + STAT_ROWS - 1) / STAT_ROWS;
+    const int64_t nch = (N + stat_rows(N) - 1) / stat_rows(N);
     const int64_t nsb = (P + BN - 1) / BN;
     const int64_t BH = static_cast<int64_t>(B) * HQ, BHK = static_cast<int64_t>(B) * HKV;
     PrefillLayout L{};
@@ -1782,7 +1967,6 @@ PrefillLayout prefill_layout(int B, int HQ, int HKV, int64_t N, int64_t T, int W
     auto take = [&](size_t bytes) { const size_t o = off; off += align256(std::max<size_t>(bytes, 1)); return o; };
     L.kpart = take(BHK * nch * PD * 8);
     L.vpart = take(BHK * nch * PD * 4);
-    L.km = take(BHK * PD * 2);
     L.vscale = take(BHK * PD * 4);
     L.k16 = take(BHK * N * PD * 2);
     L.v16 = take(BHK * N * PD * 2);
@@ -1802,27 +1986,45 @@ PrefillLayout prefill_layout(int B, int HQ, int HKV, int64_t N, int64_t T, int W
     return L;
 }
 
-int launch_lists(const int64_t* vidx, int64_t vi_b, int64_t vi_h, int64_t vi_t, int BH, int H, int T, int P,
-                 int nblk, int W, int32_t* vert, int32_t* rest, int32_t* rcount, int32_t* nr, int32_t* nv,
-                 int* gscratch, hipStream_t stream) {
-    static bool attr_set = false;
-    const int n2 = next_pow2(std::max(T, 1));
-    if (lists_in_lds(T, P)) {
-        const size_t lds = sizeof(int) * static_cast<size_t>(lists_row_ints(T, P));
-        if (!attr_set && lds > 64 * 1024) {
-            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&lists_kernel<false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_budget())) != hipSuccess)
-                return fail(HYQ_EDEVICE, "prefill lists: cannot raise the LDS limit of lists_kernel");
-            attr_set = true;
-        }
-        hipLaunchKernelGGL(lists_kernel<false>, dim3(BH), dim3(LIST_THREADS), lds, stream, vidx, vi_b, vi_h, vi_t, H, T,
-                           n2, P, nblk, W, vert, rest, rcount, nr, nv, nullptr);
+// lists_lds_kernel and prep_kernel may take more than the default 64 KiB of
+// dynamic LDS (set once per process; a repeated call is harmless)
+int raise_lds_limit(size_t lds) {
+    static std::atomic<bool> done{false};
+    if (lds <= 64 * 1024 || done.load(std::memory_order_acquire)) return HYQ_OK;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&lists_lds_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            static_cast<int>(lds_budget())) != hipSuccess)
+        return fail(HYQ_EDEVICE, "prefill lists: cannot raise the LDS limit of lists_lds_kernel");
+    done.store(true, std::memory_order_release);
+    return HYQ_OK;
+}
+
+size_t lists_lds(const ListArgs& l) { return sizeof(int) * static_cast<size_t>(lists_row_ints(l.T, l.P)); }
+
+int launch_lists(const ListArgs& l, int BH, int* gscratch, hipStream_t stream) {
+    if (lists_in_lds(l.T, l.P)) {
+        const size_t lds = lists_lds(l);
+        if (int st = raise_lds_limit(lds)) return st;
+        hipLaunchKernelGGL(lists_lds_kernel, dim3(BH), dim3(LIST_THREADS), lds, stream, l);
     } else {
         if (!gscratch) return fail(HYQ_ENOSPC, "prefill lists: no scratch for lists larger than LDS");
-        hipLaunchKernelGGL(lists_kernel<true>, dim3(BH), dim3(LIST_THREADS), 0, stream, vidx, vi_b, vi_h, vi_t, H, T,
-                           n2, P, nblk, W, vert, rest, rcount, nr, nv, gscratch);
+        hipLaunchKernelGGL(lists_kernel, dim3(BH), dim3(LIST_THREADS), 0, stream, l.vidx, l.vi_b, l.vi_h, l.vi_t, l.HQ,
+                           l.T, l.n2, l.P, l.nblk, l.W, l.vert, l.rest, l.rcount, l.nr, l.nv, gscratch);
     }
     return check_launch("lists_kernel");
+}
+
+// The lists and the statistics.  One launch while the lists' LDS leaves the
+// statistics' workgroups two to a CU; `chunks` 0: no statistics are needed.
+constexpr size_t PREP_LDS = 48 * 1024;
+int launch_prep(const ListArgs* l, int BH, int* gscratch, const StatArgs& st, int chunks, hipStream_t stream) {
+    const bool one = l && chunks > 0 && lists_in_lds(l->T, l->P) && lists_lds(*l) <= PREP_LDS;
+    if (l && !one)
+        if (int rc = launch_lists(*l, BH, gscratch, stream)) return rc;
+    if (chunks == 0 && !one) return HYQ_OK;
+    const int nlists = one ? BH : 0;
+    hipLaunchKernelGGL(prep_kernel, dim3(static_cast<unsigned>(nlists + chunks)), dim3(PREP_THREADS),
+                       one ? lists_lds(*l) : 0, stream, one ? *l : ListArgs{}, nlists, st);
+    return check_launch("prep_kernel");
 }
 
 }  // namespace
@@ -1888,8 +2090,9 @@ extern "C" int hyq_prefill_lists(const int64_t* vidx, int64_t vi_b, int64_t vi_h
     const size_t need = hyq_prefill_lists_workspace_size(b, h, n, t, window);
     if (need > 0 && (!workspace || workspace_bytes < need || !aligned(workspace, 4)))
         return fail(HYQ_ENOSPC, "hyq_prefill_lists: workspace too small (need " + std::to_string(need) + " bytes)");
-    return launch_lists(vidx, vi_b, vi_h, vi_t, b * h, h, static_cast<int>(t), static_cast<int>(P), nblk, window, vert,
-                        rest, rcount, nr, nv, need > 0 ? static_cast<int*>(workspace) : nullptr, s);
+    const ListArgs l{vidx, vi_b, vi_h, vi_t, h, static_cast<int>(t), next_pow2(std::max(static_cast<int>(t), 1)),
+                     static_cast<int>(P), nblk, window, vert, rest, rcount, nr, nv};
+    return launch_lists(l, b * h, need > 0 ? static_cast<int*>(workspace) : nullptr, s);
 }
 
 namespace hyq {
@@ -1929,34 +2132,37 @@ int prefill_run(const hyq_prefill_params* p, void* ws, size_t ws_bytes, hipStrea
     auto at = [&](size_t off) { return static_cast<void*>(base + off); };
     const int BH = B * HQ, BHK = B * HKV;
     const int nblk = static_cast<int>((N + BM - 1) / BM);
-    const int nch = static_cast<int>((N + STAT_ROWS - 1) / STAT_ROWS);
+    const int srows = static_cast<int>(stat_rows(N)), nch = static_cast<int>((N + srows - 1) / srows);
     const int nsb = static_cast<int>((P + BN - 1) / BN);
     const int Pi = static_cast<int>(P), Ti = static_cast<int>(P > 0 ? T : 0), Ni = static_cast<int>(N);
     const uint16_t* k = static_cast<const uint16_t*>(p->k);
     const uint16_t* v = static_cast<const uint16_t*>(p->v);
 
-    hipLaunchKernelGGL(kv_stats_kernel, dim3(nch, BHK), dim3(256), 0, stream, k, p->k_stride_b, p->k_stride_h,
-                       p->k_stride_n, v, p->v_stride_b, p->v_stride_h, p->v_stride_n, HKV, Ni, nch, f16,
-                       static_cast<double*>(at(L.kpart)), static_cast<float*>(at(L.vpart)));
-    if (int st = check_launch("kv_stats_kernel")) return st;
-    hipLaunchKernelGGL(kv_final_kernel, dim3(BHK), dim3(PD), 0, stream, static_cast<const double*>(at(L.kpart)),
-                       static_cast<const float*>(at(L.vpart)), nch, Ni, p->smooth_k ? 1 : 0, f16,
-                       static_cast<uint16_t*>(at(L.km)), static_cast<float*>(at(L.vscale)));
-    if (int st = check_launch("kv_final_kernel")) return st;
-    const int cblocks = static_cast<int>((N * 16 + 255) / 256);
-    hipLaunchKernelGGL(kv_convert_kernel, dim3(cblocks, BHK), dim3(256), 0, stream, k, p->k_stride_b,
-                       p->k_stride_h, p->k_stride_n, v, p->v_stride_b, p->v_stride_h, p->v_stride_n, HKV, Ni, f16,
-                       static_cast<const uint16_t*>(at(L.km)), static_cast<const float*>(at(L.vscale)),
-                       static_cast<uint16_t*>(at(L.k16)), static_cast<uint16_t*>(at(L.v16)),
-                       p->pv_mode ? static_cast<uint8_t*>(at(L.v8)) : nullptr);
+    const ListArgs lists{p->vidx, p->vi_stride_b, p->vi_stride_h, p->vi_stride_t, HQ, Ti, next_pow2(std::max(Ti, 1)),
+                         Pi, nblk, W, static_cast<int32_t*>(at(L.vert)), static_cast<int32_t*>(at(L.rest)),
+                         static_cast<int32_t*>(at(L.rcount)), static_cast<int32_t*>(at(L.nr)),
+                         static_cast<int32_t*>(at(L.nv))};
+    const StatArgs stats{k, v, p->k_stride_b, p->k_stride_h, p->k_stride_n, p->v_stride_b, p->v_stride_h,
+                         p->v_stride_n, HKV, Ni, nch, srows, f16, static_cast<double*>(at(L.kpart)),
+                         static_cast<float*>(at(L.vpart))};
+    // the K mean and the V maximum are read only with smoothing or fp8 V
+    const int chunks = p->smooth_k || p->pv_mode ? nch * BHK : 0;
+    if (int st = launch_prep(P > 0 ? &lists : nullptr, BH, L.lscratch ? static_cast<int*>(at(L.lscratch)) : nullptr,
+                             stats, chunks, stream))
+        return st;
+    // rows per workgroup, which reads its head's partials (up to 48 KB) once.
+    // Whole calls, 64 / 128 / 256 rows: N = 1531 76.9 / 79.6 / 83.1 us, 8K 568
+    // / 568 / 574 us, 12000 1118 / 1134 / 1146 us; at 32K the partials are the
+    // larger half of what 64 rows would read.
+    const int crows = N <= 16384 ? 64 : 128;
+    hipLaunchKernelGGL(kv_convert_kernel, dim3(static_cast<unsigned>((N + crows - 1) / crows), BHK), dim3(256), 0, stream,
+                       k, p->k_stride_b, p->k_stride_h, p->k_stride_n, v, p->v_stride_b, p->v_stride_h, p->v_stride_n,
+                       HKV, Ni, f16, crows, static_cast<const double*>(at(L.kpart)),
+                       static_cast<const float*>(at(L.vpart)), nch, p->smooth_k ? 1 : 0,
+                       static_cast<float*>(at(L.vscale)), static_cast<uint16_t*>(at(L.k16)),
+                       static_cast<uint16_t*>(at(L.v16)), p->pv_mode ? static_cast<uint8_t*>(at(L.v8)) : nullptr);
     if (int st = check_launch("kv_convert_kernel")) return st;
     if (P > 0) {
-        if (int st = launch_lists(p->vidx, p->vi_stride_b, p->vi_stride_h, p->vi_stride_t, BH, HQ, Ti, Pi, nblk, W,
-                                  static_cast<int32_t*>(at(L.vert)), static_cast<int32_t*>(at(L.rest)),
-                                  static_cast<int32_t*>(at(L.rcount)), static_cast<int32_t*>(at(L.nr)),
-                                  static_cast<int32_t*>(at(L.nv)),
-                                  L.lscratch ? static_cast<int*>(at(L.lscratch)) : nullptr, stream))
-            return st;
         const int nvb = (Ti + BN - 1) / BN;
         hipLaunchKernelGGL(gather_kernel, dim3(nsb + nvb, BH), dim3(256), 0, stream,
                            static_cast<const uint16_t*>(at(L.k16)), static_cast<const uint16_t*>(at(L.v16)),
