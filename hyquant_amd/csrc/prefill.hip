@@ -27,7 +27,8 @@
 //                                        k16, v16 (and fp8 V) per KV head
 //   gather_kernel                        rest K -> int8 per 64-block (+ scale),
 //                                        rest V and vertical K/V rows per head
-//   prefill_main_kernel                  one workgroup per (query block, head)
+//   prefill_main_kernel                  one workgroup per (query block, head),
+//                                        in the order of block_order
 //
 // prefill_main_kernel: 4 wavefronts, wavefront w owns query rows 32w..32w+31
 // of the block as two 16-row sub-blocks (sb).  Q is quantised in the kernel
@@ -74,6 +75,7 @@ constexpr float FP8_MAX = 448.0f;        // src/ops/sage_unified_fp8.py:44
 constexpr float S_FP8_OFFSET = 8.807f;   // vendor/sageattention/csrc/qattn/attn_utils.cuh:30 (log2 448)
 constexpr int LIST_THREADS = 1024;
 constexpr int PREP_THREADS = 512;
+constexpr int ORDER_BLOCKS = 256;        // query blocks of an XCD taken together (block_order)
 // The main kernel's buffer descriptors take 32-bit byte sizes and offsets:
 // fp16 rows of 256 bytes (rest V, vertical rows, the window) stay below 2^32
 // bytes per head up to 2^24 rows, so a head has at most 2^24 positions.
@@ -854,6 +856,16 @@ __global__ __launch_bounds__(256) void per_block_int8_kernel(const uint16_t* __r
 // main attention kernel
 // ---------------------------------------------------------------------------
 
+// Which query block of which head each workgroup takes (block_order).
+struct Order {
+    int nblk;      // query blocks per head
+    int heads;     // whole heads per XCD
+    int shared;    // heads beyond 8 * heads, whose blocks all XCDs share
+    int group;     // whole heads whose blocks are taken together
+    int spread;    // shared blocks per XCD
+    int per_xcd;
+};
+
 struct PfArgs {
     const uint16_t* q; int64_t q_b, q_h, q_n;
     uint16_t* out; int64_t o_b, o_h, o_n;
@@ -863,11 +875,29 @@ struct PfArgs {
     const int32_t* nr; const int32_t* nv;                            // [BH][nblk]
     int B, HQ, HKV, N, nblk, W, P, T, nsb;
     float c;                                                          // fp32(sm_scale * log2e)
-    int total, per_xcd;
+    Order ord;
     const float* vscale;                                              // fp8 PV: [BHK][128] per-channel V scale
     int rest_causal;       // all keys int8 up to the diagonal (rest list = positions, causal mask, no window)
     int f16;               // q and out are fp16 (an fp16 model), else bf16
 };
+
+// The head and query block of workgroup j of XCD x (consecutive workgroups go
+// to the XCDs in turn); false: none.
+__host__ __device__ inline bool block_of(const Order& o, int x, int j, int& bh, int& blk) {
+    if (j < o.spread) {
+        const int k = 8 * j + x;
+        if (k >= o.shared * o.nblk) return false;
+        bh = 8 * o.heads + k % o.shared;
+        blk = o.nblk - 1 - k / o.shared;
+        return true;
+    }
+    j -= o.spread;
+    const int g = j / (o.group * o.nblk), k = j - g * o.group * o.nblk;
+    const int n = o.group < o.heads - g * o.group ? o.group : o.heads - g * o.group;
+    bh = x * o.heads + g * o.group + k % n;
+    blk = o.nblk - 1 - k / n;
+    return true;
+}
 
 __device__ __forceinline__ f32x4 mfma_f16(const f16x8& a, const f16x8& b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -907,12 +937,8 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t s_v1[TBUF];
     __shared__ float s_red[4];
 
-    // XCD-aware order: consecutive items (same head, heaviest block first) land on one XCD
-    const int wg = blockIdx.x;
-    const int item = (wg & 7) * a.per_xcd + (wg >> 3);
-    if (item >= a.total) return;
-    const int bh = item / a.nblk;
-    const int blk = a.nblk - 1 - (item - bh * a.nblk);
+    int bh, blk;
+    if (!block_of(a.ord, blockIdx.x & 7, blockIdx.x >> 3, bh, blk)) return;
     const int b = bh / a.HQ, h = bh - b * a.HQ;
     const int G = a.HQ / a.HKV;
     const int64_t bhk = static_cast<int64_t>(b) * a.HKV + h / G;
@@ -2097,6 +2123,28 @@ extern "C" int hyq_prefill_lists(const int64_t* vidx, int64_t vi_b, int64_t vi_h
 
 namespace hyq {
 namespace {
+// Query blocks differ in work as their rows' keys do, up to nblk : 1, and the
+// device holds 64 of an XCD at once.  An XCD keeps its heads (a KV head's
+// query heads share its cache) and takes the blocks of a group of them, about
+// ORDER_BLOCKS in all, the heaviest blocks of every head first: with head
+// after head the last head's heaviest blocks began when little else was left
+// (N = 3072, 32 heads: 162 us a call, 141 now; 6144: 377 -> 357; 4 x 1024:
+// 132 -> 113) unless nblk happened to be 64 or more.  64 / 128 / 256 / 1024
+// blocks: N = 5000 314 / 325 / 284 / 286 us, 6144 377 / 360 / 358 / 356, 32K
+// 7499 / 7452 / 7489 / 7900 (too many heads' tiles for the XCD's cache).
+// Heads beyond a multiple of eight are dealt block by block to all XCDs, and
+// first (28 heads, N = 8192: 531 -> 520 us).
+Order block_order(int bh, int nblk) {
+    Order o{};
+    o.nblk = nblk;
+    o.heads = bh / 8;
+    o.shared = bh % 8;
+    o.group = std::clamp(ORDER_BLOCKS / nblk, 1, std::max(1, o.heads));   // (1 where an XCD has no whole head)
+    o.spread = (o.shared * nblk + 7) / 8;
+    o.per_xcd = o.spread + o.heads * nblk;
+    return o;
+}
+
 // Both prefill entry points: the hybrid partition, or with rest_causal (the
 // unified kernel's window 0) every key through int8 up to the diagonal.
 int prefill_run(const hyq_prefill_params* p, void* ws, size_t ws_bytes, hipStream_t stream, bool rest_causal,
@@ -2193,17 +2241,16 @@ int prefill_run(const hyq_prefill_params* p, void* ws, size_t ws_bytes, hipStrea
     a.B = B; a.HQ = HQ; a.HKV = HKV; a.N = Ni; a.nblk = nblk; a.W = W; a.P = Pi; a.T = Ti; a.nsb = nsb;
     const double sm = p->sm_scale > 0.0 ? p->sm_scale : std::pow(static_cast<double>(PD), -0.5);
     a.c = static_cast<float>(sm * 1.44269504);
-    a.total = BH * nblk;
-    a.per_xcd = (a.total + 7) / 8;
+    a.ord = block_order(BH, nblk);
     a.vscale = static_cast<const float*>(at(L.vscale));
     a.rest_causal = rest_causal ? 1 : 0;
     a.f16 = f16;
     if (qk_fp8)
-        hipLaunchKernelGGL((prefill_main_kernel<false, true>), dim3(8 * a.per_xcd), dim3(PF_THREADS), 0, stream, a);
+        hipLaunchKernelGGL((prefill_main_kernel<false, true>), dim3(8 * a.ord.per_xcd), dim3(PF_THREADS), 0, stream, a);
     else if (p->pv_mode)
-        hipLaunchKernelGGL((prefill_main_kernel<true, false>), dim3(8 * a.per_xcd), dim3(PF_THREADS), 0, stream, a);
+        hipLaunchKernelGGL((prefill_main_kernel<true, false>), dim3(8 * a.ord.per_xcd), dim3(PF_THREADS), 0, stream, a);
     else
-        hipLaunchKernelGGL((prefill_main_kernel<false, false>), dim3(8 * a.per_xcd), dim3(PF_THREADS), 0, stream, a);
+        hipLaunchKernelGGL((prefill_main_kernel<false, false>), dim3(8 * a.ord.per_xcd), dim3(PF_THREADS), 0, stream, a);
     return check_launch("prefill_main_kernel");
 }
 }  // namespace
