@@ -270,6 +270,19 @@ __device__ __forceinline__ uint32_t pack_e4m3x4_raw(float a, float b, float c, f
 // K mean / V max statistics
 // ---------------------------------------------------------------------------
 
+// Workgroups go to the XCDs in turn, each with its own L2.  The preparation's
+// kernels give XCD x the x-th eighth of their items, ordered by KV head and
+// position, so that a row's statistics, conversion and gathers, and its
+// head's tiles (block_order), run on one XCD.  Gathers at 8K (8 KV heads, 32
+// query heads) 38.5 -> 30.0 us; whole calls at N = 512 49 -> 46 us, 8 x 1024
+// 209 -> 199, 4 x 6000 (2 KV heads) 1284 -> 1259.  Conversion alone dealt
+// this way, or the gathers' groups dealt to the XCDs in turn, gave half of it.
+// Item j of XCD x, of n (n: none).
+__device__ __forceinline__ int xcd_item(int x, int j, int n) {
+    const int per = (n + 7) >> 3;
+    return j < per ? min(n, x * per + j) : n;
+}
+
 // One chunk of rows of a KV head, THREADS threads: 16 lanes hold a row's
 // channels (8 each), so a load instruction of a wavefront reads four whole
 // rows.  Partial sums are float64 and added in a fixed order, so km does not
@@ -352,7 +365,7 @@ __device__ void stats_chunk(const StatArgs& a, int bhk, int chunk) {
     }
 }
 
-// grid (ceil(N / rows), B*HKV), 256 threads: first every workgroup sums its
+// grid xcd_grid(B * HKV * ceil(N / rows)), 256 threads: first every workgroup sums its
 // head's nch partials in chunk order (km = the model dtype's rounding of
 // sum / N, one rounding of the float64 quotient, 0 without smoothing; fp8 V
 // scale = max|v| / 448), which saves a launch between the statistics and the
@@ -369,13 +382,17 @@ __global__ __launch_bounds__(256) void kv_convert_kernel(const uint16_t* __restr
                                                          const double* __restrict__ kpart,
                                                          const float* __restrict__ vpart, int nch, int smooth,
                                                          float* __restrict__ vscale, uint16_t* __restrict__ k16,
-                                                         uint16_t* __restrict__ v16, uint8_t* __restrict__ v8) {
+                                                         uint16_t* __restrict__ v16, uint8_t* __restrict__ v8, int nitems) {
     __shared__ __align__(16) float s_km[PD], s_vs[PD];
-    const int bhk = blockIdx.y, b = bhk / HKV, hk = bhk % HKV;
+    const int per = (N + rows - 1) / rows;
+    const int item = xcd_item(blockIdx.x, blockIdx.y + blockIdx.z * gridDim.y, nitems);
+    if (item >= nitems) return;
+    const int bhk = item / per, chunk = item - bhk * per;
+    const int b = bhk / HKV, hk = bhk % HKV;
     // this thread's next four rows, 16 apart; the first four are loaded before
     // the partials are summed, the others while the rows before are converted
     const int co = threadIdx.x & 15;
-    const int row_end = min(N, (static_cast<int>(blockIdx.x) + 1) * rows);
+    const int row_end = min(N, (chunk + 1) * rows);
     const uint16_t* const kr = k + b * k_b + hk * k_h + 8 * co;
     const uint16_t* const vr = v + b * v_b + hk * v_h + 8 * co;
     u32x4 kn[4] = {}, vn[4] = {};
@@ -389,7 +406,7 @@ __global__ __launch_bounds__(256) void kv_convert_kernel(const uint16_t* __restr
             }
         }
     };
-    const int first = static_cast<int>(blockIdx.x) * rows + (threadIdx.x >> 4);
+    const int first = chunk * rows + (threadIdx.x >> 4);
     load(first);
     {
         const int ch = threadIdx.x & (PD - 1);
@@ -418,7 +435,7 @@ __global__ __launch_bounds__(256) void kv_convert_kernel(const uint16_t* __restr
                 for (int j = 0; j < 8; ++j) m = fmaxf(m, x[j]);
             }
             s_vs[ch] = m / FP8_MAX;
-            if (blockIdx.x == 0) vscale[bhk * PD + ch] = m / FP8_MAX;
+            if (chunk == 0) vscale[bhk * PD + ch] = m / FP8_MAX;
         }
     }
     __syncthreads();
@@ -607,18 +624,18 @@ __global__ __launch_bounds__(LIST_THREADS) void lists_lds_kernel(ListArgs a) {
 }
 
 // Blocks [0, nlists): one query head's lists; then one statistics chunk each
-// (chunk fastest).  Neither reads what the other writes.
+// (chunk fastest, in xcd_item's order).  Neither reads what the other writes.
 // Statistics, their final sum and the lists were three launches: 9.0 + 4.9 +
 // 16.4 us at 8K (8 KV heads, 32 query heads), 10.6 us here; 25.8 + 14.3 + 43.9
 // at 32K with fp8 P.V, 31.5 us here.
-__global__ __launch_bounds__(PREP_THREADS) void prep_kernel(ListArgs l, int nlists, StatArgs st) {
+__global__ __launch_bounds__(PREP_THREADS) void prep_kernel(ListArgs l, int nlists, StatArgs st, int chunks) {
     extern __shared__ int s_lists[];
     const int i = blockIdx.x;
     if (i < nlists) {
         lists_row<PREP_THREADS>(l, i, s_lists);
     } else {
-        const int j = i - nlists;
-        stats_chunk<PREP_THREADS>(st, j / st.nch, j % st.nch);
+        const int j = xcd_item(i & 7, (i - nlists) >> 3, chunks);
+        if (j < chunks) stats_chunk<PREP_THREADS>(st, j / st.nch, j % st.nch);
     }
 }
 
@@ -717,42 +734,49 @@ __global__ __launch_bounds__(LIST_THREADS) void lists_kernel(const int64_t* __re
     }
 }
 
-// grid (nsb + nvb, B*HQ), 256 threads.  Blocks [0, nsb): 64 entries of the
+// grid xcd_grid(B * HQ * nb), nb = nsb + nvb blocks a head, 256 threads; the query heads of a
+// KV head side by side, since their lists are mostly the same rows: the second to
+// last of them find them in the XCD's L2.  Blocks [0, nsb): 64 entries of the
 // rest list -> int8 K (per-64 block scale, sm = 1) and V rows (fp16 or fp8);
 // blocks [nsb, nsb + nvb): 64 entries of the vertical list -> fp16 K and V.
 // Thread t: row t/4 of the block, channels 32(t%4) .. +31.
 __global__ __launch_bounds__(256) void gather_kernel(
-    const uint16_t* __restrict__ k16, const uint16_t* __restrict__ v16, const uint8_t* __restrict__ v8, int HQ,
-    int G, int HKV, int N, int P, int T, int nsb, const int32_t* __restrict__ rest,
+    const uint16_t* __restrict__ k16, const uint16_t* __restrict__ v16, const uint8_t* __restrict__ v8, int G,
+    int N, int P, int T, int nsb, int nb, int nitems, const int32_t* __restrict__ rest,
     const int32_t* __restrict__ rcount, const int32_t* __restrict__ vert, int8_t* __restrict__ k8r,
     float* __restrict__ k8r_scale, uint8_t* __restrict__ vr, uint16_t* __restrict__ kv16,
     uint16_t* __restrict__ vv16, int k_fp8) {
     __shared__ float s_amax[4];
-    const int bh = blockIdx.y, b = bh / HQ, h = bh % HQ;
-    const int64_t bhk = static_cast<int64_t>(b) * HKV + h / G;
+    const int item = xcd_item(blockIdx.x, blockIdx.y + blockIdx.z * gridDim.y, nitems);
+    if (item >= nitems) return;
+    // KV head, block of the list, query head of the group (fastest)
+    const int pg = item / G, bhk = pg / nb, blk = pg - bhk * nb;
+    const int bh = bhk * G + item - pg * G;
     const int tid = threadIdx.x, r = tid >> 2, qq = tid & 3;
-    if (static_cast<int>(blockIdx.x) < nsb) {
+    if (blk < nsb) {
+        const int base = blk * BN;
+        // (the index is loaded beside the count: past it the row's memory is unused)
+        const int row = rest[static_cast<int64_t>(bh) * P + min(base + r, P - 1)];
         const int rc = rcount[bh];
-        const int base = blockIdx.x * BN;
         if (base >= rc) return;                                 // uniform per block
         const int cnt = min(BN, rc - base);
         const bool ok = r < cnt;
         u32x4 kk[4] = {};
         if (ok) {
-            const int pos = rest[static_cast<int64_t>(bh) * P + base + r];
-            const uint16_t* src = k16 + (bhk * N + pos) * PD + 32 * qq;
+            const int64_t pos = static_cast<int64_t>(bhk) * N + row;
+            const uint16_t* src = k16 + pos * PD + 32 * qq;
 #pragma unroll
             for (int i = 0; i < 4; ++i) kk[i] = reinterpret_cast<const u32x4*>(src)[i];
             const int64_t dst = (static_cast<int64_t>(bh) * P + base + r) * PD;
             // V rows are plain copies: 16-byte chunk qq + 4 i of the row, so
             // the four lanes of a row cover 64 contiguous bytes per instruction
             if (v8 != nullptr) {
-                const u32x4* vs = reinterpret_cast<const u32x4*>(v8 + (bhk * N + pos) * PD);
+                const u32x4* vs = reinterpret_cast<const u32x4*>(v8 + pos * PD);
                 u32x4* vd = reinterpret_cast<u32x4*>(vr + dst);
                 vd[qq] = vs[qq];
                 vd[qq + 4] = vs[qq + 4];
             } else {
-                const u32x4* vs = reinterpret_cast<const u32x4*>(v16 + (bhk * N + pos) * PD);
+                const u32x4* vs = reinterpret_cast<const u32x4*>(v16 + pos * PD);
                 u32x4* vd = reinterpret_cast<u32x4*>(vr + 2 * dst);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) vd[qq + 4 * i] = vs[qq + 4 * i];
@@ -773,7 +797,7 @@ __global__ __launch_bounds__(256) void gather_kernel(
         // int8: amax / 127; e4m3 (FP8-QK): amax / 448, 1 for an all-zero block
         float scale = amax / (k_fp8 ? FP8_MAX : 127.0f);
         if (k_fp8 && !(scale > 0.0f)) scale = 1.0f;
-        if (tid == 0) k8r_scale[static_cast<int64_t>(bh) * nsb + blockIdx.x] = scale;
+        if (tid == 0) k8r_scale[static_cast<int64_t>(bh) * nsb + blk] = scale;
         if (ok) {
             uint32_t wds[8];
 #pragma unroll
@@ -787,11 +811,11 @@ __global__ __launch_bounds__(256) void gather_kernel(
             dst[1] = u32x4{wds[4], wds[5], wds[6], wds[7]};
         }
     } else {
-        const int base = (blockIdx.x - nsb) * BN;
+        const int base = (blk - nsb) * BN;
         if (base + r >= T) return;
-        const int pos = vert[static_cast<int64_t>(bh) * T + base + r];
-        const u32x4* ks = reinterpret_cast<const u32x4*>(k16 + (bhk * N + pos) * PD);
-        const u32x4* vs = reinterpret_cast<const u32x4*>(v16 + (bhk * N + pos) * PD);
+        const int64_t pos = static_cast<int64_t>(bhk) * N + vert[static_cast<int64_t>(bh) * T + base + r];
+        const u32x4* ks = reinterpret_cast<const u32x4*>(k16 + pos * PD);
+        const u32x4* vs = reinterpret_cast<const u32x4*>(v16 + pos * PD);
         const int64_t dst = (static_cast<int64_t>(bh) * T + base + r) * PD;
         u32x4* kd = reinterpret_cast<u32x4*>(kv16 + dst);
         u32x4* vd = reinterpret_cast<u32x4*>(vv16 + dst);
@@ -2048,8 +2072,8 @@ int launch_prep(const ListArgs* l, int BH, int* gscratch, const StatArgs& st, in
         if (int rc = launch_lists(*l, BH, gscratch, stream)) return rc;
     if (chunks == 0 && !one) return HYQ_OK;
     const int nlists = one ? BH : 0;
-    hipLaunchKernelGGL(prep_kernel, dim3(static_cast<unsigned>(nlists + chunks)), dim3(PREP_THREADS),
-                       one ? lists_lds(*l) : 0, stream, one ? *l : ListArgs{}, nlists, st);
+    hipLaunchKernelGGL(prep_kernel, dim3(static_cast<unsigned>(nlists + (chunks + 7) / 8 * 8)), dim3(PREP_THREADS),
+                       one ? lists_lds(*l) : 0, stream, one ? *l : ListArgs{}, nlists, st, chunks);
     return check_launch("prep_kernel");
 }
 
@@ -2123,6 +2147,12 @@ extern "C" int hyq_prefill_lists(const int64_t* vidx, int64_t vi_b, int64_t vi_h
 
 namespace hyq {
 namespace {
+// one workgroup per item of xcd_item: x the XCD, y and z its item
+dim3 xcd_grid(int64_t n) {
+    const int64_t per = (n + 7) / 8, y = std::min<int64_t>(per, 32768);
+    return dim3(8, static_cast<unsigned>(y), static_cast<unsigned>((per + y - 1) / y));
+}
+
 // Query blocks differ in work as their rows' keys do, up to nblk : 1, and the
 // device holds 64 of an XCD at once.  An XCD keeps its heads (a KV head's
 // query heads share its cache) and takes the blocks of a group of them, about
@@ -2203,19 +2233,21 @@ int prefill_run(const hyq_prefill_params* p, void* ws, size_t ws_bytes, hipStrea
     // / 568 / 574 us, 12000 1118 / 1134 / 1146 us; at 32K the partials are the
     // larger half of what 64 rows would read.
     const int crows = N <= 16384 ? 64 : 128;
-    hipLaunchKernelGGL(kv_convert_kernel, dim3(static_cast<unsigned>((N + crows - 1) / crows), BHK), dim3(256), 0, stream,
+    const int citems = static_cast<int>((N + crows - 1) / crows) * BHK;
+    hipLaunchKernelGGL(kv_convert_kernel, xcd_grid(citems), dim3(256), 0, stream,
                        k, p->k_stride_b, p->k_stride_h, p->k_stride_n, v, p->v_stride_b, p->v_stride_h, p->v_stride_n,
                        HKV, Ni, f16, crows, static_cast<const double*>(at(L.kpart)),
                        static_cast<const float*>(at(L.vpart)), nch, p->smooth_k ? 1 : 0,
                        static_cast<float*>(at(L.vscale)), static_cast<uint16_t*>(at(L.k16)),
-                       static_cast<uint16_t*>(at(L.v16)), p->pv_mode ? static_cast<uint8_t*>(at(L.v8)) : nullptr);
+                       static_cast<uint16_t*>(at(L.v16)), p->pv_mode ? static_cast<uint8_t*>(at(L.v8)) : nullptr, citems);
     if (int st = check_launch("kv_convert_kernel")) return st;
     if (P > 0) {
         const int nvb = (Ti + BN - 1) / BN;
-        hipLaunchKernelGGL(gather_kernel, dim3(nsb + nvb, BH), dim3(256), 0, stream,
+        const int nb = nsb + nvb, gitems = nb * BH;
+        hipLaunchKernelGGL(gather_kernel, xcd_grid(gitems), dim3(256), 0, stream,
                            static_cast<const uint16_t*>(at(L.k16)), static_cast<const uint16_t*>(at(L.v16)),
-                           p->pv_mode ? static_cast<const uint8_t*>(at(L.v8)) : nullptr, HQ, HQ / HKV, HKV, Ni, Pi, Ti,
-                           nsb, static_cast<const int32_t*>(at(L.rest)), static_cast<const int32_t*>(at(L.rcount)),
+                           p->pv_mode ? static_cast<const uint8_t*>(at(L.v8)) : nullptr, HQ / HKV, Ni, Pi, Ti, nsb, nb, gitems,
+                           static_cast<const int32_t*>(at(L.rest)), static_cast<const int32_t*>(at(L.rcount)),
                            static_cast<const int32_t*>(at(L.vert)), static_cast<int8_t*>(at(L.k8r)),
                            static_cast<float*>(at(L.k8r_scale)), static_cast<uint8_t*>(at(L.vr)),
                            static_cast<uint16_t*>(at(L.kv16)), static_cast<uint16_t*>(at(L.vv16)), qk_fp8 ? 1 : 0);
