@@ -1118,7 +1118,8 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
         // under the tile's DMA wait).  Tile t uses buffer pair t & 1 (chosen at
         // run time: the K and V reads are inline asm, so the compiler does not
         // order them after the other buffer's in-flight DMAs); the last tile of
-        // a run prefetches the next run's first tile.
+        // a run prefetches the next run's first tile.  (With fp16 P.V the
+        // vertical and window tiles are one run.)
         const Rsrc rsc = pf_rsrc(ksc_row, static_cast<uint32_t>(nrt) * 4u);
         auto sources = [&](auto KT, Rsrc& rk, Rsrc& rv) __attribute__((always_inline)) {
             constexpr int KIND = decltype(KT)::value;
@@ -1654,31 +1655,40 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
             using KR = std::integral_constant<int, T_REST>;
             using KV = std::integral_constant<int, T_VERT>;
             using KW = std::integral_constant<int, T_WIN>;
+            // Scalar registers do not hold the buffer resources of all three
+            // kinds.  The rest run keeps its own; what it issues beyond its end
+            // (and the prologue) builds the others where they are needed, from
+            // the argument block through a pointer the compiler cannot match
+            // with earlier loads.
+            auto args = [&]() __attribute__((always_inline)) {
+                auto p = (const __attribute__((address_space(4))) PfArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+                asm volatile("" : "+s"(p));
+                return p;
+            };
+            auto src16 = [&](bool vert, bool vpart) __attribute__((always_inline)) {
+                const auto p = args();
+                const uint16_t* base;
+                if (vert) base = (vpart ? p->vv16 : p->kv16) + static_cast<int64_t>(bh) * p->T * PD;
+                else base = (vpart ? p->v16 : p->k16) + bhk * p->N * PD;
+                return pf_rsrc(base, static_cast<uint32_t>(vert ? nv_b : wend) * RS16);
+            };
             // the K (V) DMAs of tile t, whatever its kind (uniform branches)
             auto issue_k_any = [&](int t, int par) __attribute__((always_inline)) {
-                Rsrc rk, rv;
                 if (t < nrt) {
-                    sources(KR{}, rk, rv);
-                    issue_k(KR{}, rk, first_of(KR{}, t), par);
-                } else if (t < nrt + nvt) {
-                    sources(KV{}, rk, rv);
-                    issue_k(KV{}, rk, first_of(KV{}, t), par);
+                    issue_k(KR{}, pf_rsrc(args()->k8r + static_cast<int64_t>(bh) * args()->P * PD,
+                                          static_cast<uint32_t>(nr_b) * RS8), BN * t, par);
                 } else {
-                    sources(KW{}, rk, rv);
-                    issue_k(KW{}, rk, first_of(KW{}, t), par);
+                    const bool vert = t < nrt + nvt;
+                    issue_k(KV{}, src16(vert, false), vert ? first_of(KV{}, t) : first_of(KW{}, t), par);
                 }
             };
             auto issue_v_any = [&](int t, int par) __attribute__((always_inline)) {
-                Rsrc rk, rv;
                 if (t < nrt) {
-                    sources(KR{}, rk, rv);
-                    issue_v(KR{}, rv, first_of(KR{}, t), par);
-                } else if (t < nrt + nvt) {
-                    sources(KV{}, rk, rv);
-                    issue_v(KV{}, rv, first_of(KV{}, t), par);
+                    issue_v(KR{}, pf_rsrc(args()->vr + static_cast<int64_t>(bh) * args()->P * PD,
+                                          static_cast<uint32_t>(nr_b) * RS16), BN * t, par);
                 } else {
-                    sources(KW{}, rk, rv);
-                    issue_v(KW{}, rv, first_of(KW{}, t), par);
+                    const bool vert = t < nrt + nvt;
+                    issue_v(KV{}, src16(vert, true), vert ? first_of(KV{}, t) : first_of(KW{}, t), par);
                 }
             };
             const int row0 = BM * blk + 32 * w;           // this wavefront's first row
@@ -1719,23 +1729,32 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                 }
             };
             float ks_pend = 0.0f;          // k_scale of tile t + 2, loaded during step t
-            // one run: tiles [t0, t1) of kind KIND
-            auto prun = [&](auto KT, int t0, int t1) __attribute__((always_inline)) {
-                constexpr int KIND = decltype(KT)::value;
+            // one run: tiles [t0, t1), rest tiles or the fp16 tiles
+            auto prun = [&](auto RT, int t0, int t1) __attribute__((always_inline)) {
+                constexpr bool REST = decltype(RT)::value;
                 if (t0 >= t1) return;
-                const int valid = KIND == T_REST ? nr_b : KIND == T_VERT ? nv_b : wend;
-                const bool causal = KIND == T_WIN || (KIND == T_REST && a.rest_causal);
-                auto needs_mask = [&](int i0) __attribute__((always_inline)) {
-                    return i0 + BN > valid || (causal && i0 + BN - 1 > row0);
+                // tile t's first key (window) or list entry, its end, and
+                // whether its keys are bounded by their query's position too
+                auto key_of = [&](int t) __attribute__((always_inline)) {
+                    return REST ? first_of(KR{}, t) : t < nrt + nvt ? first_of(KV{}, t) : first_of(KW{}, t);
+                };
+                auto valid_of = [&](int t) __attribute__((always_inline)) {
+                    return REST ? nr_b : t < nrt + nvt ? nv_b : wend;
+                };
+                auto causal_of = [&](int t) __attribute__((always_inline)) {
+                    return REST ? a.rest_causal != 0 : t >= nrt + nvt;
+                };
+                auto needs_mask = [&](int t) __attribute__((always_inline)) {
+                    return key_of(t) + BN > valid_of(t) || (causal_of(t) && key_of(t) + BN - 1 > row0);
                 };
                 // the scores of tile t (K in buffer t & 1), -inf masked
                 auto scores = [&](auto MT, int t, float (&s)[2][4][4]) __attribute__((always_inline)) {
-                    if constexpr (KIND == T_REST) qk_rest(kbase[t & 1], s);
+                    if constexpr (REST) qk_rest(kbase[t & 1], s);
                     else qk_f16(kbase[t & 1], s);
-                    if constexpr (decltype(MT)::value) mask_keys(first_of(KT, t), valid, causal, s);
+                    if constexpr (decltype(MT)::value) mask_keys(key_of(t), valid_of(t), causal_of(t), s);
                 };
                 auto scale_of = [&](float ks) __attribute__((always_inline)) {
-                    if constexpr (KIND == T_REST) {
+                    if constexpr (REST) {
                         const float qks = q_scale * ks;
                         return qks > 0.0f ? qks : 1.0f;
                     } else {
@@ -1743,11 +1762,12 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                     }
                 };
                 // int8 rest tiles hand their scores on as raw int32 bits
-                constexpr bool RAW = KIND == T_REST && !QF8;
+                constexpr bool RAW = REST && !QF8;
                 // one piece of a next tile's P: scores (sb, kbk, 2 hf .. 2 hf +
-                // 1) converted, masked, exponentiated with the current m and
-                // packed; their maximum joins mx[sb]
-                auto piece = [&](auto MT, auto PI, const float (&sn)[2][4][4], float ssc, int i0,
+                // 1) converted, masked (this lane's keys 16 kbk + r of the
+                // tile are valid below lim[sb]), exponentiated with the
+                // current m and packed; their maximum joins mx[sb]
+                auto piece = [&](auto MT, auto PI, const float (&sn)[2][4][4], float ssc, const int (&lim)[2],
                                  u32x4 (&pn)[2][2], float (&mx)[2]) __attribute__((always_inline)) {
                     constexpr int pi = decltype(PI)::value, sb = pi >> 3, kbk = (pi >> 1) & 3, hf = pi & 1;
                     float v[2];
@@ -1757,10 +1777,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                         float x = sn[sb][kbk][r];
                         if constexpr (RAW) x = static_cast<float>(__builtin_bit_cast(int, x));
                         if constexpr (decltype(MT)::value) {
-                            const int row = BM * blk + 32 * w + 16 * sb + c16;
-                            const int key = i0 + 16 * kbk + 4 * g + r;
-                            const bool ok = (key < valid) & (!causal | (key <= row));
-                            x = ok ? x : -INFINITY;
+                            x = 16 * kbk + r < lim[sb] ? x : -INFINITY;
                         }
                         v[e] = x;
                     }
@@ -1774,7 +1791,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                 // MFMA one piece (8 VALU instructions, two of them
                 // exponentials); scheduling fences keep that interleave
                 auto pv_fused = [&](auto MT, uint32_t vb, const u32x4 (&pc)[2][2], const float (&sn)[2][4][4],
-                                    float ssc, int i0, u32x4 (&pn)[2][2], float (&lmx)[2]) __attribute__((always_inline)) {
+                                    float ssc, const int (&lim)[2], u32x4 (&pn)[2][2], float (&lmx)[2]) __attribute__((always_inline)) {
                     float mx[2];
                     u32x2 v16[2][2][2];        // [stage][j][h]
                     const uint32_t o0 = opaque_v(ov0);
@@ -1798,7 +1815,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
 #pragma unroll
                             for (int sb = 0; sb < 2; ++sb)
                                 acc[sb][cb] = mfma_f16(av, __builtin_bit_cast(f16x8, pc[sb][j]), acc[sb][cb]);
-                            piece(MT, std::integral_constant<int, 2 * cb + j>{}, sn, ssc, i0, pn, mx);
+                            piece(MT, std::integral_constant<int, 2 * cb + j>{}, sn, ssc, lim, pn, mx);
                             __builtin_amdgcn_sched_barrier(0);
                         });
                     });
@@ -1821,25 +1838,41 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                 auto body = [&](auto MT, int t, const u32x4 (&pc)[2][2], float ssc_n, u32x4 (&pn)[2][2])
                                 __attribute__((always_inline)) {
                     float sn[2][4][4];
-                    if constexpr (KIND == T_REST) qk_rest_t(std::integral_constant<bool, RAW>{}, kbase[(t + 1) & 1], sn);
+                    if constexpr (REST) qk_rest_t(std::integral_constant<bool, RAW>{}, kbase[(t + 1) & 1], sn);
                     else qk_f16(kbase[(t + 1) & 1], sn);
-                    const int i0 = first_of(KT, t + 1);
+                    int lim[2] = {0, 0};
+                    if constexpr (decltype(MT)::value) {
+                        const int i0 = key_of(t + 1) + 4 * g, end = valid_of(t + 1);
+                        const bool causal = causal_of(t + 1);
+#pragma unroll
+                        for (int sb = 0; sb < 2; ++sb)
+                            lim[sb] = (causal ? min(end, row0 + 16 * sb + c16 + 1) : end) - i0;
+                    }
                     float lmx[2];
-                    pv_fused(MT, vbase[t & 1], pc, sn, ssc_n, i0, pn, lmx);
+                    pv_fused(MT, vbase[t & 1], pc, sn, ssc_n, lim, pn, lmx);
                     if (__builtin_amdgcn_ballot_w64(lmx[0] > m_run[0] + PF_SLACK) |
                         __builtin_amdgcn_ballot_w64(lmx[1] > m_run[1] + PF_SLACK)) {
                         rescale(lmx);
                         // the scores again from K(t + 1), still in LDS (not
                         // held through the step)
                         float sr[2][4][4];
-                        if constexpr (KIND == T_REST) qk_rest_t(std::integral_constant<bool, RAW>{}, kbase[(t + 1) & 1], sr);
+                        if constexpr (REST) qk_rest_t(std::integral_constant<bool, RAW>{}, kbase[(t + 1) & 1], sr);
                         else qk_f16(kbase[(t + 1) & 1], sr);
                         float mx[2];
                         static_for<16>([&](auto PI) __attribute__((always_inline)) {
-                            piece(MT, PI, sr, ssc_n, i0, pn, mx);
+                            piece(MT, PI, sr, ssc_n, lim, pn, mx);
                         });
                     }
                 };
+                Rsrc rk, rv, rkw, rvw;
+                if constexpr (REST) {
+                    sources(KR{}, rk, rv);
+                } else {
+                    rk = src16(true, false);
+                    rv = src16(true, true);
+                    rkw = src16(false, false);
+                    rvw = src16(false, true);
+                }
                 auto step = [&](int t, const u32x4 (&pc)[2][2], u32x4 (&pn)[2][2]) __attribute__((always_inline)) {
                     // own DMAs of K(t + 1) and V(t) landed; the barrier extends
                     // that to the workgroup and frees the buffers of K(t) and
@@ -1849,11 +1882,18 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                     const float ks1 = rfl(ks_pend);
                     if (t + 2 < nrt)
                         ks_pend = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsc, 0, 4 * (t + 2), 0));
-                    if (t + 2 < ntiles) issue_k_any(t + 2, t & 1);
-                    if (t + 1 < ntiles) issue_v_any(t + 1, (t + 1) & 1);
+                    if constexpr (REST) {
+                        if (t + 2 < nrt) issue_k(KR{}, rk, BN * (t + 2), t & 1);
+                        else if (t + 2 < ntiles) issue_k_any(t + 2, t & 1);
+                        if (t + 1 < nrt) issue_v(KR{}, rv, BN * (t + 1), (t + 1) & 1);
+                        else if (t + 1 < ntiles) issue_v_any(t + 1, (t + 1) & 1);
+                    } else {
+                        if (t + 2 < ntiles) issue_k(KV{}, t + 2 < nrt + nvt ? rk : rkw, key_of(t + 2), t & 1);
+                        if (t + 1 < ntiles) issue_v(KV{}, t + 1 < nrt + nvt ? rv : rvw, key_of(t + 1), (t + 1) & 1);
+                    }
                     if (t + 1 < t1) {
                         const float ssc_n = scale_of(ks1);
-                        if (needs_mask(first_of(KT, t + 1))) body(std::true_type{}, t, pc, ssc_n, pn);
+                        if (needs_mask(t + 1)) body(std::true_type{}, t, pc, ssc_n, pn);
                         else body(std::false_type{}, t, pc, ssc_n, pn);
                     } else {
                         pv16(vbase[t & 1], pc);
@@ -1864,10 +1904,10 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                 u32x4 pX[2][2], pY[2][2];
                 {
                     float s0[2][4][4];
-                    if (needs_mask(first_of(KT, t0))) scores(std::true_type{}, t0, s0);
+                    if (needs_mask(t0)) scores(std::true_type{}, t0, s0);
                     else scores(std::false_type{}, t0, s0);
                     float ssc0 = 1.0f;
-                    if constexpr (KIND == T_REST) ssc0 = scale_of(rfl(sc_next));
+                    if constexpr (REST) ssc0 = scale_of(rfl(sc_next));
                     const float lmx[2] = {tile_max16(s0[0]) * ssc0, tile_max16(s0[1]) * ssc0};
                     rescale(lmx);
                     exp_pack(ssc0, s0, pX);
@@ -1888,7 +1928,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __syncthreads();
             }
-            prun(KR{}, 0, nrt);
+            prun(std::true_type{}, 0, nrt);
             // the fp16 tiles' Q operand, from Q again (through a pointer and
             // lane coordinates the compiler cannot match with the first
             // loads: it would otherwise hold those values, or addresses, in
@@ -1906,8 +1946,16 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_main_kernel(PfArgs a) {
                         make_qh(sb, cc, xv);
                     }
             }
-            prun(KV{}, nrt, nrt + nvt);
-            prun(KW{}, nrt + nvt, ntiles);
+            // Vertical and window tiles as one run (a bound per row tells their
+            // masks apart): a run for each cost another pipeline start and 34 KB
+            // more code, 104 KB against an instruction cache of 64 KB.  With the
+            // resources above out of the rest loop (they had been spilled to
+            // vector lanes and read back per tile): whole calls, int8 / fp8 QK,
+            // 32 heads, N = 1531 76.5 -> 73.6 / 71.3 -> 68.5 us, 8192 572 -> 562 /
+            // 509 -> 505, 16384 1865 -> 1857, 8 x 1024 195 -> 188 / 186 -> 177.
+            // Steps that are not unrolled by two (54 KB; P moved instead) cost
+            // 8% at 8192 and gained nothing at 1531.
+            prun(std::false_type{}, nrt, ntiles);
         }
     }
 
