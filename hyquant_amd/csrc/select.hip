@@ -331,7 +331,13 @@ constexpr int POL_NT = 2;                   // non-temporal: the K prefix is rea
 // of row r sequentially in channel order in float64.  GM is G rounded up to
 // 1, 2, 4, 8 or 16; the means are stored with zero rows past G, so the FMA
 // loop has no branches and only the key store skips heads g >= G.  Rows past
-// the prefix read zeros through the descriptor and are not stored.
+// the prefix read zeros through the descriptor and are not stored.  Where the
+// smallest workgroups leave CUs idle, each takes one head (GM = 1, G in the
+// grid's z): a row's chain of GM times 128 float64 multiply-adds is what the
+// pass waits for.  Rows x query / key heads, all heads of a key head together
+// -> one each: 1403 x 32 / 8 12.3 -> 9.4 us, 3968 x 32 / 8 12.5 -> 11.3, 2872 x
+// 64 / 8 19.4 -> 13.2, 2 x 2872 x 32 / 2 37.2 -> 13.2; with a workgroup per CU
+// and more they stay together (the rows are read once).
 constexpr int SC_ROWS = 64;                 // rows per block
 constexpr int SC_PITCH = 144;               // LDS bytes per half-row (128 + 16)
 constexpr int SC_BLOCKS = 4;                // blocks per wavefront
@@ -339,7 +345,7 @@ constexpr int SC_WG_ROWS = 4 * SC_BLOCKS * SC_ROWS;
 
 template <int GM, bool F16>
 __global__ __launch_bounds__(256) void score_kernel(const uint16_t* __restrict__ k, int64_t ks_b, int64_t ks_h,
-                                                    int64_t ks_n, int HK, int G, int64_t P, int64_t KP, int wg_rows,
+                                                    int64_t ks_n, int HK, int G, int GP, int64_t P, int64_t KP, int wg_rows,
                                                     const double* __restrict__ qm, uint16_t* __restrict__ keys,
                                                     uint32_t* __restrict__ unc, uint32_t* __restrict__ hist) {
     __shared__ __align__(16) uint8_t s_rows[4][SC_ROWS * SC_PITCH];
@@ -348,6 +354,8 @@ __global__ __launch_bounds__(256) void score_kernel(const uint16_t* __restrict__
     __syncthreads();
     const int bh = blockIdx.y;                     // b * HK + hk
     const int b = bh / HK, hk = bh % HK;
+    const int h0 = blockIdx.z * GM, nh = min(GM, G - h0);     // this workgroup's query heads
+    const int64_t out0 = static_cast<int64_t>(bh) * G + h0;   // and their first output row
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int64_t r0 = static_cast<int64_t>(blockIdx.x) * wg_rows;
@@ -376,7 +384,7 @@ __global__ __launch_bounds__(256) void score_kernel(const uint16_t* __restrict__
         // loads issued after it, so interleaved stages would wait for each other
         __builtin_amdgcn_sched_barrier(0);
     };
-    const double* qg = qm + static_cast<int64_t>(bh) * GM * 128;
+    const double* qg = qm + (static_cast<int64_t>(bh) * GP + h0) * 128;
     const int64_t UW = unc_words(P);
     uint4 ra[8], rb[8];
     if (nst > 0) {                                 // (nst is even: both first stages hold rows)
@@ -398,7 +406,7 @@ __global__ __launch_bounds__(256) void score_kernel(const uint16_t* __restrict__
     auto compute = [&](int s) {
         const uint8_t* row = lds + lane * SC_PITCH;
         const int half = s & 1;
-#pragma unroll 1
+#pragma unroll(GM == 1 ? 4 : 1)
         for (int c = 0; c < 8; ++c) {
             const uint4 w = *reinterpret_cast<const uint4*>(row + 16 * c);
             const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
@@ -420,15 +428,14 @@ __global__ __launch_bounds__(256) void score_kernel(const uint16_t* __restrict__
             if (p < P) {
 #pragma unroll
                 for (int g = 0; g < GM; ++g)
-                    if (g < G) {
+                    if (g < nh) {
                         const uint32_t key = orderable_key(f64_to_half_rne(acc[g], F16));
-                        keys[(static_cast<int64_t>(bh) * G + g) * KP + p] = static_cast<uint16_t>(key);
+                        keys[(out0 + g) * KP + p] = static_cast<uint16_t>(key);
                         hist_add16(s_hist[g], key);
                     }
             }
             // every key here is exact: the block's uncertain words are zero
-            if (lane < 2 * G && pb + 32 * (lane & 1) < P)
-                unc[(static_cast<int64_t>(bh) * G + (lane >> 1)) * UW + pb / 32 + (lane & 1)] = 0u;
+            if (lane < 2 * nh && pb + 32 * (lane & 1) < P) unc[(out0 + (lane >> 1)) * UW + pb / 32 + (lane & 1)] = 0u;
 #pragma unroll
             for (int g = 0; g < GM; ++g) acc[g] = 0.0;
         }
@@ -449,7 +456,7 @@ __global__ __launch_bounds__(256) void score_kernel(const uint16_t* __restrict__
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last (empty) loads retire before the wave ends
     }
     __syncthreads();
-    hist_flush16(&s_hist[0][0], G, hist, static_cast<int64_t>(bh) * G);
+    hist_flush16(&s_hist[0][0], nh, hist, out0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1821,8 +1828,14 @@ extern "C" int hyq_vertical_select(const uint16_t* q, int64_t qs_b, int64_t qs_h
     auto score_f64 = [&](auto gm) {
         const int rows = score_rows(p, static_cast<int64_t>(b) * hk, SC_WG_ROWS, 4 * SC_ROWS, device_cus());
         const dim3 grid(static_cast<unsigned>((p + rows - 1) / rows), static_cast<unsigned>(b * hk));
-        score_kernel<decltype(gm)::value, true><<<grid, dim3(256), 0, s>>>(
-            k, ks_b, ks_h, ks_n, hk, G, p, KP, rows, qm, keys, unc, hist);
+        auto launch = [&](auto g, dim3 gr) {
+            score_kernel<decltype(g)::value, true><<<gr, dim3(256), 0, s>>>(
+                k, ks_b, ks_h, ks_n, hk, G, GP, p, KP, rows, qm, keys, unc, hist);
+        };
+        if (static_cast<int64_t>(grid.x) * grid.y < device_cus())
+            launch(std::integral_constant<int, 1>{}, dim3(grid.x, grid.y, static_cast<unsigned>(G)));
+        else
+            launch(gm, grid);
     };
     auto score_mfma = [&](auto gm) {
         constexpr int GM = decltype(gm)::value, STAGES = GM <= 4 ? 8 / GM : 2;   // stages per loop pass (SGRP)
