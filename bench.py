@@ -657,7 +657,7 @@ def prefill_trace_summary(trace_csv):
     rows.sort(key=lambda r: int(r["Start_Timestamp"]))
     calls, cur = [], {}
     short = lambda n: n.replace("void ", "").replace("hyq::(anonymous namespace)::", "").split("(")[0]
-    ours = ("prefill_main_kernel", "kv_stats_kernel", "kv_final_kernel", "kv_convert_kernel", "gather_kernel",
+    ours = ("prefill_main_kernel", "prep_kernel", "kv_convert_kernel", "gather_kernel",
             "per_block_int8_kernel", "zero_counts_kernel", "lists_kernel")
     for r in rows:
         n = short(r["Kernel_Name"])
@@ -772,7 +772,7 @@ def kernel_trace_summary(trace_csv):
     for r in csv.DictReader(open(trace_csv)):
         n = r["Kernel_Name"].replace("void ", "").replace("hyq::(anonymous namespace)::", "")
         if not n.startswith(("score", "topk", "qmean", "mark", "zero_words", "compact_quant", "gather_rows",
-                             "quant_pack", "decode_kernel", "dequant", "prefill", "kv_", "lists", "per_block",
+                             "quant_pack", "decode_kernel", "dequant", "prefill", "prep", "kv_", "lists", "per_block",
                              "legacy")):
             continue
         grid = r.get("Grid_Size_X", r.get("Grid_Size", ""))
