@@ -1964,10 +1964,17 @@ struct PrefixUnits {
     int64_t units;
     int tokens;            // per unit (full ones)
     int64_t bytes;         // per unit
+    int64_t span;          // per unit, from its first row of K or V (the wider) to the next unit's
 };
 PrefixUnits group_units(int64_t n_quant, int kb, int vb) {
-    return {(n_quant + GROUP - 1) / GROUP, GROUP, static_cast<int64_t>(GROUP) * (16 * kb + 16 * vb + 4)};
+    return {(n_quant + GROUP - 1) / GROUP, GROUP, static_cast<int64_t>(GROUP) * (16 * kb + 16 * vb + 4),
+            static_cast<int64_t>(GROUP) * 16 * std::max(kb, vb)};
 }
+
+// Bytes from a piece's first row to its end, in K or in V: its descriptors and
+// the offsets into it are 32 bits wide, and the register slots are loaded up
+// to 12 blocks past the end (4 MB covers 640 rows of the widest stride, 4096).
+constexpr int64_t PIECE_SPAN = (int64_t{1} << 32) - (4 << 20);
 
 size_t round256(size_t x) { return (x + 255) / 256 * 256; }
 
@@ -2006,19 +2013,20 @@ size_t round256(size_t x) { return (x + 255) / 256 * 256; }
 // Each segment gets its bytes / target pieces (rounded, at least one); the
 // target grows until the pieces fit the merge tables.
 
-// A head's segments as pieces: starting from one each, every further piece
-// goes to the segment whose pieces are the largest.
+// A head's segments as pieces: starting from the fewest (one each, or as many
+// as PIECE_SPAN takes), every further piece goes to the segment whose pieces
+// are the largest.
 struct Pieces {
     const int64_t *su, *sc;             // units, bytes per unit
     int ks[4] = {0, 0, 0, 0};
     int64_t size[4] = {0, 0, 0, 0};     // bytes of the segment's largest piece
     int total = 0;
-    Pieces(const int64_t (&u)[4], const int64_t (&c)[4]) : su(u), sc(c) {
+    Pieces(const int64_t (&u)[4], const int64_t (&c)[4], const int (&least)[4]) : su(u), sc(c) {
         for (int s = 0; s < 4; ++s)
             if (su[s] > 0) {
-                ks[s] = 1;
-                size[s] = su[s] * sc[s];
-                ++total;
+                ks[s] = least[s];
+                size[s] = (su[s] + ks[s] - 1) / ks[s] * sc[s];
+                total += ks[s];
             }
     }
     int largest() const {
@@ -2049,9 +2057,8 @@ int merge_loads(int G, int k) {
 // the largest piece at 32 KB/us on a CU of its own or 26 KB/us shared by a
 // CU's two, plus 0.05 (G <= 4, a wavefront's merge) or 0.095 (a workgroup's)
 // per partial loaded.  Fitted to the sweep above.
-Pieces cheapest_pieces(const int64_t (&su)[4], const int64_t (&sc)[4], int bh_kv, int G, int kmax, int64_t slots,
-                       int64_t cus) {
-    Pieces p(su, sc), best = p;
+Pieces cheapest_pieces(const Pieces& fewest, int bh_kv, int G, int kmax, int64_t slots, int64_t cus) {
+    Pieces p = fewest, best = p;
     const int most = std::min<int64_t>(kmax, std::max<int64_t>(p.total, slots * 15 / 16 / bh_kv));
     double least = 1e30;
     for (;;) {
@@ -2079,14 +2086,17 @@ Plan make_plan(const PrefixUnits& pre, const int64_t seg_n[3], int bh_kv, int G,
     const int64_t su[4] = {p.nqg, p.segu[0], p.segu[1], p.segu[2]};             // units per segment
     const int64_t sc[4] = {cq, cb, cb, cb};
     int64_t head_bytes = 0;
-    int nonempty = 0;
+    int least[4], fewest = 0;          // pieces that PIECE_SPAN takes
     for (int s = 0; s < 4; ++s) {
         head_bytes += su[s] * sc[s];
-        nonempty += su[s] > 0;
+        const int64_t most = std::max<int64_t>(1, PIECE_SPAN / (s == 0 ? pre.span : cb / 2));   // units per piece
+        least[s] = static_cast<int>((su[s] + most - 1) / most);
+        fewest += least[s];
     }
     p.nwg = 0;
-    if (nonempty == 0) return p;
-    const int kmax = std::max(nonempty, std::min(MAX_NWG, MAX_PARTIALS / G));
+    if (fewest == 0) return p;
+    // (2^24 rows of stride 4096 and three segments of 2^24 rows: 39 pieces at most)
+    const int kmax = std::max(fewest, std::min(MAX_NWG, MAX_PARTIALS / G));
     int ks[4];
     int bdiv = 1;                      // the bf16 segments' pieces: target / bdiv bytes
     auto counts_for = [&](int64_t target) {
@@ -2094,7 +2104,7 @@ Plan make_plan(const PrefixUnits& pre, const int64_t seg_n[3], int bh_kv, int G,
         for (int s = 0; s < 4; ++s) {
             const int64_t tg = s == 0 ? target : std::max<int64_t>(1, target / bdiv);
             ks[s] = su[s] > 0 ? static_cast<int>(std::min<int64_t>(
-                                    su[s], std::max<int64_t>(1, (su[s] * sc[s] + tg / 2) / tg)))
+                                    su[s], std::max<int64_t>(least[s], (su[s] * sc[s] + tg / 2) / tg)))
                               : 0;
             total += ks[s];
         }
@@ -2116,11 +2126,11 @@ Plan make_plan(const PrefixUnits& pre, const int64_t seg_n[3], int bh_kv, int G,
         target = std::max<int64_t>(target, (head_bytes + 47) / 48);
         total = counts_for(target);
     } else if (bh_kv <= 64 && (twelve || bh_kv < 20 || head_bytes * bh_kv < (G <= WAVES ? 48000000 : 80000000))) {
-        Pieces best(su, sc);
+        Pieces best(su, sc, least);
         if (twelve) {
             while (best.total < std::min(kmax, 12) && best.split()) {}
         } else {
-            best = cheapest_pieces(su, sc, bh_kv, G, kmax, slots > 0 ? slots : 512, sl_.cus > 0 ? sl_.cus : 256);
+            best = cheapest_pieces(best, bh_kv, G, kmax, slots > 0 ? slots : 512, sl_.cus > 0 ? sl_.cus : 256);
         }
         for (int s = 0; s < 4; ++s) ks[s] = best.ks[s];
         total = best.total;
@@ -2307,7 +2317,7 @@ Slots legacy_slots(int kb, int vb, int blk, int G) {
 }
 
 Plan legacy_plan(const hyq_legacy_params* p) {
-    PrefixUnits pre{0, GROUP, 1};
+    PrefixUnits pre{0, GROUP, 1, 1};
     int blk = 4;
     if (p->n > 0) {
         const int group = legacy_group(p);
@@ -2316,6 +2326,7 @@ Plan legacy_plan(const hyq_legacy_params* p) {
         pre.units = full * (cpg / blk) + ((rest + GROUP - 1) / GROUP + blk - 1) / blk;
         pre.tokens = blk * GROUP;
         pre.bytes = static_cast<int64_t>(pre.tokens) * (16 * p->k_bits + 16 * p->v_bits) + 4 * D;
+        pre.span = std::min<int64_t>(pre.tokens, group) * std::max(p->kc_stride_n, p->vc_stride_n);
     }
     return make_plan(pre, p->seg_n, p->bh_kv, p->kv_repeat, 0, legacy_slots(p->k_bits, p->v_bits, blk, p->kv_repeat));
 }
