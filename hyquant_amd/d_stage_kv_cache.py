@@ -77,6 +77,15 @@ class _PrefixStore:
         self.n += m
 
 
+def _staging_buffers(BH: int, D: int, device, dtype) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Zeroed K and V staging buffers [BH, 128, D], filled in one launch.
+    Each is a tensor of its own (`.data`) on half of the allocation: autograd
+    does not let the outputs of an unbind, or views made under no_grad, be
+    written in place by a copy that it records."""
+    k, v = torch.zeros(2, BH, GROUP_SIZE, D, device=device, dtype=dtype)
+    return k.data, v.data
+
+
 class DStageLayerCache:
     """Per-layer KV cache with the prefill -> decode phase transition
     (src/ops/d_stage_kv_cache.py:36-357)."""
@@ -187,7 +196,7 @@ class DStageLayerCache:
             self.v_window.data_ptr(), self.v_window.stride(0), self.v_window.stride(1),
             ws.data_ptr(), ws.numel(), stream)
         _lib.check(st, "freeze")
-        self._staging_buf_k, self._staging_buf_v = torch.zeros(2, BH, GROUP_SIZE, D, device=dev, dtype=dtype)
+        self._staging_buf_k, self._staging_buf_v = _staging_buffers(BH, D, dev, dtype)
         self._staging_ptr = 0
         self._keys = None
         self._values = None
