@@ -116,6 +116,7 @@ class PrefillParams(Structure):
     ]
 
 
+_REBUILD = "rebuild it with `python -m hyquant_amd.build`"
 _lib = None
 _lock = threading.Lock()
 
@@ -199,11 +200,14 @@ def lib():
                         f"{LIB_PATH} is missing: build it with `python -m hyquant_amd.build` "
                         "(there is no fallback implementation)")
                 l = ctypes.CDLL(LIB_PATH)
+                version = l.hyq_abi_version()
+                if version != ABI_VERSION:
+                    raise RuntimeError(f"{LIB_PATH} reports ABI {version}, these bindings need {ABI_VERSION}: {_REBUILD}")
+                # an entry point added since does not change the version
+                missing = [name for name in EXPORTS if not hasattr(l, name)]
+                if missing:
+                    raise RuntimeError(f"{LIB_PATH} lacks {', '.join(missing)}: {_REBUILD}")
                 _declare(l)
-                if l.hyq_abi_version() != ABI_VERSION:
-                    raise RuntimeError(
-                        f"{LIB_PATH} reports ABI {l.hyq_abi_version()}, these bindings need {ABI_VERSION}: "
-                        "rebuild it with `python -m hyquant_amd.build`")
                 _lib = l
     return _lib
 

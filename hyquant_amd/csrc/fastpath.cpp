@@ -187,6 +187,7 @@ std::tuple<int64_t, int64_t, int64_t> layout() {
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    m.def("entries", [] { return 2; }, "the number of addresses that set_entry takes");
     m.def("layout", &layout, "sizeof(hyq_decode_params), offsetof(seg_n), offsetof(dtype_flags)");
     m.def("set_entry", &set_entry, "the addresses of hyq_decode_hybrid and hyq_append_rows");
     m.def("decode", &decode, "fused_d_stage_decode eager fast path");
