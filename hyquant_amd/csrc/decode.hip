@@ -939,20 +939,34 @@ __host__ __device__ inline int merge_batch(int G, int nwg) {
 // ---------------------------------------------------------------------------
 // ragged lengths: the pieces planned on the device
 // ---------------------------------------------------------------------------
-// With per-head lengths only the device knows how much there is to read: cut
-// by the longest head, 16 sequences of 700 to 32000 tokens (28% of the padded
-// tokens) left three quarters of the pieces empty and the rest as large as a
-// full batch's.  So every workgroup of a ragged launch reads all lengths (at
-// most RAGGED_HEADS heads, four per thread), forms the same totals and piece
-// sizes, numbers the pieces (int4 pieces of all heads, then bf16 pieces) by a
-// prefix sum and takes the piece of its own number; workgroups past the last
-// piece leave.  Piece size, with `cus` and `slots` as in make_plan: 4/5 of a
-// piece per CU below 48 MB, 5/4 per resident slot above (of at least 96 KiB),
-// at least 16 KiB, and large enough for the merge tables and, with G > 4, for
-// the merge to load a head's partials in one or two batches.  The grid covers
-// any lengths (ragged_grid).  That batch, 32 query heads on 8 key heads, K4V4:
-// 62.8 us by the padded plan, 41.0 us by this one.
-constexpr int RAGGED_HEADS = 4 * THREADS;
+// With per-head lengths only the device knows how much there is to read.  The
+// padded plan, cut by the longest head, leaves short heads' pieces empty and
+// the long ones' as large as a full batch's.  So every workgroup of a large
+// ragged launch reads all lengths.  Where they fill RAGGED_FILL of the padded
+// bytes or more, it takes its piece of the padded plan; else it forms piece
+// sizes from the bytes that are there, numbers the pieces (int4 pieces of all
+// heads, then bf16 pieces) by a prefix sum and takes the piece of its own
+// number; workgroups past the last piece leave.  Piece size, with `cus` and
+// `slots` as in make_plan: 4/5 of a piece per CU below 48 MB, 5/4 per resident
+// slot above (of at least 96 KiB), at least 16 KiB, and large enough for the
+// merge tables and, with G > 4, for the merge to load a head's partials in one
+// or two batches.  The grid covers any lengths (ragged_grid).
+//
+// Both plans over 400 calls (32/8 heads K4V4 and K8V8, 64/8 K4V2, 32/2 K4V4;
+// batches 2-32, longest 1K-32K tokens, shortest 600 tokens to the longest):
+//   - reading the lengths costs a launch 0.1-1.5 us: up to 2% of the calls from
+//     240 MB of padded bytes on that then keep the padded plan (41 us and
+//     more), 5-10% of a 7 us call;
+//   - from 240 MB on and filled to less than 60% the device's pieces are the
+//     faster ones (16 sequences of 600 to 32000 tokens 63.3 -> 37.8 us, 32/2
+//     heads 33.2 -> 21.5, 8 sequences 36.2 -> 25.8; 8000 to 32000, filled to
+//     55%, 72.2 -> 64.1); at 73% they take -14 to +12%, full -7 to +12%;
+//   - below 240 MB the coarser pieces and that cost outweigh the balance (2 x 1000-2000 tokens 7.3 -> 8.8 us, 16 x
+//     2000 14.8 -> 19.4), except for some very ragged calls (4 x 600-32000,
+//     157 MB, 25.6 -> 22.5).
+constexpr int RAGGED_HEADS = 256;        // four per lane
+constexpr float RAGGED_FILL = 0.6f;
+constexpr int64_t RAGGED_BYTES = 240000000;
 
 // pieces a ragged launch can have: total / target, and one rounded up per
 // head and segment
@@ -965,123 +979,132 @@ struct RaggedPiece {
     int head, piece, pieces;   // head -1: no piece of this number
     int first;                 // slot of the head's first partial
     int u0, u1, nqg, nb;       // schedule units: the piece's, and the head's int4 and bf16 units
+    int nq, ns;                // the head's valid prefix and bf16 tokens
 };
 
+// inclusive prefix sum over the wavefront (rows of 16, then across rows)
+__device__ __forceinline__ uint32_t wave_scan64(uint32_t v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
+// Every wavefront for itself: no barrier, no LDS.  Lane l holds heads 4l ..
+// 4l + 3; all its loads are issued before any is waited for (heads past bh
+// read zero).  `p` comes in as the padded plan's piece.
 template <int KB, int VB>
-__device__ __forceinline__ RaggedPiece ragged_piece(int bh, int G, int nquant, int sn0, const int32_t* len_q,
-                                                    const int32_t* len_s0, int cus, int slots) {
+__device__ __forceinline__ void ragged_piece(RaggedPiece& p, int bh, int G, int nquant, int sn0, const int32_t* len_q,
+                                             const int32_t* len_s0, int cus, int slots) {
     constexpr int CQ = GROUP * (16 * KB + 16 * VB + 4), CB = BUNIT * 4 * D;   // bytes per unit
-    __shared__ uint32_t s_sum[WAVES][2];
-    __shared__ float s_max[WAVES];
-    __shared__ uint32_t s_pieces[WAVES];
-    __shared__ int s_out[8];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    uint32_t nq[4], nb[4], sq = 0, sb = 0;
-    float mx = 0.f;
+    const int lane = threadIdx.x & 63;
+    int lq[4], ls[4];
+    {
+        const uint32_t bytes = static_cast<uint32_t>(bh) * 4;
+        const Rsrc rq = make_rsrc(len_q, len_q ? bytes : 0u), rs = make_rsrc(len_s0, len_s0 ? bytes : 0u);
+        uint32_t a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            a[i] = bld32(rq, 16 * lane + 4 * i);
+            b[i] = bld32(rs, 16 * lane + 4 * i);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool in = 4 * lane + i < bh;
+            lq[i] = len_q ? min(nquant, max(0, static_cast<int>(a[i]))) : in ? nquant : 0;
+            ls[i] = len_s0 ? min(sn0, max(0, static_cast<int>(b[i]))) : in ? sn0 : 0;
+        }
+    }
+    uint32_t nq[4], nb[4];
+    float sum = 0.f, mx = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int h = 4 * t + i;
-        int lq = 0, lb = 0;
-        if (h < bh) {
-            lq = len_q ? min(nquant, max(0, len_q[h])) : nquant;
-            lb = len_s0 ? min(sn0, max(0, len_s0[h])) : sn0;
-        }
-        nq[i] = static_cast<uint32_t>(lq + GROUP - 1) / GROUP;
-        nb[i] = static_cast<uint32_t>(lb + BUNIT - 1) / BUNIT;
-        sq += nq[i];
-        sb += nb[i];
-        mx = fmaxf(mx, static_cast<float>(nq[i]) * CQ + static_cast<float>(nb[i]) * CB);
+        nq[i] = static_cast<uint32_t>(lq[i] + GROUP - 1) / GROUP;
+        nb[i] = static_cast<uint32_t>(ls[i] + BUNIT - 1) / BUNIT;
+        const float bytes = static_cast<float>(nq[i]) * CQ + static_cast<float>(nb[i]) * CB;
+        sum += bytes;
+        mx = fmaxf(mx, bytes);
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        sq += __shfl_xor(sq, off, 64);
-        sb += __shfl_xor(sb, off, 64);
-        mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    const float total = wave_sum64(sum);
+    // the valid tokens of head h
+    auto tokens = [&](int h) {
+        const int i = h & 3, l = h >> 2;
+        p.nq = __builtin_amdgcn_readlane(i == 0 ? lq[0] : i == 1 ? lq[1] : i == 2 ? lq[2] : lq[3], l);
+        p.ns = __builtin_amdgcn_readlane(i == 0 ? ls[0] : i == 1 ? ls[1] : i == 2 ? ls[2] : ls[3], l);
+    };
+    const float padded = (static_cast<float>(p.nqg) * CQ + static_cast<float>(p.nb) * CB) * static_cast<float>(bh);
+    if (__builtin_amdgcn_readfirstlane(total >= RAGGED_FILL * padded)) {
+        if (p.piece >= p.pieces) p.head = -1;
+        else tokens(p.head);
+        return;
     }
-    if (lane == 0) {
-        s_sum[wave][0] = sq;
-        s_sum[wave][1] = sb;
-        s_max[wave] = mx;
-    }
-    __syncthreads();
-    sq = sb = 0;
-    mx = 0.f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-        sq += s_sum[w][0];
-        sb += s_sum[w][1];
-        mx = fmaxf(mx, s_max[w]);
-    }
-    const float total = static_cast<float>(sq) * CQ + static_cast<float>(sb) * CB;
+    mx = wave_max64(mx);
     float target = total < 48e6f ? total / static_cast<float>(cus * 4 / 5)
                                  : fmaxf(98304.f, total / static_cast<float>(slots * 5 / 4));
-    const int most = G > 8 ? 24 : G > WAVES ? 24 : MAX_PARTIALS / 16;       // pieces per head (below the tables' limits)
+    const int most = G > WAVES ? 24 : MAX_PARTIALS / 16;   // pieces per head (below the tables' limits)
     target = fmaxf(fmaxf(target, 16384.f), mx / static_cast<float>(most - 3));
     const uint32_t uq = static_cast<uint32_t>(target / CQ) + 1, ub = static_cast<uint32_t>(target / CB) + 1;
-    uint32_t pc[4], sum = 0;                          // pieces: int4 in the low half, bf16 in the high
+    uint32_t pc[4], mine = 0;                         // pieces: int4 in the low half, bf16 in the high
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int h = 4 * t + i;
         const uint32_t pq = (nq[i] + uq - 1) / uq;
         uint32_t pb = (nb[i] + ub - 1) / ub;
         if (pq + pb == 0) pb = 1;                     // an empty head still writes its (zero) output
-        pc[i] = h < bh ? pq | pb << 16 : 0u;
-        sum += pc[i];
+        pc[i] = 4 * lane + i < bh ? pq | pb << 16 : 0u;
+        mine += pc[i];
     }
-    uint32_t incl = sum;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t o = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += o;
-    }
-    if (lane == 63) s_pieces[wave] = incl;
-    if (t == 0) s_out[0] = -1;
-    __syncthreads();
-    uint32_t base = incl - sum, all = 0;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-        if (w < wave) base += s_pieces[w];
-        all += s_pieces[w];
-    }
-    const int id = blockIdx.x, totq = static_cast<int>(all & 0xffffu);
+    const uint32_t incl = wave_scan64(mine);
+    const int totq = static_cast<int>(__builtin_amdgcn_readlane(incl, 63) & 0xffffu);
+    const int id = blockIdx.y * bh + blockIdx.x;
+    uint32_t base = incl - mine;
+    int o[8] = {};
+    bool found = false;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int bq = static_cast<int>(base & 0xffffu), bb = static_cast<int>(base >> 16);
         const int pq = static_cast<int>(pc[i] & 0xffffu), pb = static_cast<int>(pc[i] >> 16);
         const int iq = id - bq, ib = id - totq - bb;
         const bool q = iq >= 0 && iq < pq, b = ib >= 0 && ib < pb;
-        if (q || b) {                                 // one thread of the workgroup at most
+        if (q || b) {                                 // one lane at most
             const int n0 = static_cast<int>(nq[i]), n1 = static_cast<int>(nb[i]);
-            s_out[0] = 4 * t + i;
-            s_out[1] = q ? iq : pq + ib;
-            s_out[2] = pq + pb;
-            s_out[3] = bq + bb;
-            // units: n0 * (iq + 1) stays below 2^31 (2^19 units, 64 pieces)
-            s_out[4] = q ? n0 * iq / pq : n0 + static_cast<int>(static_cast<int64_t>(n1) * ib / pb);
-            s_out[5] = q ? n0 * (iq + 1) / pq : n0 + static_cast<int>(static_cast<int64_t>(n1) * (ib + 1) / pb);
-            s_out[6] = n0;
-            s_out[7] = n1;
+            found = true;
+            o[0] = 4 * lane + i;
+            o[1] = q ? iq : pq + ib;
+            o[2] = pq + pb;
+            o[3] = bq + bb;
+            // (units times pieces stay below 2^27: 2^21 units, 64 pieces)
+            o[4] = q ? n0 * iq / pq : n0 + n1 * ib / pb;
+            o[5] = q ? n0 * (iq + 1) / pq : n0 + n1 * (ib + 1) / pb;
+            o[6] = n0;
+            o[7] = n1;
         }
         base += pc[i];
     }
-    __syncthreads();
-    RaggedPiece r;
-    r.head = __builtin_amdgcn_readfirstlane(s_out[0]);
-    r.piece = __builtin_amdgcn_readfirstlane(s_out[1]);
-    r.pieces = __builtin_amdgcn_readfirstlane(s_out[2]);
-    r.first = __builtin_amdgcn_readfirstlane(s_out[3]);
-    r.u0 = __builtin_amdgcn_readfirstlane(s_out[4]);
-    r.u1 = __builtin_amdgcn_readfirstlane(s_out[5]);
-    r.nqg = __builtin_amdgcn_readfirstlane(s_out[6]);
-    r.nb = __builtin_amdgcn_readfirstlane(s_out[7]);
-    return r;
+    const uint64_t who = __builtin_amdgcn_ballot_w64(found);
+    if (who == 0) {
+        p.head = -1;
+        return;
+    }
+    const int l = __builtin_ctzll(who);
+    p.head = __builtin_amdgcn_readlane(o[0], l);
+    p.piece = __builtin_amdgcn_readlane(o[1], l);
+    p.pieces = __builtin_amdgcn_readlane(o[2], l);
+    p.first = __builtin_amdgcn_readlane(o[3], l);
+    p.u0 = __builtin_amdgcn_readlane(o[4], l);
+    p.u1 = __builtin_amdgcn_readlane(o[5], l);
+    p.nqg = __builtin_amdgcn_readlane(o[6], l);
+    p.nb = __builtin_amdgcn_readlane(o[7], l);
+    tokens(p.head);
 }
 
 // ---------------------------------------------------------------------------
 // the kernel
 // ---------------------------------------------------------------------------
-// RAGGED: the pieces of ragged_piece (grid: ragged_grid workgroups; bnd[0] and
-// bnd[1] hold the CU and slot counts, segments 1 and 2 are empty).
+// RAGGED: the pieces of ragged_piece.  Segments 1 and 2 are empty; the head
+// strides of their K hold the device's CUs and resident workgroups.
 template <int KB, int VB, bool RAGGED>
 __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
 #ifdef HYQ_PHASE_TRACE
@@ -1091,7 +1114,7 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
 #endif
     int head = blockIdx.x;
     int wg = blockIdx.y;                             // piece of the head
-    KArgs K = kernel_args(wg);
+    KArgs K = kernel_args(RAGGED ? min(wg, MAX_NWG - 1) : wg);
     int u0 = static_cast<int>(K.bnd[0]), u1 = static_cast<int>(K.bnd[1]);         // its schedule units
     const uint16_t* const qp = kptr<const uint16_t>(K, 0);
     const uint8_t* const kp = kptr<const uint8_t>(K, 2);
@@ -1113,8 +1136,9 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
     const int32_t skb0 = static_cast<int32_t>(kdw(K, 31)), skb1 = static_cast<int32_t>(kdw(K, 32));
     const int32_t skb2 = static_cast<int32_t>(kdw(K, 33)), svb0 = static_cast<int32_t>(kdw(K, 34));
     const int32_t svb1 = static_cast<int32_t>(kdw(K, 35)), svb2 = static_cast<int32_t>(kdw(K, 36));
-    const int nquant = static_cast<int>(kdw(K, 37));
-    const int sn0 = static_cast<int>(kdw(K, 38)), sn1 = static_cast<int>(kdw(K, 39)), sn2 = static_cast<int>(kdw(K, 40));
+    int nquant = static_cast<int>(kdw(K, 37));
+    int sn0 = static_cast<int>(kdw(K, 38));
+    const int sn1 = static_cast<int>(kdw(K, 39)), sn2 = static_cast<int>(kdw(K, 40));
     const int G = static_cast<int>(kdw(K, 41));
     int nqg = static_cast<int>(kdw(K, 42));
     int su0 = static_cast<int>(kdw(K, 43));
@@ -1125,7 +1149,9 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
     int pieces = 0, first = 0;                     // RAGGED: the head's pieces and first slot
     if constexpr (RAGGED) {
         epilogue_args(K);                          // (before anything can move the registers of those loads)
-        const RaggedPiece r = ragged_piece<KB, VB>(static_cast<int>(K.e1[3]), G, nquant, sn0, len_q, len_s0, u0, u1);
+        const int nwg = static_cast<int>(K.e1[1]);
+        RaggedPiece r{head, wg, nwg, head * nwg, u0, u1, nqg, su0, 0, 0};
+        ragged_piece<KB, VB>(r, static_cast<int>(K.e1[3]), G, nquant, sn0, len_q, len_s0, skb1, skb2);
         if (r.head < 0) return;
         head = r.head;
         wg = r.piece;
@@ -1134,6 +1160,8 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
         u0 = r.u0;
         u1 = r.u1;
         nqg = r.nqg;
+        nquant = r.nq;
+        sn0 = r.ns;
         su0 = r.nb;
     }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1170,7 +1198,7 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
         // ---------------- int4 part: groups wave, wave+WAVES, ... ----------------
         const int lo = u0 * GROUP;
         int nq = nquant;
-        if (len_q != nullptr) nq = min(nq, max(0, sload_i32(len_q + head)));
+        if (!RAGGED && len_q != nullptr) nq = min(nq, max(0, sload_i32(len_q + head)));
         const int ntok = max(0, min((min(u1, nqg) - u0) * GROUP, nq - lo));   // 0: past a ragged head's end
         QCtx x;
         x.k = make_rsrc(kp + static_cast<int64_t>(head) * kp_bh + static_cast<int64_t>(lo) * prow(KB),
@@ -1282,7 +1310,7 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
             if (ua >= ub) continue;
             const int lo = (ua - sb) * BUNIT;
             int seg_len = seg == 0 ? sn0 : seg == 1 ? sn1 : sn2;
-            if (seg == 0 && len_s0 != nullptr) seg_len = min(seg_len, max(0, sload_i32(len_s0 + head)));
+            if (!RAGGED && seg == 0 && len_s0 != nullptr) seg_len = min(seg_len, max(0, sload_i32(len_s0 + head)));
             const int n = max(0, min((ub - ua) * BUNIT, seg_len - lo));     // 0: past a ragged head's end
             const uint16_t* const skp = seg == 0 ? sk0 : seg == 1 ? sk1 : sk2;
             const uint16_t* const svp = seg == 0 ? sv0 : seg == 1 ? sv1 : sv2;
@@ -1953,7 +1981,9 @@ struct Slots {
 
 struct Plan {
     int nwg;               // pieces per head
-    int grid;              // workgroups of a ragged launch (0: nwg for each head)
+    int rows;              // workgroups per head that a ragged launch may have (0: none)
+    bool ragged;           // planned on the device
+    int cus, slots;        // of the device (rows > 0)
     int nqg, segu[3];      // schedule units: prefix units, bf16 units per segment
     int bnd[MAX_NWG + 1];  // piece p covers units [bnd[p], bnd[p+1])
 };
@@ -2194,18 +2224,22 @@ Slots resident_slots(int kb, int vb, int G) {
     }
 }
 
-// Ragged lengths are planned on the device (ragged_piece) where its limits
-// allow; else by the padded lengths, like a full batch.
+// Large calls with ragged lengths are planned on the device (ragged_piece);
+// the others by the padded lengths, like a full batch.  The workspace of a
+// ragged call is sized for the device's pieces either way.
 Plan plan_for(const hyq_decode_params* p, bool ragged = true) {
     const int kb = p->n_quant > 0 ? p->k_bits : 4, vb = p->n_quant > 0 ? p->v_bits : 4;
     const Slots sl = resident_slots(kb, vb, p->kv_repeat);
-    Plan pl = make_plan(group_units(p->n_quant, kb, vb), p->seg_n, p->bh_kv, p->kv_repeat, p->split_tokens, sl);
+    const PrefixUnits pre = group_units(p->n_quant, kb, vb);
+    Plan pl = make_plan(pre, p->seg_n, p->bh_kv, p->kv_repeat, p->split_tokens, sl);
     const bool lens = (p->n_quant > 0 && p->seq_lens_quant) || (p->seg_n[0] > 0 && p->seq_lens_seg0);
     if (ragged && lens && p->bh_kv <= RAGGED_HEADS && p->seg_n[1] == 0 && p->seg_n[2] == 0 && p->split_tokens <= 0 &&
         sl.slots > 0) {
-        pl.grid = ragged_grid(p->bh_kv, sl.cus, sl.slots);
-        pl.bnd[0] = sl.cus;
-        pl.bnd[1] = sl.slots;
+        const int64_t head_bytes = pre.units * pre.bytes + static_cast<int64_t>(pl.segu[0]) * BUNIT * 4 * D;
+        pl.rows = std::max(pl.nwg, (ragged_grid(p->bh_kv, sl.cus, sl.slots) + p->bh_kv - 1) / p->bh_kv);
+        pl.ragged = p->bh_kv * head_bytes >= RAGGED_BYTES;
+        pl.cus = sl.cus;
+        pl.slots = sl.slots;
     }
     return pl;
 }
@@ -2217,7 +2251,7 @@ struct Layout {
     size_t cnt, ml, part, total;
 };
 Layout layout(const Plan& pl, int bh_kv, int G) {
-    const size_t slots = (pl.grid > 0 ? static_cast<size_t>(pl.grid) : static_cast<size_t>(bh_kv) * std::max(pl.nwg, 1)) * G;
+    const size_t slots = static_cast<size_t>(bh_kv) * std::max({pl.nwg, pl.rows, 1}) * G;
     Layout L;
     L.cnt = 0;
     L.ml = static_cast<size_t>(CNT_CAP) * CNT_PAD * sizeof(uint32_t);
@@ -2466,7 +2500,11 @@ int launch_decode(const hyq_decode_params* p, const Plan& pl, const Layout& L, v
     a.qk_scale = p->sm_scale * LOG2E;
     a.nqg = pl.nqg; a.nwg = pl.nwg;
     a.mj = merge_batch(p->kv_repeat, pl.nwg);
-    for (int i = 0; i <= (pl.grid > 0 ? 1 : pl.nwg); ++i) a.bnd[i] = pl.bnd[i];
+    for (int i = 0; i <= pl.nwg; ++i) a.bnd[i] = pl.bnd[i];
+    if (pl.ragged) {
+        a.sk_bh[1] = pl.cus;
+        a.sk_bh[2] = pl.slots;
+    }
     char* ws = static_cast<char*>(workspace);
     a.cnt = reinterpret_cast<uint32_t*>(ws + L.cnt);
     a.ml = reinterpret_cast<float*>(ws + L.ml);
@@ -2476,12 +2514,12 @@ int launch_decode(const hyq_decode_params* p, const Plan& pl, const Layout& L, v
     hipStream_t s = static_cast<hipStream_t>(stream);
     // x: KV head, y: piece; workgroups dispatch x-fastest, so piece 0 of
     // every head goes first
-    const dim3 grid(static_cast<unsigned>(p->bh_kv), static_cast<unsigned>(pl.nwg)), block(THREADS);
+    const dim3 grid(static_cast<unsigned>(p->bh_kv), static_cast<unsigned>(pl.ragged ? pl.rows : pl.nwg)), block(THREADS);
     const size_t lds = lds_bytes(p->kv_repeat);
     const int bits = p->n_quant > 0 ? 10 * p->k_bits + p->v_bits : 44;   // no prefix: any instance
     auto launch = [&](auto k, auto v) {
         constexpr int KB = decltype(k)::value, VB = decltype(v)::value;
-        if (pl.grid > 0) decode_kernel<KB, VB, true><<<dim3(static_cast<unsigned>(pl.grid)), block, lds, s>>>(a);
+        if (pl.ragged) decode_kernel<KB, VB, true><<<grid, block, lds, s>>>(a);
         else decode_kernel<KB, VB, false><<<grid, block, lds, s>>>(a);
     };
     constexpr std::integral_constant<int, 2> b2;
@@ -2517,7 +2555,7 @@ int prepare(const hyq_decode_params* p, Plan& pl, Layout& L) {
 // A ragged call whose workspace is too small for the device's plan, but sized
 // for the padded lengths, runs by those.
 void fit_plan(const hyq_decode_params* p, size_t bytes, Plan& pl, Layout& L) {
-    if (bytes >= L.total || pl.grid == 0) return;
+    if (bytes >= L.total || pl.rows == 0) return;
     const Plan padded = plan_for(p, false);
     const Layout PL = layout(padded, p->bh_kv, p->kv_repeat);
     if (PL.total > bytes) return;
