@@ -1493,34 +1493,81 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
 // one folding of the scales among a 128-token group's chunks; BLK = 1 folds
 // them for every chunk.  Pieces, partials, arrival and merge are
 // decode_kernel's.
+//
+// Kernel arguments.  The numbered dwords are read in one batch of scalar
+// loads (legacy_args), so their layout is fixed, as DecArgs' is; qk_scale and
+// mj stand in the lines of the arguments read later, which that batch brings
+// into the scalar cache.
 struct LegArgs {
-    const uint16_t* q;
-    int64_t q_stride;
-    const uint8_t* kc;             // prefix codes [bh][n][16 * bits] (byte strides)
-    const uint8_t* vc;
-    int64_t kc_bh, kc_n, vc_bh, vc_n;
-    const uint16_t* ks;            // prefix scales [bh][groups][D] (element strides)
-    const uint16_t* vs;
-    int64_t ks_bh, ks_g, vs_bh, vs_g;
-    int64_t ks_rows, vs_rows;      // scale rows per head (the descriptors' ranges)
-    int n_leg, group;
-    int cpg;                       // chunks per scale group
-    int nqg;                       // prefix schedule units (blocks) per head
-    int segu[2];                   // bf16 schedule units (BUNIT tokens) of segments 0 and 1
+    const uint16_t* q;             // dwords 0-1
+    const uint8_t* kc;             // 2-3    prefix codes [bh][n][16 * bits] (byte strides)
+    const uint8_t* vc;             // 4-5
+    const uint16_t* ks;            // 6-7    prefix scales [bh][groups][D] (element head strides)
+    const uint16_t* vs;            // 8-9
+    int64_t kc_bh, vc_bh, ks_bh, vs_bh;   // 10-17
+    uint64_t cdiv;                 // 18-19  2^40 / cpg, rounded up
+    int32_t q_stride;              // 20
+    uint32_t kc_n, vc_n;           // 21-22  bytes between code rows
+    uint32_t ks_row, vs_row;       // 23-24  bytes between scale rows
+    uint32_t ks_bytes, vs_bytes;   // 25-26  bytes of a head's scale rows (the descriptors' ranges)
+    int32_t n_leg, group;          // 27-28
+    int32_t cpg;                   // 29     chunks per scale group
+    int32_t nqg;                   // 30     prefix schedule units (blocks) per head
+    int32_t G;                     // 31
+    int32_t segu[2];               // 32-33  bf16 schedule units (BUNIT tokens) of segments 0 and 1
+    int32_t sn[3];                 // 34-36
+    int32_t nwg;                   // 37
     const uint16_t* sk[3];         // top-k, staging, window rows [bh][n][D]
+    int32_t pad0[4];
+    float qk_scale;                // 48     sm_scale * log2(e)
+    int32_t pad1;
     const uint16_t* sv[3];
     int64_t sk_bh[3], sv_bh[3];
-    int sn[3];
-    int G;
-    float qk_scale;                // sm_scale * log2(e)
+    int32_t mj;                    // 68
+    int32_t pad2;
     float* part;
     float* ml;
     uint32_t* cnt;
     uint16_t* out;
     int64_t out_stride;
-    int nwg, mj;
-    int bnd[MAX_NWG + 1];          // piece p: schedule units [bnd[p], bnd[p + 1]) of its head
+    int32_t bnd[MAX_NWG + 1];      // piece p: schedule units [bnd[p], bnd[p + 1]) of its head
 };
+static_assert(offsetof(LegArgs, cdiv) == 4 * 18 && offsetof(LegArgs, nqg) == 4 * 30 && offsetof(LegArgs, nwg) == 4 * 37 &&
+                  offsetof(LegArgs, qk_scale) == 4 * 48 && offsetof(LegArgs, mj) == 4 * 68 &&
+                  offsetof(LegArgs, bnd) == 4 * 80, "argument block layout");
+
+// The numbered arguments and the piece's bounds in one batch with one wait.
+// Left to the compiler they came in five round trips one after the other (q,
+// the bounds, the groups, the strides, the pointers), with two divisions
+// between them, which show in a short cache's call of 7-10 us.
+struct LegK {
+    u32x16 a, b;
+    u32x8 c;
+    u32x2 bnd;
+    uint32_t qk_scale, mj;
+    __device__ __forceinline__ uint32_t d(int i) const { return i < 16 ? a[i] : i < 32 ? b[i - 16] : c[i - 32]; }
+    __device__ __forceinline__ int i(int n) const { return static_cast<int>(d(n)); }
+    __device__ __forceinline__ uint64_t q(int n) const { return d(n) | static_cast<uint64_t>(d(n + 1)) << 32; }
+    template <typename T>
+    __device__ __forceinline__ const T* p(int n) const { return reinterpret_cast<const T*>(static_cast<uintptr_t>(q(n))); }
+};
+__device__ __forceinline__ LegK legacy_args(int wg) {
+    const char* const base = (const char*)__builtin_amdgcn_kernarg_segment_ptr();
+    const char* const bp = base + offsetof(LegArgs, bnd) + 4 * wg;
+    LegK k;
+    asm volatile(
+        "s_load_dwordx16 %0, %6, 0x0\n\t"
+        "s_load_dwordx16 %1, %6, 0x40\n\t"
+        "s_load_dwordx8 %2, %6, 0x80\n\t"
+        "s_load_dwordx2 %3, %7, 0x0\n\t"
+        "s_load_dword %4, %6, 0xc0\n\t"
+        "s_load_dword %5, %6, 0x110\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&s"(k.a), "=&s"(k.b), "=&s"(k.c), "=&s"(k.bnd), "=&s"(k.qk_scale), "=&s"(k.mj)
+        : "s"(base), "s"(bp)
+        : "memory");
+    return k;
+}
 
 // one 32-token chunk, in QRaw's layout (the scales are per group)
 template <int KB, int VB>
@@ -1741,7 +1788,9 @@ __global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
 #endif
     const int head = blockIdx.x;
     const int wg = blockIdx.y;
-    const int G = a.G;
+    const LegK K = legacy_args(wg);
+    const int G = K.i(31);
+    const int64_t h64 = head;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int c = lane & 15, kb = lane >> 4;
@@ -1762,38 +1811,49 @@ __global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
     // Q row of head c (zero for c >= G): channels 32kb..32kb+31
     u32x4 qs[4];
     {
-        const Rsrc rq = make_rsrc(a.q + static_cast<int64_t>(head) * G * a.q_stride,
-                                  static_cast<uint32_t>(G * a.q_stride * 2));
-        const uint32_t qo = static_cast<uint32_t>(c * a.q_stride * 2 + 64 * kb);
+        const int q_stride = K.i(20);
+        const Rsrc rq = make_rsrc(K.p<uint16_t>(0) + h64 * G * q_stride, static_cast<uint32_t>(G * q_stride * 2));
+        const uint32_t qo = static_cast<uint32_t>(c * q_stride * 2 + 64 * kb);
 #pragma unroll
         for (int i = 0; i < 4; ++i) qs[i] = bld128(rq, qo + 16 * i);
     }
 
-    const int u0 = a.bnd[wg], u1 = a.bnd[wg + 1];   // this piece's schedule units
-    if (u0 < a.nqg) {
-        // chunk x of the head: group x / cpg, tokens [x / cpg * group + 32 (x % cpg), ...)
-        const int cpg = a.cpg, group = a.group;
-        auto chunk_token = [&](int x) { return x / cpg * group + x % cpg * GROUP; };
-        const int x0 = u0 * BLK, x1 = min(u1, a.nqg) * BLK;
+    const int u0 = static_cast<int>(K.bnd[0]), u1 = static_cast<int>(K.bnd[1]);   // this piece's schedule units
+    const int nqg = K.i(30);
+    if (u0 < nqg) {
+        // chunk x of the head: group x / cpg, tokens [x / cpg * group + 32 (x % cpg), ...).
+        // The quotient by multiplication: exact while x * cpg <= 2^40 (x is at
+        // most 2^20 chunks and the loads past them, cpg at most 2^19)
+        const int cpg = K.i(29), group = K.i(28), n_leg = K.i(27);
+        const float qk_scale = __uint_as_float(K.qk_scale);
+        const uint64_t cdiv = K.q(18);
+        auto chunk_group = [&](int x) { return static_cast<int>(static_cast<uint32_t>(x) * cdiv >> 40); };
+        auto chunk_token = [&](int x) {
+            const int g = chunk_group(x);
+            return g * group + (x - g * cpg) * GROUP;
+        };
+        const int x0 = u0 * BLK, x1 = min(u1, nqg) * BLK;
         const int lo = chunk_token(x0);
-        const int n = min(a.n_leg, chunk_token(x1)) - lo;      // the piece's tokens
-        const uint32_t kc_n = static_cast<uint32_t>(a.kc_n), vc_n = static_cast<uint32_t>(a.vc_n);
-        const uint32_t ks_row = static_cast<uint32_t>(a.ks_g * 2), vs_row = static_cast<uint32_t>(a.vs_g * 2);
-        const Rsrc rk = make_rsrc(a.kc + head * a.kc_bh + lo * a.kc_n, static_cast<uint32_t>(n) * kc_n);
-        const Rsrc rv = make_rsrc(a.vc + head * a.vc_bh + lo * a.vc_n, static_cast<uint32_t>(n) * vc_n);
-        const Rsrc rks = make_rsrc(a.ks + head * a.ks_bh, static_cast<uint32_t>(a.ks_rows) * ks_row);
-        const Rsrc rvs = make_rsrc(a.vs + head * a.vs_bh, static_cast<uint32_t>(a.vs_rows) * vs_row);
+        const int n = min(n_leg, chunk_token(x1)) - lo;        // the piece's tokens
+        const uint32_t kc_n = K.d(21), vc_n = K.d(22), ks_row = K.d(23), vs_row = K.d(24);
+        const int64_t lo64 = lo;
+        const Rsrc rk = make_rsrc(K.p<uint8_t>(2) + h64 * static_cast<int64_t>(K.q(10)) + lo64 * kc_n,
+                                  static_cast<uint32_t>(n) * kc_n);
+        const Rsrc rv = make_rsrc(K.p<uint8_t>(4) + h64 * static_cast<int64_t>(K.q(12)) + lo64 * vc_n,
+                                  static_cast<uint32_t>(n) * vc_n);
+        const Rsrc rks = make_rsrc(K.p<uint16_t>(6) + h64 * static_cast<int64_t>(K.q(14)), K.d(25));
+        const Rsrc rvs = make_rsrc(K.p<uint16_t>(8) + h64 * static_cast<int64_t>(K.q(16)), K.d(26));
         const uint32_t klane = static_cast<uint32_t>(krow_token(c)) * kc_n + 4 * KB * kb;
         const uint32_t vlane = static_cast<uint32_t>(kb) * vc_n + VB * c;
         const int nblk = (x1 - x0) / BLK;
         // first token (from lo) and scale group of block b of the piece
         auto block_at = [&](int b, int& g) {
             const int x = x0 + b * BLK;
-            g = __builtin_amdgcn_readfirstlane(x / cpg);
+            g = __builtin_amdgcn_readfirstlane(chunk_group(x));
             return __builtin_amdgcn_readfirstlane(g * group + (x - g * cpg) * GROUP - lo);
         };
         // tokens of the group (and the prefix) from chunk start t on
-        auto valid = [&](int t, int g) { return min((g + 1) * group, a.n_leg) - lo - t; };
+        auto valid = [&](int t, int g) { return min((g + 1) * group, n_leg) - lo - t; };
         f32x4 tot[8];
 #pragma unroll
         for (int nb = 0; nb < 8; ++nb) tot[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1823,7 +1883,7 @@ __global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
                 float qk;
                 {
                     const u32x4 qn[4] = {s_q[0][lane], s_q[1][lane], s_q[2][lane], s_q[3][lane]};
-                    legacy_q_operand<KB>(qop, kbias, qk, qn, ksc, a.qk_scale, qex);
+                    legacy_q_operand<KB>(qop, kbias, qk, qn, ksc, qk_scale, qex);
                 }
                 legacy_scales(vsc, rvs, g, vs_row, lane);
 #pragma unroll
@@ -1858,7 +1918,7 @@ __global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
                 f16x8 qop[4];
                 f32x4 kbias;
                 float qk;
-                legacy_q_operand<KB>(qop, kbias, qk, qs, y.ks, a.qk_scale, qex);
+                legacy_q_operand<KB>(qop, kbias, qk, qs, y.ks, qk_scale, qex);
                 legacy_compute<KB, VB>(st, tot, y.r, qop, kbias, qk, valid(y.t, y.g), lane);
                 legacy_flush<VB>(st, tot, y.vs);
             };
@@ -1878,14 +1938,15 @@ __global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
                               __builtin_bit_cast(bf16x8, qs[2]), __builtin_bit_cast(bf16x8, qs[3])};
         constexpr int TSTRIDE = WAVES * TILE;
         const int t0 = wave * TILE;
-        const int b1 = a.nqg + a.segu[0], b2 = b1 + a.segu[1];
+        const float qk_scale = __uint_as_float(K.qk_scale);
+        const int b1 = nqg + K.i(32), b2 = b1 + K.i(33);
         const int sg = u0 < b1 ? 0 : u0 < b2 ? 1 : 2;            // a piece lies inside one segment
-        const int lo = (u0 - (sg == 0 ? a.nqg : sg == 1 ? b1 : b2)) * BUNIT;
-        const int n = min((u1 - u0) * BUNIT, a.sn[sg] - lo);
+        const int lo = (u0 - (sg == 0 ? nqg : sg == 1 ? b1 : b2)) * BUNIT;
+        const int n = min((u1 - u0) * BUNIT, (sg == 0 ? K.i(34) : sg == 1 ? K.i(35) : K.i(36)) - lo);
         const int ntile = (n + TILE - 1) / TILE;
         const int nmine = ntile > wave ? (ntile - wave + WAVES - 1) / WAVES : 0;
-        const uint16_t* kbase = a.sk[sg] + head * a.sk_bh[sg] + static_cast<int64_t>(lo) * BROW;
-        const uint16_t* vbase = a.sv[sg] + head * a.sv_bh[sg] + static_cast<int64_t>(lo) * BROW;
+        const uint16_t* kbase = a.sk[sg] + h64 * a.sk_bh[sg] + static_cast<int64_t>(lo) * BROW;
+        const uint16_t* vbase = a.sv[sg] + h64 * a.sv_bh[sg] + static_cast<int64_t>(lo) * BROW;
         const uint32_t nbytes = static_cast<uint32_t>(n) * (BROW * 2);
         const Rsrc rk = make_rsrc(kbase, nbytes), rv = make_rsrc(vbase, nbytes);
         Bf16Raw r0, r1;
@@ -1893,17 +1954,18 @@ __global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
         bf16_load(r1, rk, rv, t0 + TSTRIDE, lane);
         for (int i = 0; i < nmine; i += 2) {
             const int t = t0 + i * TSTRIDE;
-            bf16_compute(st, r0, qb, n - t, lane, a.qk_scale);
+            bf16_compute(st, r0, qb, n - t, lane, qk_scale);
             if (i + 1 >= nmine) break;
             bf16_load(r0, rk, rv, t + 2 * TSTRIDE, lane);
-            bf16_compute(st, r1, qb, n - t - TSTRIDE, lane, a.qk_scale);
+            bf16_compute(st, r1, qb, n - t - TSTRIDE, lane, qk_scale);
             if (i + 2 >= nmine) break;
             bf16_load(r1, rk, rv, t + 3 * TSTRIDE, lane);
         }
     }
 
     // ---- wave -> LDS -> this piece's partial, then decode_kernel's arrival protocol ----
-    const MergeArgs ma{G, a.nwg, static_cast<int64_t>(head) * a.nwg, a.part, a.ml, a.out, a.out_stride, 0};
+    const int nwg = K.i(37), mj = static_cast<int>(K.mj);
+    const MergeArgs ma{G, nwg, h64 * nwg, a.part, a.ml, a.out, a.out_stride, 0};
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the rings' last (empty) loads
     st.l = col_sum(st.l);
     if (kb == 0) {
@@ -1957,7 +2019,7 @@ __global__ __launch_bounds__(THREADS, 2) void legacy_decode_kernel(LegArgs a) {
     __syncthreads();
     if (s_last) {
         if (threadIdx.x == 0) __hip_atomic_store(a.cnt + head * CNT_PAD, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        switch (a.mj) {
+        switch (mj) {
             case 4: merge_head_waves<4>(ma, head, s_acc TRACE_ARG); break;
             case 8: merge_head_waves<8>(ma, head, s_acc TRACE_ARG); break;
             case 12: merge_head_waves<12>(ma, head, s_acc TRACE_ARG); break;
@@ -2419,15 +2481,20 @@ int validate_legacy(const hyq_legacy_params* p) {
 
 int launch_legacy(const hyq_legacy_params* p, const Plan& pl, const Layout& L, void* workspace, void* stream) {
     LegArgs a{};
-    a.q = p->q; a.q_stride = p->q_stride;
+    a.q = p->q; a.q_stride = static_cast<int32_t>(p->q_stride);
     a.kc = p->k_codes; a.vc = p->v_codes;
-    a.kc_bh = p->kc_stride_bh; a.kc_n = p->kc_stride_n; a.vc_bh = p->vc_stride_bh; a.vc_n = p->vc_stride_n;
+    a.kc_bh = p->kc_stride_bh; a.vc_bh = p->vc_stride_bh;
+    a.kc_n = static_cast<uint32_t>(p->kc_stride_n); a.vc_n = static_cast<uint32_t>(p->vc_stride_n);
     a.ks = p->k_scale; a.vs = p->v_scale;
-    a.ks_bh = p->ks_stride_bh; a.ks_g = p->ks_stride_g; a.vs_bh = p->vs_stride_bh; a.vs_g = p->vs_stride_g;
+    a.ks_bh = p->ks_stride_bh; a.vs_bh = p->vs_stride_bh;
     a.group = p->n > 0 ? legacy_group(p) : GROUP;
-    a.ks_rows = a.vs_rows = (p->n + a.group - 1) / a.group;
+    const int64_t rows = (p->n + a.group - 1) / a.group;
+    a.ks_row = static_cast<uint32_t>(p->ks_stride_g * 2); a.vs_row = static_cast<uint32_t>(p->vs_stride_g * 2);
+    a.ks_bytes = static_cast<uint32_t>(rows * p->ks_stride_g * 2);
+    a.vs_bytes = static_cast<uint32_t>(rows * p->vs_stride_g * 2);
     a.n_leg = static_cast<int>(p->n);
     a.cpg = (a.group + GROUP - 1) / GROUP;
+    a.cdiv = ((uint64_t{1} << 40) + a.cpg - 1) / a.cpg;
     a.nqg = pl.nqg;
     a.segu[0] = pl.segu[0]; a.segu[1] = pl.segu[1];
     for (int s = 0; s < 3; ++s) {

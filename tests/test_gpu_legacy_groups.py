@@ -20,6 +20,8 @@ pytestmark = pytest.mark.gpu
     (2, 16, 33, 128, 2, 2, False),       # one token past a chunk
     (3, 1, 1, 128, 4, 2, False),
     (3, 4, 129, 4096, 4, 4, True),       # the group longer than the prefix
+    (3, 4, 700, 96, 4, 2, False),        # three chunks a group
+    (2, 4, 1200, 1184, 2, 4, False),     # 37 chunks in the first, one in the second
     (128, 2, 1100, 112, 4, 4, False),    # blocks of four chunks, the last 16 tokens
     (130, 4, 1151, 128, 2, 4, True),     # blocks of four, one token short of a chunk
     (128, 8, 1153, 256, 4, 2, False),    # two blocks per group, one token in the last

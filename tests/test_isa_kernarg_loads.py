@@ -30,7 +30,9 @@ def _regs(text):
     return out
 
 
-def test_epilogue_argument_loads_are_not_read_before_their_wait():
+@pytest.fixture(scope="module")
+def lines():
+    """decode.hip's device code as lines of assembly."""
     from hyquant_amd.build import HIPCC_FLAGS, hipcc
     if not os.path.exists(hipcc()):
         pytest.skip("hipcc not available")
@@ -40,7 +42,10 @@ def test_epilogue_argument_loads_are_not_read_before_their_wait():
         proc = subprocess.run([hipcc(), *flags, "--cuda-device-only", "-S", "-o", asm, SRC],
                               capture_output=True, text=True)
         assert proc.returncode == 0, proc.stderr[-2000:]
-        lines = open(asm).read().split("\n")
+        return open(asm).read().split("\n")
+
+
+def test_epilogue_argument_loads_are_not_read_before_their_wait(lines):
     kernel, checked, bad = None, 0, []
     for i, line in enumerate(lines):
         if re.match(r"^_Z\S*decode_kernel\S*:", line):
@@ -63,3 +68,25 @@ def test_epilogue_argument_loads_are_not_read_before_their_wait():
                 bad.append((kernel, j + 1, t))
     assert checked >= 2, "no epilogue argument loads found: the test no longer matches the kernel"
     assert not bad, bad[:5]
+
+
+def test_legacy_kernels_start_streaming_after_one_batch_of_arguments(lines):
+    """A short legacy cache's call shows every round trip before its first
+    loads: one for the arguments, and a second, for their segment's pointers,
+    in the pieces of 16-bit rows."""
+    kernels = {}
+    kernel = None
+    for line in lines:
+        if re.match(r"^_Z\S*legacy_decode_kernel\S*:", line):
+            kernel = line.split(":")[0]
+            kernels[kernel] = [0, False]             # scalar waits before the first streaming load, seen
+        elif kernel is not None:
+            t = line.split(";")[0]
+            if re.search(r"buffer_load_\S+ .*\bnt\b", t):
+                kernels[kernel][1] = True
+            if "s_waitcnt" in t and "lgkmcnt" in t and not kernels[kernel][1]:
+                kernels[kernel][0] += 1
+            if "s_endpgm" in t:
+                kernel = None
+    assert len(kernels) == 8, sorted(kernels)
+    assert all(seen and waits <= 2 for waits, seen in kernels.values()), kernels
