@@ -70,6 +70,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <mutex>
 #include <string>
 
@@ -2057,10 +2058,12 @@ struct PrefixUnits {
     int tokens;            // per unit (full ones)
     int64_t bytes;         // per unit
     int64_t span;          // per unit, from its first row of K or V (the wider) to the next unit's
+    int64_t conv;          // what converting a unit's codes costs, in bytes that a workgroup could read meanwhile
+    bool legacy;
 };
 PrefixUnits group_units(int64_t n_quant, int kb, int vb) {
     return {(n_quant + GROUP - 1) / GROUP, GROUP, static_cast<int64_t>(GROUP) * (16 * kb + 16 * vb + 4),
-            static_cast<int64_t>(GROUP) * 16 * std::max(kb, vb)};
+            static_cast<int64_t>(GROUP) * 16 * std::max(kb, vb), kb + vb <= 8 ? 4750 : 9250, false};
 }
 
 // Bytes from a piece's first row to its end, in K or in V: its descriptors and
@@ -2079,19 +2082,27 @@ size_t round256(size_t x) { return (x + 255) / 256 * 256; }
 //     per-piece round trips), G <= 4: every segment cut into pieces of
 //     equal bytes, total / (0.8 CUs) (measured best at B=1 from 2K to 32K
 //     prefixes), at most 48 per head.
-//   up to 64 KV heads and a launch of less than 48 MB (G <= 4) or 80 MB (G > 4;
-//     any size with fewer than 20 heads), 7-25 us that mix one piece's latency
-//     and the merge: the piece count with the least modelled time
-//     (cheapest_pieces).  Swept over 200 shapes (32/8, 64/8 and 32/2 heads,
-//     batches 1-32, 1K-32K tokens; graph replay over 400 MB of copies): in this
-//     range it is 1-2% above each shape's best piece count on average, where
-//     power-of-two pieces (fewer than 32 heads) and 1.25 rounds of at least
-//     96 KiB were 19% above.  12 x 2 heads, G = 16, 4096 tokens 20.5 -> 11.7 us;
-//     3 x 8 heads, G = 8, 4000 tokens 17.7 -> 10.9 us; 4 x 8 heads, G = 4,
-//     1024 tokens 9.6 -> 7.2 us.
-//   G > 8, 20 to 64 KV heads and 60 MB or more: 12 pieces, the most that the
-//     merge loads in one batch (48 heads, 16384 tokens 33.7 -> 29.5 us, 13001
-//     tokens with 2-bit V 27.5 -> 23.4 us; 32 heads, 32768 tokens 38.8 -> 36.8).
+//   up to 64 KV heads and a launch of less than 48 MB (G <= 4, fewer than 32
+//     heads in the legacy format only) or 80 MB (G > 4; any size with fewer
+//     than 20 heads, or with G > 8 and codes of more than 8 bits a pair), 7-25
+//     us that mix one piece's latency and the merge: the piece count with the
+//     least modelled time (cheapest_pieces).  Swept over 515 shapes (32/8,
+//     64/8 and 32/2 heads, batches 1-32, 1K-30K tokens, K4V4, K4V2 and K8V8;
+//     graph replay over 700 MB of copies) and every count: 0.2% above each
+//     shape's best on average, 4% at the worst, and up to 3% above
+//     power-of-two pieces (fewer than 32 heads) and 1.25 rounds of at least 96
+//     KiB, which are 11% above it on average.  6 x 2 heads, G = 16, 3600
+//     tokens 15.3 (power-of-two pieces) -> 11.0 us; 5 x 8 heads, G = 4, 5151
+//     tokens of K4V2 11.9 (1.25 rounds; 13.4 in pieces of equal bytes) ->
+//     11.5; legacy 2-bit codes, 3 x 8 heads, 5151 tokens 17.4 (equal bytes) ->
+//     12.2, 4 x 3600 16.1 -> 10.9.
+//   G > 8, 20 to 64 KV heads, 60 MB or more and codes of at most 8 bits a
+//     pair: 12 pieces, the most that the merge loads in one batch (48 heads,
+//     16384 tokens 33.4 (1.25 rounds) -> 30.0 us, 13001 tokens with 2-bit V
+//     25.9 -> 24.2; 32 heads, 30000 tokens 35.9 -> 35.2; 64 heads within 1%
+//     of 1.25 rounds).  8-bit codes take longer per piece and lose by the
+//     second round (32 heads, 30000 tokens 62.5 us in 1.25 rounds, 73.2 in 12
+//     pieces, 54.2 in the model's ten).
 //   else: pieces of about total / (1.25 * slots) bytes, `slots`
 //     being the workgroups the device holds at once: the first round fills
 //     every slot and the remaining quarter, with the short segment pieces,
@@ -2145,19 +2156,35 @@ int merge_loads(int G, int k) {
 }
 
 // The piece count (at most kmax, and 15/16 of the resident slots: a full
-// device starts its last workgroups late) with the least modelled time, in us:
-// the largest piece at 32 KB/us on a CU of its own or 26 KB/us shared by a
-// CU's two, plus 0.05 (G <= 4, a wavefront's merge) or 0.095 (a workgroup's)
-// per partial loaded.  Fitted to the sweep above.
-Pieces cheapest_pieces(const Pieces& fewest, int bh_kv, int G, int kmax, int64_t slots, int64_t cus) {
+// device starts its last workgroups late) with the least modelled time, in us.
+// The grid runs piece by piece and fills every CU once, then a second time, so
+// workgroup j shares its CU with workgroup j + cus: what both have to do at
+// 32 KB/us and 0.2 us for the sharing, what the larger has left at 36.5 KB/us;
+// plus 0.053 (G <= 4, a wavefront's merge) or 0.175 (a workgroup's) per
+// partial loaded.  A unit of codes counts for more than its bytes (conv).
+// Fitted to the sweep above.
+Pieces cheapest_pieces(const Pieces& fewest, int64_t conv, int bh_kv, int G, int kmax, int64_t slots, int64_t cus) {
     Pieces p = fewest, best = p;
     const int most = std::min<int64_t>(kmax, std::max<int64_t>(p.total, slots * 15 / 16 / bh_kv));
     double least = 1e30;
     for (;;) {
-        const double m = static_cast<double>(p.size[p.largest()]);
-        const double wgs = static_cast<double>(p.total) * bh_kv;
-        const double stream = wgs <= cus ? m / 32e3 : std::max(m / 32e3, 2.0 * m * (wgs / slots) / 26e3);
-        const double cost = stream + (G <= WAVES ? 0.05 : 0.095) * merge_loads(G, p.total);
+        double w[4];                    // modelled bytes of a segment's largest piece
+        int64_t end[4];                 // workgroups up to the segment's last
+        for (int s = 0; s < 4; ++s) {
+            w[s] = static_cast<double>(p.size[s]);
+            if (s == 0 && p.ks[0] > 0) w[0] += static_cast<double>((p.su[0] + p.ks[0] - 1) / p.ks[0] * conv);
+            end[s] = (s > 0 ? end[s - 1] : 0) + static_cast<int64_t>(p.ks[s]) * bh_kv;
+        }
+        double stream = 0;
+        int x = 0, y = 0;               // the segments of workgroups j and j + cus
+        for (int64_t j = 0; j < std::min(cus, end[3]);) {
+            while (end[x] <= j) ++x;
+            while (y < 4 && end[y] <= j + cus) ++y;
+            const double u = w[x], v = y < 4 ? w[y] : 0.0;
+            stream = std::max(stream, 2.0 * std::min(u, v) / 32e3 + std::fabs(u - v) / 36.5e3 + (v > 0 ? 0.2 : 0.0));
+            j = y < 4 ? std::min(end[x], end[y] - cus) : end[x];
+        }
+        const double cost = stream + (G <= WAVES ? 0.053 : 0.175) * merge_loads(G, p.total);
         if (cost < least) {
             least = cost;
             for (int s = 0; s < 4; ++s) best.ks[s] = p.ks[s];
@@ -2204,11 +2231,14 @@ Plan make_plan(const PrefixUnits& pre, const int64_t seg_n[3], int bh_kv, int G,
     };
     int total;
     int64_t target;
-    const bool twelve = G > 8 && bh_kv >= 20 && bh_kv <= 64 && head_bytes * bh_kv >= 60000000;
+    const bool wide = cq > static_cast<int64_t>(pre.tokens) * (16 * 8 + 4);   // codes of more than 8 bits a pair
+    const bool large = G > 8 && bh_kv >= 20 && head_bytes * bh_kv >= 60000000;
+    const bool twelve = large && !wide;
+    const bool small = head_bytes * bh_kv < (G <= WAVES ? 48000000 : 80000000);
     if (requested > 0) {
         target = std::max<int64_t>(1, (requested + pre.tokens - 1) / pre.tokens) * cq;
         total = counts_for(target);
-    } else if (bh_kv < 32 && G <= WAVES) {
+    } else if (bh_kv < 32 && G <= WAVES && !(pre.legacy && small)) {
         // few heads, G <= 4: pieces of equal bytes, about 0.8 per CU (a
         // workgroup per CU streams faster than two sharing one, and the
         // merge grows with the piece count), at least 8 KiB and at most 48
@@ -2217,12 +2247,13 @@ Plan make_plan(const PrefixUnits& pre, const int64_t seg_n[3], int bh_kv, int G,
         target = std::max<int64_t>(8 << 10, head_bytes * bh_kv * 5 / (4 * cus));
         target = std::max<int64_t>(target, (head_bytes + 47) / 48);
         total = counts_for(target);
-    } else if (bh_kv <= 64 && (twelve || bh_kv < 20 || head_bytes * bh_kv < (G <= WAVES ? 48000000 : 80000000))) {
+    } else if (bh_kv <= 64 && (small || large || bh_kv < 20)) {
         Pieces best(su, sc, least);
         if (twelve) {
             while (best.total < std::min(kmax, 12) && best.split()) {}
         } else {
-            best = cheapest_pieces(best, bh_kv, G, kmax, slots > 0 ? slots : 512, sl_.cus > 0 ? sl_.cus : 256);
+            best = cheapest_pieces(best, pre.conv, bh_kv, G, kmax, slots > 0 ? slots : 512,
+                                   sl_.cus > 0 ? sl_.cus : 256);
         }
         for (int s = 0; s < 4; ++s) ks[s] = best.ks[s];
         total = best.total;
@@ -2385,10 +2416,10 @@ int legacy_group(const hyq_legacy_params* p) {
 // Chunks per block: four, which share one folding of the scales, when the
 // group's chunk count is a multiple of four (128-token groups) and one
 // workgroup per CU gets a block for each of its wavefronts; else single
-// chunks, which spread a short cache over more wavefronts (8 KV heads at 1100
-// tokens, kernel time: 7.8 us with single chunks, 9.5 us with blocks of four;
-// at 31000 tokens, where the rule changes over, 16.6 us with blocks against
-// 20.5 us for dequantising every element).
+// chunks, which spread a short cache over more wavefronts.  Kernel time with
+// the best piece count of each, single chunks / blocks: 8 KV heads at 1100
+// tokens 6.7 / 8.3 us, at 7300 8.8 / 9.1, at 10000 9.9 / 9.5, at 30000 16.8 /
+// 14.7; 32 heads at 1100 8.1 / 8.8, at 3600 11.1 / 10.6, at 7300 15.7 / 13.8.
 int legacy_blk(const hyq_legacy_params* p, int cus) {
     const int64_t cpg = (legacy_group(p) + GROUP - 1) / GROUP;
     return cpg % 4 == 0 && p->n / (4 * GROUP) * p->bh_kv >= WAVES * (cus > 0 ? cus : 256) ? 4 : 1;
@@ -2413,7 +2444,7 @@ Slots legacy_slots(int kb, int vb, int blk, int G) {
 }
 
 Plan legacy_plan(const hyq_legacy_params* p) {
-    PrefixUnits pre{0, GROUP, 1, 1};
+    PrefixUnits pre{0, GROUP, 1, 1, 0, true};
     int blk = 4;
     if (p->n > 0) {
         const int group = legacy_group(p);
@@ -2423,6 +2454,7 @@ Plan legacy_plan(const hyq_legacy_params* p) {
         pre.tokens = blk * GROUP;
         pre.bytes = static_cast<int64_t>(pre.tokens) * (16 * p->k_bits + 16 * p->v_bits) + 4 * D;
         pre.span = std::min<int64_t>(pre.tokens, group) * std::max(p->kc_stride_n, p->vc_stride_n);
+        pre.conv = blk == 4 ? 44000 : 20500;
     }
     return make_plan(pre, p->seg_n, p->bh_kv, p->kv_repeat, 0, legacy_slots(p->k_bits, p->v_bits, blk, p->kv_repeat));
 }
