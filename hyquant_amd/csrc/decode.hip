@@ -953,21 +953,27 @@ __host__ __device__ inline int merge_batch(int G, int nwg) {
 // merge tables and, with G > 4, for the merge to load a head's partials in one
 // or two batches.  The grid covers any lengths (ragged_grid).
 //
-// Both plans over 400 calls (32/8 heads K4V4 and K8V8, 64/8 K4V2, 32/2 K4V4;
-// batches 2-32, longest 1K-32K tokens, shortest 600 tokens to the longest):
-//   - reading the lengths costs a launch 0.1-1.5 us: up to 2% of the calls from
-//     240 MB of padded bytes on that then keep the padded plan (41 us and
-//     more), 5-10% of a 7 us call;
-//   - from 240 MB on and filled to less than 60% the device's pieces are the
-//     faster ones (16 sequences of 600 to 32000 tokens 63.3 -> 37.8 us, 32/2
-//     heads 33.2 -> 21.5, 8 sequences 36.2 -> 25.8; 8000 to 32000, filled to
-//     55%, 72.2 -> 64.1); at 73% they take -14 to +12%, full -7 to +12%;
-//   - below 240 MB the coarser pieces and that cost outweigh the balance (2 x 1000-2000 tokens 7.3 -> 8.8 us, 16 x
-//     2000 14.8 -> 19.4), except for some very ragged calls (4 x 600-32000,
-//     157 MB, 25.6 -> 22.5).
+// Both plans over 570 calls of up to 256 heads (32/8, 64/8 and 32/2 heads;
+// K4V4, K4V2 and K8V8; batches 2-32, longest 2.5K-30K tokens; evenly spread,
+// log-spread, one long among short, nearly equal lengths), device / padded:
+//   - reading the lengths and planning costs 0.7-1.1 us of a launch whatever it
+//     then takes: 4-5% of calls of 60-130 MB of padded bytes that keep the
+//     padded plan, 2-4% from 130 MB on, 1% from 240 MB on, 5-15% of a 7-14 us
+//     call;
+//   - filled to less than 60% the device's pieces are the faster ones from 90
+//     MB on: 0.66-0.86 times the padded plan's time (mean 0.77) at less than a
+//     quarter, 0.82 to 40%, 0.94 to 50%, 0.99 to 60% at 90-130 MB, where the
+//     two lines lie; 0.55, 0.68, 0.78 and 0.89 from 240 MB on (16 sequences
+//     of 600 to 32000 tokens 63.3 -> 37.8 us; 16 on two key heads, 154 MB,
+//     29.8 -> 22; 4 at G = 8, 154 MB, 27.2 -> 20);
+//   - at 60-80% and above they gain nothing (0.86-1.12 times), hence the fill;
+//   - at 20-60 MB the coarser pieces and the cost outweigh the balance (1.07
+//     and 1.0 times on average, to 1.27).
+// More than four heads per lane would take registers from every ragged launch
+// (sixteen: 10-25% slower), so more than 256 heads keep the padded plan.
 constexpr int RAGGED_HEADS = 256;        // four per lane
 constexpr float RAGGED_FILL = 0.6f;
-constexpr int64_t RAGGED_BYTES = 240000000;
+constexpr int64_t RAGGED_BYTES = 100000000;
 
 // pieces a ragged launch can have: total / target, and one rounded up per
 // head and segment
