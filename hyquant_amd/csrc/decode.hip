@@ -217,6 +217,15 @@ constexpr int TRACE_PH = 14;
 __device__ uint64_t g_trace[TRACE_SLOTS][TRACE_MAX_WG * 4][TRACE_PH];
 __device__ uint32_t g_trace_launch;
 __device__ uint32_t g_trace_done;
+// One workgroup has ended (called by one of its threads): the launch's last
+// advances the ring.
+__device__ __forceinline__ void trace_end() {
+    const uint32_t total = gridDim.x * gridDim.y;
+    if (__hip_atomic_fetch_add(&g_trace_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
+        __hip_atomic_store(&g_trace_done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(&g_trace_launch, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
 #define HYQ_STAMP(i) (ph[i] = __builtin_amdgcn_s_memrealtime())
 #define TRACE_PARAM , uint64_t (&ph)[TRACE_PH]
 #define TRACE_ARG , ph
@@ -1159,7 +1168,12 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
         const int nwg = static_cast<int>(K.e1[1]);
         RaggedPiece r{head, wg, nwg, head * nwg, u0, u1, nqg, su0, 0, 0};
         ragged_piece<KB, VB>(r, static_cast<int>(K.e1[3]), G, nquant, sn0, len_q, len_s0, skb1, skb2);
-        if (r.head < 0) return;
+        if (r.head < 0) {
+#ifdef HYQ_PHASE_TRACE
+            if (threadIdx.x == 0) trace_end();
+#endif
+            return;
+        }
         head = r.head;
         wg = r.piece;
         pieces = r.pieces;
@@ -1452,13 +1466,7 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
         for (int i = 0; i < TRACE_PH; ++i) dst[i] = ph[i];
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t total = gridDim.x * gridDim.y;
-        if (__hip_atomic_fetch_add(&g_trace_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
-            __hip_atomic_store(&g_trace_done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&g_trace_launch, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
+    if (threadIdx.x == 0) trace_end();
 #endif
 }
 
