@@ -6,11 +6,14 @@
 // output and calls hyq_decode_hybrid through the pointer the Python side
 // hands over at set-up (the library ctypes loaded, whichever file that is).
 //
-// It takes exactly the calls the Python fast path takes (bf16 / fp16 q with
-// unit channel stride, kv_repeat dividing the query heads, CUDA tensors, the
-// three bf16 segments with unit channel strides, equal K / V lengths and one
-// dtype, the quantised prefix with unit innermost strides); anything else
-// returns status -1 and the caller takes its other paths.  The library
+// decode takes exactly the calls the Python fast path takes (bf16 / fp16 q
+// with unit channel stride, kv_repeat dividing the query heads, CUDA tensors,
+// the three bf16 segments with unit channel strides, equal K / V lengths and
+// one dtype, the quantised prefix with unit innermost strides); decode_cache
+// the same over a cache's buffers, with q's heads one stride apart; append
+// plain CUDA rows of the buffers' type and device that autograd does not
+// record.  Anything else returns status -1 and the caller takes its other
+// paths (the checked call, two tensor copies).  The library
 // validates every field (alignment, 32-bit strides, sizes) before it
 // launches, as for every other caller.  Host code only: no kernel here.
 
@@ -134,10 +137,10 @@ Result decode(const at::Tensor& q, const at::Tensor& kp, const at::Tensor& vp, c
                kw, vw, k_bits, v_bits, kv_repeat, sm_scale, split_tokens, stream, ws, ws_bytes);
 }
 
-// One layer's decode step over its cache's own buffers: q [b, hq, 1, d], the
-// first nq tokens of the prefix store, the first ns rows of the staging
-// buffers.  Returns [b, hq, 1, d].
-Result decode_cache(const at::Tensor& q, const at::Tensor& kp, const at::Tensor& vp, const at::Tensor& ks,
+// One layer's decode step over its cache's own buffers: q [b, hq, 1, d] of the
+// cache's batch, the first nq tokens of the prefix store, the first ns rows of
+// the staging buffers.  Returns [b, hq, 1, d].
+Result decode_cache(const at::Tensor& q, int64_t batch, const at::Tensor& kp, const at::Tensor& vp, const at::Tensor& ks,
                     const at::Tensor& vs, int64_t nq, const at::Tensor& kt, const at::Tensor& vt, const at::Tensor& kst,
                     const at::Tensor& vst, int64_t ns, const at::Tensor& kw, const at::Tensor& vw, int64_t k_bits,
                     int64_t v_bits, int64_t kv_repeat, int64_t stream, int64_t ws, int64_t ws_bytes) {
@@ -147,7 +150,7 @@ Result decode_cache(const at::Tensor& q, const at::Tensor& kp, const at::Tensor&
     // the rows of all heads have to be one stride apart
     if (q.size(2) != 1 || q.stride(3) != 1 || b * h * d == 0 || (h > 1 && b > 1 && q.stride(0) != h * q.stride(1)))
         return skip;
-    if (kt.size(0) * kv_repeat != b * h) return skip;
+    if (b != batch || kt.size(0) * kv_repeat != b * h) return skip;
     const int64_t row = h > 1 ? q.stride(1) : b > 1 ? q.stride(0) : d;
     return run(q, b * h, d, row, {b, h, 1, d}, kp, vp, ks, vs, nq, kt, vt, kst, vst, ns, kw, vw, k_bits, v_bits,
                kv_repeat, std::nan(""), 0, stream, ws, ws_bytes);
@@ -187,7 +190,7 @@ std::tuple<int64_t, int64_t, int64_t> layout() {
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-    m.def("entries", [] { return 2; }, "the number of addresses that set_entry takes");
+    m.def("signatures", [] { return 2; }, "counts up when a function of this module takes other arguments");
     m.def("layout", &layout, "sizeof(hyq_decode_params), offsetof(seg_n), offsetof(dtype_flags)");
     m.def("set_entry", &set_entry, "the addresses of hyq_decode_hybrid and hyq_append_rows");
     m.def("decode", &decode, "fused_d_stage_decode eager fast path");

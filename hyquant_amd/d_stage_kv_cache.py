@@ -249,7 +249,7 @@ class DStageLayerCache:
                 stream = _stream(query_states.device)
                 w = dd._ws_raw.get((dev, stream), dd._NO_WS)
                 ks, vs = self._kstore, self._vstore
-                st, out = fx.decode_cache(query_states, ks.packed, vs.packed, ks.scale, vs.scale, ks.n, self.k_topk,
+                st, out = fx.decode_cache(query_states, self._B, ks.packed, vs.packed, ks.scale, vs.scale, ks.n, self.k_topk,
                                           self.v_topk, self._staging_buf_k, self._staging_buf_v, self._staging_ptr,
                                           self.k_window, self.v_window, self.k_bits, self.v_bits, kv_repeat, stream,
                                           w[0], w[1])

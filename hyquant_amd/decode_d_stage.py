@@ -310,8 +310,8 @@ def _load_fast_ext():
             _FX = False
             return False
         P = _lib.DecodeParams
-        # (a build of earlier sources has no entries())
-        if getattr(m, "entries", lambda: 0)() == 2 and m.layout() == (ctypes.sizeof(P), P.seg_n.offset, P.dtype_flags.offset):
+        # (a build of earlier sources has no signatures())
+        if getattr(m, "signatures", lambda: 0)() == 2 and m.layout() == (ctypes.sizeof(P), P.seg_n.offset, P.dtype_flags.offset):
             m.set_entry(*(ctypes.cast(f, ctypes.c_void_p).value
                           for f in (_lib.lib().hyq_decode_hybrid, _lib.lib().hyq_append_rows)))
             mod = m
