@@ -658,7 +658,7 @@ def prefill_trace_summary(trace_csv):
     calls, cur = [], {}
     short = lambda n: n.replace("void ", "").replace("hyq::(anonymous namespace)::", "").split("(")[0]
     ours = ("prefill_main_kernel", "prep_kernel", "kv_convert_kernel", "gather_kernel",
-            "per_block_int8_kernel", "zero_counts_kernel", "lists_kernel")
+            "per_block_int8_kernel", "zero_counts_kernel", "lists_")
     for r in rows:
         n = short(r["Kernel_Name"])
         if not any(o in n for o in ours):

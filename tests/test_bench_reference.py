@@ -32,3 +32,22 @@ def test_error_vs_known_answers():
     assert math.isclose(e["rel_max"], 0.3 / 4.0, rel_tol=1e-6)
     assert math.isclose(e["mse"], (0.01 + 0.09) / 4, rel_tol=1e-6)
     assert math.isclose(e["rel_l2"], math.sqrt(0.1) / math.sqrt(1 + 4 + 0.25 + 16), rel_tol=1e-6)
+
+
+def test_prefill_trace_summary_counts_every_list_kernel(tmp_path):
+    """A prefill call's kernels by name, the lists' stand-alone launches among them."""
+    rows, t = ["Kernel_Name,Start_Timestamp,End_Timestamp"], 0
+    calls = len(bench.PREFILL_NS) * len(bench.PREFILL_VARIANTS) * bench.PREFILL_CALLS
+    for _ in range(calls):
+        for name, us in (("lists_lds_kernel", 5), ("lists_kernel", 7), ("prep_kernel", 3), ("at::fill", 100),
+                         ("prefill_main_kernel<true>", 40)):
+            rows.append(f'"void hyq::(anonymous namespace)::{name}(int)",{t},{t + 1000 * us}')
+            t += 1000 * us + 10
+    path = tmp_path / "run_kernel_trace.csv"
+    path.write_text("\n".join(rows) + "\n")
+    table = bench.prefill_trace_summary(str(path))
+    assert len(table) * bench.PREFILL_CALLS == calls
+    for row in table:
+        assert row["kernels_us"] == {"lists_lds_kernel": 5.0, "lists_kernel": 7.0, "prep_kernel": 3.0,
+                                     "prefill_main_kernel<true>": 40.0}
+        assert row["total_us"] == 55.0
