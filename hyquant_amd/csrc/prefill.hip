@@ -2133,8 +2133,8 @@ PrefillLayout prefill_layout(int B, int HQ, int HKV, int64_t N, int64_t T, int W
     return L;
 }
 
-// lists_lds_kernel and prep_kernel may take more than the default 64 KiB of
-// dynamic LDS (set once per process; a repeated call is harmless)
+// lists_lds_kernel may take more than the default 64 KiB of dynamic LDS (set
+// once per process; a repeated call is harmless)
 int raise_lds_limit(size_t lds) {
     static std::atomic<bool> done{false};
     if (lds <= 64 * 1024 || done.load(std::memory_order_acquire)) return HYQ_OK;
@@ -2163,6 +2163,9 @@ int launch_lists(const ListArgs& l, int BH, int* gscratch, hipStream_t stream) {
 // The lists and the statistics.  One launch while the lists' LDS leaves the
 // statistics' workgroups two to a CU; `chunks` 0: no statistics are needed.
 constexpr size_t PREP_LDS = 48 * 1024;
+// within the default limit beside the kernel's own arrays (stats_chunk's sums
+// and maxima, lists_row's scan)
+static_assert(PREP_LDS + (PREP_THREADS / 64) * PD * (sizeof(double) + sizeof(float)) + 256 <= 64 * 1024, "prep_kernel's LDS");
 int launch_prep(const ListArgs* l, int BH, int* gscratch, const StatArgs& st, int chunks, hipStream_t stream) {
     const bool one = l && chunks > 0 && lists_in_lds(l->T, l->P) && lists_lds(*l) <= PREP_LDS;
     if (l && !one)
