@@ -1499,7 +1499,7 @@ __global__ __launch_bounds__(THREADS, 2) void decode_kernel(DecArgs a) {
 // tokens (618 MB with the bf16 rows): K4V4 161 -> 101 us (6.1 TB/s, near the
 // 6.8 TB/s of a read-only stream), K4V2 172 -> 91, K2V4 159 -> 94, K2V2 169 ->
 // 90 us; 60 heads at G = 16, 5838 tokens 43 -> 21 us.  Two workgroups per CU
-// (217-233 VGPRs, no spill).  Error against float64, K4V4: 3.2e-3 -> 2.0e-3 of
+// (214-233 VGPRs, no spill; BLK = 1 at three per CU spills in its loop).  Error against float64, K4V4: 3.2e-3 -> 2.0e-3 of
 // the output's norm.
 //
 // Prefix units are chunks of 32 tokens that never cross a scale group (a
